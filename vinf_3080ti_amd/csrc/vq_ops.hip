@@ -1127,44 +1127,70 @@ size_t split_ws_bytes(const SegTable &T, int span_rows, int heads, int kv_heads,
 
 // ---- causal conv update ----------------------------------------------------------------------------------
 
-// Depthwise causal conv + SiLU, one thread per (channel, segment), the K-tap window in registers (K a template
-// parameter: the shift is register renaming). Per row: window <- [window[1:], x], out = silu(window . w).
+// Depthwise causal conv + SiLU, one thread per (channel, span of a segment's rows), the K-tap window in registers (K
+// a template parameter: the shift is register renaming). Per row: window <- [window[1:], x], out = silu(window . w).
 // snap (one segment only) gets the window after each row but the last, [rows - 1][channels][K]; the state
 // [slot][channels][K] gets the last window unless write_state is 0 (a verification pass leaves it untouched).
-template <int K>
-__global__ __launch_bounds__(256) void conv_update_kernel(const float *__restrict__ x, float *__restrict__ state,
-                                                          const float *__restrict__ w, float *__restrict__ out,
-                                                          int channels, SegTable T, float *__restrict__ snap,
-                                                          int write_state) {
+//
+// The window before a span's first row is the K rows of x before it (the state for what lies before the segment), so
+// spans are independent: block z takes rows z * span .. of its segment. Bound by memory latency when one thread walks
+// all rows: 512 rows x 10240 channels took 179 us on 40 workgroups with one load in flight; spans of 8 rows, their
+// loads issued together, take 9.3 us (2560 workgroups; the rows read twice come from L2). The first span's
+// thread is the only one that touches the state: it reads it, and writes the last K inputs into it. A span of
+// all rows (span >= rows, grid.z 1) keeps every read of a channel's x ahead of the writes that follow it, which x ==
+// out needs.
+constexpr int kConvRows = 8;  // rows whose loads are in flight together, and the span of a long pass
+static_assert(kConvRows >= VQ_CONV_MAX_K, "the K rows before a later span lie in the segment");
+template <int K, int TR>
+__global__ __launch_bounds__(256) void conv_update_kernel(const float *x, float *__restrict__ state,
+                                                          const float *__restrict__ w, float *out, int channels,
+                                                          SegTable T, float *__restrict__ snap, int write_state,
+                                                          int span) {
     const int c = blockIdx.x * 256 + threadIdx.x;
-    if (c >= channels) return;
     const Seg &s = T.s[blockIdx.y];
+    // TR == 1: a pass of one row per segment.
+    const int rows = TR == 1 ? 1 : s.rows, ta = TR == 1 ? 0 : blockIdx.z * span, tb = min(ta + span, rows);
+    if (c >= channels || ta >= rows) return;
     float *st = state + (static_cast<size_t>(s.slot) * channels + c) * K;
+    const float *const xc = x + static_cast<size_t>(s.row0) * channels + c;
+    float *const oc = out + static_cast<size_t>(s.row0) * channels + c;
     float win[K], wc[K];
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-        win[k] = st[k];
-        wc[k] = w[static_cast<size_t>(c) * K + k];
+    for (int k = 0; k < K; ++k) wc[k] = w[static_cast<size_t>(c) * K + k];
+    // Window slot k before row ta: input ta - K + k, for the first span the state.
+    if (ta == 0) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) win[k] = st[k];
+    } else {
+#pragma unroll
+        for (int k = 0; k < K; ++k) win[k] = xc[static_cast<size_t>(ta - K + k) * channels];
     }
-    const size_t row = static_cast<size_t>(s.row0) * channels + c;
-    for (int t = 0; t < s.rows; ++t) {
-        const float xi = x[row + static_cast<size_t>(t) * channels];
+    for (int t0 = ta; t0 < (TR == 1 ? 1 : tb); t0 += TR) {
+        float xi[TR];
 #pragma unroll
-        for (int k = 0; k + 1 < K; ++k) win[k] = win[k + 1];
-        win[K - 1] = xi;
-        float acc = 0.0f;
+        for (int j = 0; j < TR; ++j) xi[j] = xc[static_cast<size_t>(TR == 1 ? 0 : min(t0 + j, tb - 1)) * channels];
 #pragma unroll
-        for (int k = 0; k < K; ++k) acc = fmaf(win[k], wc[k], acc);
-        out[row + static_cast<size_t>(t) * channels] = silu_ieee(acc);
-        if (snap != nullptr && t + 1 < s.rows) {
-            float *sn = snap + (static_cast<size_t>(t) * channels + c) * K;
+        for (int j = 0; j < TR; ++j) {
+            const int t = t0 + j;
+            if (TR > 1 && t >= tb) break;
 #pragma unroll
-            for (int k = 0; k < K; ++k) sn[k] = win[k];
+            for (int k = 0; k + 1 < K; ++k) win[k] = win[k + 1];
+            win[K - 1] = xi[j];
+            float acc = 0.0f;
+#pragma unroll
+            for (int k = 0; k < K; ++k) acc = fmaf(win[k], wc[k], acc);
+            oc[static_cast<size_t>(t) * channels] = silu_ieee(acc);
+            if (snap != nullptr && t + 1 < rows) {
+                float *sn = snap + (static_cast<size_t>(t) * channels + c) * K;
+#pragma unroll
+                for (int k = 0; k < K; ++k) sn[k] = win[k];
+            }
         }
     }
-    if (write_state) {
+    if (write_state && ta == 0) {
 #pragma unroll
-        for (int k = 0; k < K; ++k) st[k] = win[k];
+        for (int k = 0; k < K; ++k)
+            st[k] = TR == 1 || tb == rows ? win[k] : xc[static_cast<size_t>(rows - K + k) * channels];
     }
 }
 
@@ -1658,10 +1684,24 @@ int launch_conv_update(const float *x, float *state, const float *w, float *out,
     if (!x || !state || !w || !out) return VQ_ERR_ARG;
     if (channels < 1 || K < 1 || K > VQ_CONV_MAX_K) return VQ_ERR_SHAPE;
     if (snap != nullptr && T.n != 1) return VQ_ERR_ARG;
-    const dim3 grid((channels + 255) / 256, T.n);
+    int max_rows = 1, end = 1;
+    for (int i = 0; i < T.n; ++i) {
+        max_rows = T.s[i].rows > max_rows ? T.s[i].rows : max_rows;
+        end = T.s[i].row0 + T.s[i].rows > end ? T.s[i].row0 + T.s[i].rows : end;
+    }
+    // One span per segment while it is short, or where out may overwrite rows of x that another span still reads.
+    const size_t n = static_cast<size_t>(end) * channels;
+    const bool overlap = x < out + n && out < x + n;
+    const int span = max_rows <= kConvRows || overlap ? max_rows : kConvRows;
+    const dim3 grid((channels + 255) / 256, T.n, (max_rows + span - 1) / span);
     switch (K) {
-#define VQ_CONV_CASE(KK) \
-    case KK: conv_update_kernel<KK><<<grid, 256, 0, s>>>(x, state, w, out, channels, T, snap, write_state); break;
+#define VQ_CONV_CASE(KK)                                                                                              \
+    case KK:                                                                                                          \
+        if (max_rows == 1)                                                                                            \
+            conv_update_kernel<KK, 1><<<grid, 256, 0, s>>>(x, state, w, out, channels, T, snap, write_state, span);   \
+        else                                                                                                          \
+            conv_update_kernel<KK, kConvRows><<<grid, 256, 0, s>>>(x, state, w, out, channels, T, snap, write_state, span); \
+        break;
         VQ_CONV_CASE(1) VQ_CONV_CASE(2) VQ_CONV_CASE(3) VQ_CONV_CASE(4)
         VQ_CONV_CASE(5) VQ_CONV_CASE(6) VQ_CONV_CASE(7) VQ_CONV_CASE(8)
 #undef VQ_CONV_CASE
