@@ -83,3 +83,25 @@ def test_conv_update_spans(rt, oracle_mod, K, rows, in_place):
     rt.conv_update_seg("cx" if not in_place else "co", "cs", "cw", "co", ch, K, "csn", 0)
     snaps = oracle_mod.conv_update(x[:n], cs0[segs[0][0]], w)[2]
     assert np.array_equal(get(rt, "csn", (-1, ch, K))[:n - 1], snaps)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 128, 129, 200, 256, 257])
+def test_rmsnorm_short_groups(rt, n):
+    """Groups of up to 256 values take one wave each (64, 128 or 256 values per wave), longer ones a workgroup: against
+    float64, in place and gated, 9 groups (a workgroup holds four). Bound: the fp32 sum of n squares and five
+    roundings, under 4e-7 relative for n <= 257; expf in silu adds under 2e-7."""
+    rng = np.random.default_rng(n)
+    groups, eps = 9, 1e-6
+    x, z = rng.standard_normal((2, groups, n)).astype(np.float32)
+    w = rng.standard_normal(n).astype(np.float32)
+    put_weight(rt, "nw", w)
+    put(rt, "nz", z)
+    expect = x.astype(np.float64) / np.sqrt((x.astype(np.float64) ** 2).mean(-1, keepdims=True) + eps) * w
+    for gated in (False, True):
+        put(rt, "nx", x)
+        if gated:
+            rt.gated_rmsnorm("nx", "nw", "nz", "nx", n, eps, groups)
+            expect = expect * z / (1.0 + np.exp(-z.astype(np.float64)))
+        else:
+            rt.rmsnorm("nx", "nw", "nx", n, eps, groups)
+        assert np.allclose(get(rt, "nx", (groups, n)), expect, rtol=6e-7, atol=1e-12)

@@ -152,6 +152,40 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(const float *x, c
     }
 }
 
+// Groups of up to 64 NI values (a head's gated norm, NI 1, 2 or 4): one wave per group, four groups per workgroup, every
+// load issued before the first use. Bound by bytes; with 256 threads and eight barriers per group the 24576 groups of
+// 128 of a 512-token pass took 22.5 us, so 9.7 us. The sum is the tree of the kernel above over its 256 partial values
+// (x^2, zero past n): elements 128 apart, then 64, then the lanes' halves, bit for bit.
+constexpr int kNormShort = 256;
+template <int NI>
+__global__ __launch_bounds__(256) void rmsnorm_short_kernel(const float *x, const float *__restrict__ w, const float *z,
+                                                            float *y, int n, int groups, float eps) {
+    const int lane = threadIdx.x & 63, g = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (g >= groups) return;
+    const size_t base = static_cast<size_t>(g) * n;
+    float v[NI], q[4] = {0.f, 0.f, 0.f, 0.f}, wv[NI], zv[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int e = min(lane + 64 * i, n - 1);
+        v[i] = x[base + e];
+        wv[i] = w[e];
+        zv[i] = z != nullptr ? z[base + e] : 0.0f;
+    }
+#pragma unroll
+    for (int i = 0; i < NI; ++i) q[i] = lane + 64 * i < n ? __fmul_rn(v[i], v[i]) : 0.0f;
+    float sum = __fadd_rn(__fadd_rn(q[0], q[2]), __fadd_rn(q[1], q[3]));
+#pragma unroll
+    for (int h = 32; h > 0; h >>= 1) sum = __fadd_rn(sum, __shfl_xor(sum, h, 64));
+    const float scale = 1.0f / sqrtf(sum / static_cast<float>(n) + eps);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        if (lane + 64 * i >= n) break;
+        float o = v[i] * scale * wv[i];
+        if (z != nullptr) o *= silu_ieee(zv[i]);
+        y[base + lane + 64 * i] = o;
+    }
+}
+
 // out = a + b (op 0), silu(a) * b (op 1), a * sigmoid(b) (op 2): four elements per thread.
 template <int OP>
 __device__ __forceinline__ float binop(float a, float b) {
@@ -1806,7 +1840,12 @@ extern "C" {
 int vq_rmsnorm(const float *x, const float *w, const float *z, float *y, int n, int groups, float eps, void *stream) {
     if (!x || !w || !y) return VQ_ERR_ARG;
     if (n < 1 || groups < 1 || !(eps >= 0.0f)) return VQ_ERR_SHAPE;
-    rmsnorm_kernel<<<groups, kNormThreads, 0, static_cast<hipStream_t>(stream)>>>(x, w, z, y, n, eps);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const unsigned blocks = groups / 4 + (groups % 4 != 0);
+    if (n <= 64) rmsnorm_short_kernel<1><<<blocks, 256, 0, s>>>(x, w, z, y, n, groups, eps);
+    else if (n <= 128) rmsnorm_short_kernel<2><<<blocks, 256, 0, s>>>(x, w, z, y, n, groups, eps);
+    else if (n <= kNormShort) rmsnorm_short_kernel<4><<<blocks, 256, 0, s>>>(x, w, z, y, n, groups, eps);
+    else rmsnorm_kernel<<<groups, kNormThreads, 0, s>>>(x, w, z, y, n, eps);
     return status_of(hipGetLastError());
 }
 
