@@ -259,6 +259,20 @@ int vq_gated_delta_seg(const float *conv, const float *b, const float *a, const 
                        float eps, int head_order, const int32_t *segs, int nseg, float *snap, int write_state,
                        void *stream);
 
+/* Workspace bytes of vq_gated_delta_seg_ws for this segment table: non-zero when a segment is long enough for the
+ * chunked kernels (24 rows; kd 128, vd a multiple of 32 up to 128), else 0 (the call then runs token by token). */
+size_t vq_gated_delta_seg_workspace_bytes(const int32_t *segs, int nseg, int key_heads, int value_heads, int kd, int vd);
+
+/* vq_gated_delta_seg with a workspace (16-byte aligned, >= vq_gated_delta_seg_workspace_bytes, else
+ * VQ_ERR_WORKSPACE; NULL: as vq_gated_delta_seg): long segments run in chunks of 32 tokens on fp32 MFMA, whose
+ * sums group differently from the per-token kernel's (same precision). Each segment takes its path by its own row
+ * count alone. With snap every segment runs token by token. Replaces: Runtime.gated_delta_seg
+ * (qwen_runtime.cu:2513-2565). */
+int vq_gated_delta_seg_ws(const float *conv, const float *b, const float *a, const float *ssm_a, const float *dt,
+                          void *state, int state_elem, float *out, int key_heads, int value_heads, int kd, int vd,
+                          float eps, int head_order, const int32_t *segs, int nseg, float *snap, int write_state,
+                          void *workspace, size_t workspace_bytes, void *stream);
+
 /* Activation staging flags of vq_qmv_staged: the bits of the reference megakernel's QMV flags
  * (runtime/instructions.py:179-182; QMV_FLAG_ARGMAX = 4 is vq_lmhead_argmax here). */
 #define VQ_QMV_ADD 1      /* y[t][r] += (W v)[r] instead of =                                      */

@@ -105,3 +105,103 @@ def test_rmsnorm_short_groups(rt, n):
         else:
             rt.rmsnorm("nx", "nw", "nx", n, eps, groups)
         assert np.allclose(get(rt, "nx", (groups, n)), expect, rtol=6e-7, atol=1e-12)
+
+
+def gated_delta_rows(oracle_mod, inp, segs, states, kh, vh, kd, vd, order):
+    """The float64 restatement per segment: outputs [rows][vh][vd] at the segments' rows, states after the pass."""
+    n = inp["conv"].shape[0]
+    out, fin = np.zeros((n, vh, vd)), states.astype(np.float64)
+    for slot, _, m, r0 in segs:
+        rows = slice(r0, r0 + m)
+        out[rows], fin[slot], _ = oracle_mod.gated_delta(inp["conv"][rows], inp["b"][rows], inp["a"][rows], inp["ssm_a"],
+                                                         inp["dt"], states[slot], kh, vh, kd, vd, 1e-6, order)
+    return out, fin
+
+
+def gated_delta_inputs(rng, n, kh, vh, kd, vd, slots):
+    return dict(conv=rng.standard_normal((n, 2 * kh * kd + vh * vd)).astype(np.float32),
+                b=rng.standard_normal((n, vh)).astype(np.float32), a=rng.standard_normal((n, vh)).astype(np.float32),
+                ssm_a=-rng.uniform(0.02, 2.0, vh).astype(np.float32), dt=rng.standard_normal(vh).astype(np.float32),
+                state=(0.1 * rng.standard_normal((slots, vh, kd, vd))).astype(np.float32))
+
+
+def run_gated_delta(rt, inp, segs, shape, elem, order, write):
+    kh, vh, kd, vd = shape
+    n = inp["conv"].shape[0]
+    for name in ("ssm_a", "dt"):
+        put_weight(rt, "g." + name, inp[name])
+    for name in ("conv", "b", "a"):
+        put(rt, "g." + name, inp[name])
+    put(rt, "g.s", inp["state"], elem)
+    put(rt, "g.o", np.zeros((n, vh, vd)))
+    rt.set_segments(segs)
+    rt.gated_delta_seg("g.conv", "g.b", "g.a", "g.ssm_a", "g.dt", "g.s", "g.o", kh, vh, kd, vd, 1e-6, order, None, write)
+    return get(rt, "g.o", (n, vh, vd)), get(rt, "g.s", inp["state"].shape)
+
+
+# Chunks of 32 tokens from 24 rows on, 16 chunks (less with several segments) per launch pair: below and at the
+# threshold, one chunk, a chunk and a row, two launch pairs, and long segments beside short ones; ragged head counts
+# against the XCD grouping of 8 heads, narrow states, both head orders, fp16 state.
+@pytest.mark.parametrize("rows,shape,order,elem", [
+    ((23,), (1, 2, 128, 128), 0, 4), ((24,), (1, 2, 128, 128), 1, 4), ((32,), (2, 6, 128, 64), 0, 4),
+    ((33, 1, 70), (3, 9, 128, 32), 1, 4), ((530,), (1, 1, 128, 96), 0, 4), ((65, 300, 5), (2, 10, 128, 128), 1, 2),
+    ((520,), (1, 2, 128, 32), 0, 2)])
+def test_gated_delta_chunks(rt, oracle_mod, rows, shape, order, elem):
+    """The chunked kernels against the float64 restatement, relative to the largest value: fp32 sums over 128 state rows
+    and 32 tokens per chunk, the same as the per-token kernel's error (3e-7 measured for both), so 2e-6; an fp16 state
+    rounds once (2^-11). write_state = 0 leaves the state as it was."""
+    kh, vh, kd, vd = shape
+    rng = np.random.default_rng(sum(rows) + vh + vd)
+    slots = 4
+    rt.alloc("pt", 64)
+    rt.set_paging("pt", 1024, 64 // slots, slots)
+    segs, r0 = [], 0
+    for i, m in enumerate(rows):
+        segs.append((slots - 1 - i, 0, m, r0))
+        r0 += m + (2 if i == 0 else 0)
+    inp = gated_delta_inputs(rng, r0, kh, vh, kd, vd, slots)
+    if elem == 2:
+        inp["state"] = inp["state"].astype(np.float16).astype(np.float32)
+    expect, fin = gated_delta_rows(oracle_mod, inp, segs, inp["state"], kh, vh, kd, vd, order)
+    for write in (0, 1):
+        out, st = run_gated_delta(rt, inp, segs, shape, elem, order, write)
+        assert np.abs(out - expect).max() <= 2e-6 * np.abs(expect).max()
+        want, tol = (fin, 2e-6 if elem == 4 else 5e-4) if write else (inp["state"], 0.0)
+        assert np.abs(st - want).max() <= tol * np.abs(want).max()
+
+
+@pytest.mark.parametrize("what", ["v", "k", "beta", "decay above one"])
+def test_gated_delta_chunks_keep_causality(rt, oracle_mod, what):
+    """A value that is not finite reaches its own token and the ones after it, never an earlier token of its chunk (nor,
+    in v, another column), as the per-token kernel has it; decays above one whose products leave the fp32 range while
+    the state does not are computed too."""
+    shape = kh, vh, kd, vd = 1, 2, 128, 64
+    rng = np.random.default_rng(5)
+    n, bad = 80, 45
+    rt.alloc("pt", 64)
+    rt.set_paging("pt", 64, 16, 1)
+    inp = gated_delta_inputs(rng, n, kh, vh, kd, vd, 1)
+    segs = [(0, 0, n, 0)]
+    if what == "decay above one":  # e^15 a token over a zero state and zero values, then decays near one
+        inp["ssm_a"][:], inp["dt"][:], inp["a"][:32], inp["a"][32:] = 1.0, 0.0, 15.0, -12.0
+        inp["state"][:] = inp["conv"][:32, 2 * kh * kd:] = 0.0
+        expect, fin = gated_delta_rows(oracle_mod, inp, segs, inp["state"], kh, vh, kd, vd, 0)
+        out, st = run_gated_delta(rt, inp, segs, shape, 4, 0, 1)
+        assert np.abs(out - expect).max() <= 2e-6 * np.abs(expect).max()
+        assert np.abs(st - fin).max() <= 2e-6 * np.abs(fin).max()
+        return
+    clean, _ = gated_delta_rows(oracle_mod, inp, segs, inp["state"], kh, vh, kd, vd, 0)
+    cols = slice(None)
+    if what == "v":
+        inp["conv"][bad, 2 * kh * kd + 3] = np.inf  # head 0, column 3
+        cols = 3
+    elif what == "k":
+        inp["conv"][bad, kh * kd + 7] = np.nan
+    else:
+        inp["b"][bad, 0] = np.nan
+    out, st = run_gated_delta(rt, inp, segs, shape, 4, 0, 1)
+    assert np.abs(out[:bad] - clean[:bad]).max() <= 2e-6 * np.abs(clean).max()
+    assert not np.isfinite(out[bad:, 0, cols]).any() and not np.isfinite(st[0, 0, :, cols]).any()
+    if what == "v":
+        rest = np.arange(vd) != 3
+        assert np.abs(out[:, 0, rest] - clean[:, 0, rest]).max() <= 2e-6 * np.abs(clean).max()

@@ -53,6 +53,8 @@ SIGNATURES: dict[str, tuple[object, list]] = {
     "vq_conv_update_seg": (I, [P, P, P, P, I, I, P, I, P, I, P]),
     "vq_gated_delta": (I, [P, P, P, P, P, P, I, P, I, I, I, I, F, I, I, P, I, P]),
     "vq_gated_delta_seg": (I, [P, P, P, P, P, P, I, P, I, I, I, I, F, I, P, I, P, I, P]),
+    "vq_gated_delta_seg_workspace_bytes": (SZ, [P, I, I, I, I, I]),
+    "vq_gated_delta_seg_ws": (I, [P, P, P, P, P, P, I, P, I, I, I, I, F, I, P, I, P, I, P, SZ, P]),
     "vq_quantize_x": (I, [P, I, I, P, P, P, P]),
     "vq_pack_x": (I, [P, I, I, P, P]),
     "vq_qmv_packed": (I, [I, P, I, I, P, I, P, P]),

@@ -1,0 +1,537 @@
+// vq_gdelta_impl.h -- the gated delta rule of a prompt pass in chunks of 32 tokens on fp32 MFMA (included by vq_ops.hip).
+//
+// The rule per token t (k, q normalised, g the decay, b = beta):
+//   S <- g_t S;  d_t = b_t (v_t - S^T k_t);  S <- S + k_t d_t^T;  o_t = S^T q_t.
+// Over a chunk that starts from state S0, with D(t, i) = g_{i+1} ... g_t (running products, so that a pair's decay
+// carries only its own roundings) and G_t = D(t, -1):
+//   d_t = b_t (v_t - G_t S0^T k_t) - sum_{i<t} L(t, i) d_i,   L(t, i) = b_t D(t, i) (k_i . k_t)
+//   o_t = G_t S0^T q_t + sum_{i<=t} P(t, i) d_i,              P(t, i) = D(t, i) (k_i . q_t)
+//   S_C = G_C S0 + sum_i D(C - 1, i) k_i d_i^T
+// so with T = (I + L)^-1 everything that meets the state is a matrix product:
+//   d = T (b V - (b G) K S0),   o = G (Q S0) + P d,   S_C = G_C S0 + (D(C - 1, .) K)^T d.
+// All of it in fp32 (v_mfma_f32_16x16x4_f32, fp32 operands and sums, long sums in four chains): against float64 at 512
+// tokens rel-L2 1.6e-7 (outputs) and 1.7e-7 (state); the per-token kernel 1.4e-7 and 1.6e-7.
+//
+// Two launches. gd_prep_kernel, one workgroup per (chunk, value head), all chunks at once: T and P into the workspace in
+// MFMA operand order, and the tokens' scales. gd_chunk_kernel, one workgroup per (value head, 32 state columns), walks
+// the chunks with its part of the state in accumulators, the chunk's K, Q, V rows and T, P reaching LDS by DMA a chunk
+// ahead: 116-120 MFMAs per wave and two barriers per 32 tokens, instead of 32 serial tokens of two barriers each. What bounds
+// it: the serial chunk walk's MFMA issue (33 cycles each, 1.9 us of a chunk's 3.3, on 192 of 256 CUs). Operands prepared in full
+// (W = T diag(b G) K, scaled Q and K in operand order, read straight into registers) moved 55 KB per chunk and
+// workgroup through L2 twice and took 28 + 56 us. Measured at 16 key and 48 value heads, kd = vd = 128, 512 tokens:
+// 13.8 + 54.5 us against 358 us token by token. Of a chunk's 6800 cycles the K S0 and Q S0 products take 3500 (their
+// 64 MFMAs 2100; the rest are the copies and LDS reads of the one wave per SIMD), T R 690, the state update 1720; eight
+// waves of 32 rows measured 62 us (more operand reads and a four-way exchange), one copy per four MFMAs 57 us.
+//
+// MFMA layouts used below (lane = 16 lk + lr): C/D element q is row 4 lk + q, column lr; the k index of an operand
+// element is free as long as A and B agree, so step q of a 16-deep block takes k = 4 lk + q: an accumulator tile is then
+// a B operand as it stands, and an A operand is one float4 of a row.
+//
+// Inputs that are not finite (or whose norms or decays are not) would meet zeros of T and P in these products and reach
+// tokens before their own; the prep kernel flags such chunks and the walk takes them token by token.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stddef.h>
+#include <stdint.h>
+
+#include <algorithm>
+
+namespace {
+
+constexpr int kGcC = 32, kGcKd = 128, kGcMaxVd = 128, kGcCols = 32;
+// Segments of at least this many rows take the chunks. Measured at 48 value heads, us token by token / in chunks: one
+// sequence of 16 rows 15.3 / 15.8, 24 rows 21.7 / 16.0, 64 rows 47.6 / 19.1; four of 16 rows 23.0 / 25.9, 24 rows
+// 32.2 / 26.6.
+constexpr int kGcMinRows = 24;
+constexpr int kGcRound = 16;  // chunks per segment and launch pair at one segment (bounds the workspace)
+static_assert(kGcRound <= 64, "one lane per chunk reads the non-finite flags");
+
+typedef float gc_f4 __attribute__((ext_vector_type(4)));
+
+// Workspace of one (chunk, value head), in floats: T and P as A operands [t tile 2][i tile 2][lane][4], then the tokens'
+// scales (32 each: b G / |k|, b, D(C - 1, .) / |k|, G / (|q| sqrt(kd))), G_C and the non-finite flag.
+struct GcSlot {
+    static constexpr int T = 0, P = 1024, SC = 2048, KW = 0, B = 32, KC = 64, QG = 96, GC = 128, BAD = 129;
+    static constexpr size_t floats = 2304;
+};
+
+// The long segments of a pass, and the chunks [c0, c0 + cr) of each that this launch covers; slot ((seg * cr + c - c0)
+// * value_heads + head).
+struct GcArgs {
+    const float *conv, *braw, *araw, *ssm_a, *dt;
+    float *ws;
+    int key_heads, value_heads, vd, head_order, c0, cr;
+    float eps;
+};
+
+__device__ __forceinline__ bool gc_bad(float v) { return (__float_as_uint(v) & 0x7F800000u) == 0x7F800000u; }
+__device__ __forceinline__ gc_f4 gc_mfma(float a, float b, gc_f4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ gc_f4 gc_ld(const float *p) { return *reinterpret_cast<const gc_f4 *>(p); }
+
+__global__ __launch_bounds__(256) void gd_prep_kernel(GcArgs A, SegTable T) {
+    constexpr int RS = kGcKd + 4;  // LDS row pitch (floats)
+    __shared__ __align__(16) float sK[kGcC][RS], sQ[kGcC][RS];
+    __shared__ __align__(16) float sL[kGcC][36], sT[kGcC][36], sD[kGcC][33];
+    __shared__ float sB[kGcC], sG[kGcC], sGt[kGcC], sQs[kGcC], sKs[kGcC];
+    __shared__ int s_bad;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, lr = lane & 15, lk = lane >> 4;
+    const int h = blockIdx.x, c = A.c0 + blockIdx.y;
+    const Seg &s = T.s[blockIdx.z];
+    const int t0 = c * kGcC, nt = min(kGcC, s.rows - t0);
+    if (nt <= 0) return;
+    const int vh = A.value_heads, vd = A.vd;
+    const int kh = A.head_order == 0 ? h / (vh / A.key_heads) : h % A.key_heads;
+    const size_t cdim = static_cast<size_t>(2) * A.key_heads * kGcKd + static_cast<size_t>(vh) * vd;
+    const size_t row0 = static_cast<size_t>(s.row0) + t0;
+    float *const ws = A.ws + ((static_cast<size_t>(blockIdx.z) * A.cr + blockIdx.y) * vh + h) * GcSlot::floats;
+
+    // 1. The chunk's q, k rows (zeros past the segment); v only to see that it is finite.
+    if (tid == 0) s_bad = 0;
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = (tid >> 5) + 8 * i, e = 4 * (tid & 31);
+        gc_f4 q = {0.f, 0.f, 0.f, 0.f}, k = q, v = q;
+        if (r < nt) {
+            const float *src = A.conv + (row0 + r) * cdim;
+            q = gc_ld(src + static_cast<size_t>(kh) * kGcKd + e);
+            k = gc_ld(src + static_cast<size_t>(A.key_heads + kh) * kGcKd + e);
+            if (e < vd) v = gc_ld(src + static_cast<size_t>(2) * A.key_heads * kGcKd + static_cast<size_t>(h) * vd + e);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) bad |= gc_bad(q[j]) || gc_bad(k[j]) || gc_bad(v[j]);
+        *reinterpret_cast<gc_f4 *>(&sQ[r][e]) = q;
+        *reinterpret_cast<gc_f4 *>(&sK[r][e]) = k;
+    }
+    __syncthreads();
+    // 2. Per token (eight threads each): the norm scales; beta and the decay.
+    {
+        const int t = tid >> 3, j = tid & 7;
+        const bool in = t < nt;
+        const size_t rr = (row0 + (in ? t : 0)) * vh + h;
+        const float xa = A.araw[rr] + A.dt[h], xb = A.braw[rr], sa = A.ssm_a[h];
+        float qq = 0.0f, kk = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const gc_f4 q = gc_ld(&sQ[t][4 * (j + 8 * i)]), k = gc_ld(&sK[t][4 * (j + 8 * i)]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) qq = fmaf(q[e], q[e], qq), kk = fmaf(k[e], k[e], kk);
+        }
+        qq = gsum8(qq);
+        kk = gsum8(kk);
+        if (j == 0) {
+            const float rkd = 1.0f / sqrtf(static_cast<float>(kGcKd));
+            const float qs = in ? rkd / sqrtf(qq + A.eps) : 0.0f, ks = in ? 1.0f / sqrtf(kk + A.eps) : 0.0f;
+            const float g = in ? expf(sa * (xa > 20.0f ? xa : log1pf(expf(xa)))) : 1.0f;
+            const float b = in ? sigmoid_ieee(xb) : 0.0f;
+            bad |= gc_bad(qs) || gc_bad(ks) || gc_bad(g) || gc_bad(b);
+            sQs[t] = qs, sKs[t] = ks, sG[t] = g, sB[t] = b;
+        }
+    }
+    if (bad) s_bad = 1;
+    __syncthreads();
+    // 3. Decays of the pairs: lane i of wave 0 walks D(t, i) down its column; lane 32 the decay since the chunk's start.
+    // The other waves meanwhile start on their products.
+    if (tid < kGcC) {
+        float d = 1.0f;
+#pragma unroll
+        for (int t = 0; t < kGcC; ++t) {
+            d = t <= tid ? 1.0f : d * sG[t];
+            sD[t][tid] = t < tid ? 0.0f : d;
+        }
+    } else if (tid == kGcC) {
+        float d = 1.0f, grow = 1.0f;
+#pragma unroll
+        for (int t = 0; t < kGcC; ++t) {
+            d *= sG[t];
+            grow *= fmaxf(sG[t], 1.0f);
+            sGt[t] = d;
+        }
+        if (!(grow < 1e30f)) s_bad = 1;  // decays above one: products of them could overflow where the state does not
+    }
+    // 4. Wave (jt, ji): the 16 x 16 tiles L (rows t, columns i) and P^T (rows i, columns t); nothing above the diagonal.
+    const int jt = wv >> 1, ji = wv & 1;
+    gc_f4 kk = {0.f, 0.f, 0.f, 0.f}, kq = kk, kc4[4] = {kk, kk, kk, kk}, qc4[4] = {kk, kk, kk, kk};
+    if (ji <= jt) {  // four chains each, as in the walk
+#pragma unroll
+        for (int cc = 0; cc < kGcKd / 16; ++cc) {
+            const gc_f4 kt = gc_ld(&sK[16 * jt + lr][16 * cc + 4 * lk]), ki = gc_ld(&sK[16 * ji + lr][16 * cc + 4 * lk]),
+                        qt = gc_ld(&sQ[16 * jt + lr][16 * cc + 4 * lk]);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                kc4[q] = gc_mfma(kt[q], ki[q], kc4[q]);
+                qc4[q] = gc_mfma(ki[q], qt[q], qc4[q]);
+            }
+        }
+        kk = (kc4[0] + kc4[1]) + (kc4[2] + kc4[3]);
+        kq = (qc4[0] + qc4[1]) + (qc4[2] + qc4[3]);
+    }
+    __syncthreads();
+    gc_f4 p;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int t = 16 * jt + 4 * lk + q, i = 16 * ji + lr;
+        sL[t][i] = i < t ? sB[t] * sD[t][i] * (sKs[t] * sKs[i]) * kk[q] : 0.0f;
+        const int pt = 16 * jt + lr, pi = 16 * ji + 4 * lk + q;
+        p[q] = pi <= pt ? sD[pt][pi] * (sQs[pt] * sKs[pi]) * kq[q] : 0.0f;
+    }
+    *reinterpret_cast<gc_f4 *>(ws + GcSlot::P + ((jt * 2 + ji) * 64 + lane) * 4) = p;
+    if (tid < kGcC) {
+        float *const sc = ws + GcSlot::SC;
+        sc[GcSlot::KW + tid] = sB[tid] * sGt[tid] * sKs[tid];
+        sc[GcSlot::B + tid] = sB[tid];
+        sc[GcSlot::KC + tid] = sD[kGcC - 1][tid] * sKs[tid];
+        sc[GcSlot::QG + tid] = sGt[tid] * sQs[tid];
+        if (tid == 0) sc[GcSlot::GC] = sGt[kGcC - 1], sc[GcSlot::BAD] = s_bad || gc_bad(sGt[kGcC - 1]) ? 1.0f : 0.0f;
+    }
+    __syncthreads();
+    // 5. T = (I + L)^-1: the two diagonal blocks by forward substitution (lane = column), then T21 = -T22 (L21 T11).
+    if (wv < 2 && lane < 16) {
+        const int o = 16 * wv;
+        float x[16];
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            float v = t == lane ? 1.0f : 0.0f;
+#pragma unroll
+            for (int i = 0; i < t; ++i) v = fmaf(-sL[o + t][o + i], x[i], v);
+            x[t] = v;
+            sT[o + t][o + lane] = v;
+        }
+    }
+    __syncthreads();
+    if (wv == 0) {
+        gc_f4 m = {0.f, 0.f, 0.f, 0.f}, x = m;
+        const gc_f4 l = gc_ld(&sL[16 + lr][4 * lk]), t22 = gc_ld(&sT[16 + lr][16 + 4 * lk]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) m = gc_mfma(l[q], sT[4 * lk + q][lr], m);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x = gc_mfma(t22[q], m[q], x);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sT[16 + 4 * lk + q][lr] = -x[q];
+    }
+    __syncthreads();
+    if (ji <= jt)
+        *reinterpret_cast<gc_f4 *>(ws + GcSlot::T + ((jt * 2 + ji) * 64 + lane) * 4) =
+            gc_ld(&sT[16 * jt + lr][16 * ji + 4 * lk]);
+}
+
+// The chunk walk. Wave w of a workgroup: column tile n = w & 1 (16 of the 32 columns), state rows 64 kh .. +64 with
+// kh = w >> 1. The two waves of a column tile exchange their halves of W S and of the other's 16 output rows through LDS.
+// state_in / state_out: the slot's state, or the fp32 copy between two launches of one pass (tmp, [seg][head][kd][vd]).
+template <typename ST>
+__global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, ST *__restrict__ state,
+                                                          float *__restrict__ tmp, float *__restrict__ out,
+                                                          int write_state) {
+    // One chunk's operands. A K or Q row's 16-byte pieces sit at piece ^ (row & 15): the 16 rows of an A operand and
+    // the rows 4 lk + q of a transposed one then fall on distinct banks. V rows: piece ^ 4 on every other four rows.
+    struct Buf {
+        float k[kGcC * kGcKd], q[kGcC * kGcKd], v[kGcC * kGcCols], t[1024], p[1024], sc[256];
+    };
+    __shared__ __align__(1024) Buf buf[2];
+    __shared__ __align__(16) gc_f4 ex[4][3][64];  // [wave][tile][lane]
+    __shared__ float red[2][4][3][16];            // token-by-token chunks: [wave][sum][column]
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lk = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), n = wv & 1, kh = wv >> 1;
+    const int vh = A.value_heads, vd = A.vd, tiles = vd / kGcCols;
+    // Workgroup ids go round-robin over the 8 XCDs: the column tiles of one head, which read the same operands, are 8
+    // ids apart and share an XCD's L2.
+    const int b = blockIdx.x, g8 = (b / (8 * tiles)) * 8, r8 = b - g8 * tiles, wide = min(8, vh - g8);
+    const int h = g8 + r8 % wide, c0 = (r8 / wide) * kGcCols;
+    const Seg &s = T.s[blockIdx.y];
+    const int nch = (s.rows + kGcC - 1) / kGcC, ca = A.c0, cb = min(nch, A.c0 + A.cr);
+    if (ca >= cb) return;
+    const int col = c0 + 16 * n + lr;
+    const size_t hstate = static_cast<size_t>(kGcKd) * vd;
+    ST *const S = state + (static_cast<size_t>(s.slot) * vh + h) * hstate;
+    float *const Sx = tmp + (static_cast<size_t>(blockIdx.y) * vh + h) * hstate;
+    const float *const slot0 = A.ws + (static_cast<size_t>(blockIdx.y) * A.cr * vh + h) * GcSlot::floats;
+    const size_t cstep = static_cast<size_t>(vh) * GcSlot::floats;
+
+    gc_f4 st[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const size_t e = static_cast<size_t>(64 * kh + 16 * i + 4 * lk + q) * vd + col;
+            st[i][q] = ca == 0 ? ld_state(S + e) : Sx[e];
+        }
+    const int kx = A.head_order == 0 ? h / (vh / A.key_heads) : h % A.key_heads;
+    const size_t cdim = static_cast<size_t>(2) * A.key_heads * kGcKd + static_cast<size_t>(vh) * vd;
+    // DMA of chunk c into buffer c & 1, 11 or 12 KB per wave, in three parts between the products of chunk c - 1 (ahead of
+    // them all the wave stalls 850 cycles while the copies are taken up); the lane offsets are those of a full chunk (rows
+    // past the segment repeat its last one, their scales are zero).
+    uint32_t off_k[4], off_v;
+    auto offsets = [&](int last) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int r = 2 * (wv + 4 * j) + (lane >> 5);
+            off_k[j] = (static_cast<uint32_t>(min(r, last)) * static_cast<uint32_t>(cdim) + 4u * ((lane & 31) ^ (r & 15))) * 4u;
+        }
+        const int r = 8 * wv + (lane >> 3);
+        off_v = (static_cast<uint32_t>(min(r, last)) * static_cast<uint32_t>(cdim) + 4u * ((lane & 7) ^ (r & 4))) * 4u;
+    };
+    const float *const conv0 = A.conv + static_cast<size_t>(s.row0) * cdim;
+    const uint32_t lds0 = vq::lds_addr(buf);
+    auto issue = [&](int c, int part) {
+        const float *const base = conv0 + static_cast<size_t>(c * kGcC) * cdim;
+        const float *const sl = slot0 + static_cast<size_t>(c - ca) * cstep;
+        const uint32_t d = lds0 + (c & 1) * static_cast<uint32_t>(sizeof(Buf)) + 1024u * wv;
+        if (part == 0) {
+            if (s.rows - c * kGcC < kGcC) offsets(s.rows - c * kGcC - 1);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                vq::dma16u(base + static_cast<size_t>(A.key_heads + kx) * kGcKd, off_k[j], d + offsetof(Buf, k) + 4096 * j, buf);
+        } else if (part == 1) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                vq::dma16u(base + static_cast<size_t>(kx) * kGcKd, off_k[j], d + offsetof(Buf, q) + 4096 * j, buf);
+        } else {
+            vq::dma16u(base + static_cast<size_t>(2) * A.key_heads * kGcKd + static_cast<size_t>(h) * vd + c0, off_v,
+                       d + offsetof(Buf, v), buf);
+            vq::dma16u(sl + GcSlot::T + 256 * wv, 16u * lane, d + offsetof(Buf, t), buf);
+            vq::dma16u(sl + GcSlot::P + 256 * wv, 16u * lane, d + offsetof(Buf, p), buf);
+            if (wv == 0) vq::dma16u(sl + GcSlot::SC, 16u * lane, d + offsetof(Buf, sc), buf);
+        }
+    };
+    float *const orow = out + (static_cast<size_t>(s.row0) * vh + h) * vd + col;
+    const size_t ostep = static_cast<size_t>(vh) * vd;
+
+    // One chunk from its operands (landed; all waves past the barrier that says so).
+    auto chunk = [&](int c) {
+        const Buf &f = buf[c & 1];
+        auto a_row = [&](const float *m, int t, int i) {  // A operand: rows 16 t + lr, columns 64 kh + 16 i + 4 lk ..
+            return gc_ld(m + (16 * t + lr) * kGcKd + 4 * ((16 * kh + 4 * i + lk) ^ lr));
+        };
+        // One wave per SIMD: nothing else hides an LDS read, so each part's operands are read a part ahead, and the
+        // scheduler is kept from sinking the reads back to their uses (without the fences: 57.6 us for 16 chunks).
+#define VQ_GC_FENCE() __builtin_amdgcn_sched_barrier(0)
+        gc_f4 ka[2][4], qa[2][4], x[2], o[2];
+        float kt[2][4][4];
+        auto read_kt = [&](int t) {  // K^T operand: column 64 kh + 16 i + lr of rows 16 t + 4 lk + q
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float *const kr = f.k + (16 * t + 4 * lk + q) * kGcKd + (lr & 3);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) kt[t][q][i] = kr[4 * ((16 * kh + 4 * i + (lr >> 2)) ^ (4 * lk + q))];
+            }
+        };
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ka[0][i] = a_row(f.k, 0, i), ka[1][i] = a_row(f.k, 1, i);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) qa[0][i] = a_row(f.q, 0, i), qa[1][i] = a_row(f.q, 1, i);
+        VQ_GC_FENCE();
+        // Four chains per tile: a quarter of the length, half the rounding of a 64-term sum in order.
+        gc_f4 xc[2][4], oc[2][4];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) xc[t][e] = oc[t][e] = gc_f4{0.f, 0.f, 0.f, 0.f};
+        gc_f4 kw[2], bs[2], kc[2], vv[2], tt[3], pp[2], qg;
+        float gc;
+        // K S0 and Q S0: four chains of MFMAs (a dependent one waits 8-12 cycles past its 32), in four parts that also
+        // read what the second half of the chunk needs and start the next chunk's DMA.
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (i < 2) {
+                read_kt(i);
+            } else {
+                const int t = i - 2;
+                kw[t] = gc_ld(f.sc + GcSlot::KW + 16 * t + 4 * lk);
+                bs[t] = gc_ld(f.sc + GcSlot::B + 16 * t + 4 * lk);
+                kc[t] = gc_ld(f.sc + GcSlot::KC + 16 * t + 4 * lk);
+                pp[t] = gc_ld(f.p + 4 * ((2 * kh + t) * 64 + lane));
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    vv[t][q] = f.v[(16 * t + 4 * lk + q) * kGcCols + ((16 * n + lr) ^ ((lk & 1) << 4))];
+                if (t == 0) {
+                    tt[0] = gc_ld(f.t + 4 * lane), tt[1] = gc_ld(f.t + 4 * (128 + lane));
+                    tt[2] = gc_ld(f.t + 4 * (192 + lane));
+                } else {
+                    qg = gc_ld(f.sc + GcSlot::QG + 16 * kh + 4 * lk);
+                    gc = f.sc[GcSlot::GC];
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    xc[t][q] = gc_mfma(ka[t][i][q], st[i][q], xc[t][q]);
+                    oc[t][q] = gc_mfma(qa[t][i][q], st[i][q], oc[t][q]);
+                }
+            }
+            if (i < 3 && c + 1 < cb) issue(c + 1, i);
+            VQ_GC_FENCE();
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            x[t] = (xc[t][0] + xc[t][1]) + (xc[t][2] + xc[t][3]);
+            o[t] = (oc[t][0] + oc[t][1]) + (oc[t][2] + oc[t][3]);
+        }
+        ex[wv][0][lane] = x[0];
+        ex[wv][1][lane] = x[1];
+        ex[wv][2][lane] = kh == 0 ? o[1] : o[0];  // the partner's output rows
+        __syncthreads();
+        const int pw = wv ^ 2;
+        gc_f4 xp[2] = {ex[pw][0][lane], ex[pw][1][lane]};
+        const gc_f4 op = ex[pw][2][lane];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) st[i] *= gc;
+        // R = b V - (b G) K S0, then d = T R
+        gc_f4 r[2], d[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, d1 = d[0];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) r[t][q] = fmaf(-kw[t][q], x[t][q] + xp[t][q], bs[t][q] * vv[t][q]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            d[0] = gc_mfma(tt[0][q], r[0][q], d[0]);
+            d[1] = gc_mfma(tt[1][q], r[0][q], d[1]);
+            d1 = gc_mfma(tt[2][q], r[1][q], d1);
+        }
+        d[1] += d1;
+        // S = G_C S + K^T (D(C - 1, .) d),  o = G (Q S0) + P d (the tile of P above the diagonal is zero)
+        gc_f4 y = ((kh == 0 ? o[0] : o[1]) + op) * qg;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const gc_f4 kd = d[t] * kc[t];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) st[i] = gc_mfma(kt[t][q][i], kd[q], st[i]);
+                y = gc_mfma(pp[t][q], d[t][q], y);
+            }
+        }
+#undef VQ_GC_FENCE
+        vq::wait_vm<0>();  // the next chunk's operands (not the stores that follow)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int t = c * kGcC + 16 * kh + 4 * lk + q;
+            if (t < s.rows) orow[t * ostep] = y[q];
+        }
+    };
+    // One chunk token by token (an input is not finite): the rule as the per-token kernel computes it.
+    auto serial = [&](int c) {
+        const float rkd = 1.0f / sqrtf(static_cast<float>(kGcKd));
+        // Column sums over all rows: the lane groups, then the two waves of the column tile.
+        auto total = [&](float v, int k, int par) {
+            v = xor32_add(xor16_add(v));
+            if (lk == 0) red[par][wv][k][lr] = v;
+        };
+        for (int t = c * kGcC; t < min((c + 1) * kGcC, s.rows); ++t) {
+            const size_t rr = static_cast<size_t>(s.row0) + t;
+            const float *qs = A.conv + rr * cdim + static_cast<size_t>(kx) * kGcKd + 64 * kh + 4 * lk;
+            gc_f4 qv[4], kv[4];
+            float qq = 0.0f, kk = 0.0f, mem = 0.0f, o = 0.0f;
+            const float xa = A.araw[rr * vh + h] + A.dt[h];
+            const float decay = expf(A.ssm_a[h] * (xa > 20.0f ? xa : log1pf(expf(xa))));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                qv[i] = gc_ld(qs + 16 * i);
+                kv[i] = gc_ld(qs + static_cast<size_t>(A.key_heads) * kGcKd + 16 * i);
+                st[i] *= decay;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    qq = fmaf(qv[i][q], qv[i][q], qq);
+                    kk = fmaf(kv[i][q], kv[i][q], kk);
+                    mem = fmaf(st[i][q], kv[i][q], mem);
+                }
+            }
+            total(qq, 0, 0), total(kk, 1, 0), total(mem, 2, 0);
+            __syncthreads();
+            qq = red[0][n][0][lr] + red[0][n + 2][0][lr];
+            kk = red[0][n][1][lr] + red[0][n + 2][1][lr];
+            mem = red[0][n][2][lr] + red[0][n + 2][2][lr];
+            const float ks = 1.0f / sqrtf(kk + A.eps), beta = sigmoid_ieee(A.braw[rr * vh + h]);
+            const float v = A.conv[rr * cdim + static_cast<size_t>(2) * A.key_heads * kGcKd + static_cast<size_t>(h) * vd + col];
+            const float upd = (v - mem * ks) * beta * ks;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    st[i][q] = fmaf(kv[i][q], upd, st[i][q]);
+                    o = fmaf(st[i][q], qv[i][q], o);
+                }
+            total(o, 0, 1);
+            __syncthreads();
+            if (kh == 0 && lk == 0) orow[t * ostep] = (red[1][n][0][lr] + red[1][n + 2][0][lr]) * (rkd / sqrtf(qq + A.eps));
+        }
+        __syncthreads();
+    };
+
+    offsets(kGcC - 1);
+#pragma unroll
+    for (int part = 0; part < 3; ++part) issue(ca, part);
+    const bool flagged = lane < cb - ca && slot0[lane * cstep + GcSlot::SC + GcSlot::BAD] != 0.0f;
+    const uint64_t bad = __ballot(flagged);  // chunk ca + i of this launch: bit i
+    vq::wait_vm<0>();
+    for (int c = ca; c < cb; ++c) {
+        __syncthreads();  // chunk c landed for every wave; every wave is done with chunk c - 1's buffer
+        if ((bad >> (c - ca) & 1) == 0) {
+            chunk(c);
+        } else {
+#pragma unroll
+            for (int part = 0; part < 3; ++part)
+                if (c + 1 < cb) issue(c + 1, part);
+            serial(c);
+            vq::wait_vm<0>();
+        }
+    }
+    if (cb == nch && !write_state) return;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const size_t e = static_cast<size_t>(64 * kh + 16 * i + 4 * lk + q) * vd + col;
+            if (cb == nch) st_state(S + e, st[i][q]);
+            else Sx[e] = st[i][q];
+        }
+}
+
+// The chunked path takes these shapes (every row offset 16-byte aligned) ...
+bool gc_shape(int key_heads, int value_heads, int kd, int vd) {
+    return kd == kGcKd && vd % kGcCols == 0 && vd <= kGcMaxVd && key_heads >= 1 && value_heads >= key_heads &&
+           value_heads % key_heads == 0;
+}
+// ... for these segments of a pass; chunks per launch and segment, and workspace bytes (0: no such segment).
+int gc_segments(const SegTable &T, SegTable *longs, SegTable *shorts) {
+    SegTable L{}, H{};
+    for (int i = 0; i < T.n; ++i) {
+        SegTable &d = T.s[i].rows >= kGcMinRows ? L : H;
+        d.s[d.n++] = T.s[i];
+        d.total += T.s[i].rows;
+    }
+    if (longs) *longs = L;
+    if (shorts) *shorts = H;
+    return L.n;
+}
+int gc_round(int nlong) { return nlong >= kGcRound ? 1 : kGcRound / nlong; }
+size_t gc_ws_bytes(const SegTable &T, int key_heads, int value_heads, int kd, int vd) {
+    if (!gc_shape(key_heads, value_heads, kd, vd)) return 0;
+    SegTable L;
+    const int n = gc_segments(T, &L, nullptr);
+    if (n == 0) return 0;
+    int nch = 1;
+    for (int i = 0; i < n; ++i) nch = std::max(nch, (L.s[i].rows + kGcC - 1) / kGcC);
+    const size_t slots = static_cast<size_t>(n) * std::min(gc_round(n), nch) * value_heads * GcSlot::floats;
+    const size_t copy = nch > gc_round(n) ? static_cast<size_t>(n) * value_heads * kGcKd * vd : 0;
+    return (slots + copy) * sizeof(float);
+}
+
+template <typename ST>
+int gc_launch(const SegTable &L, const float *conv, const float *b, const float *a, const float *ssm_a, const float *dt,
+              ST *state, float *out, int key_heads, int value_heads, int vd, float eps, int head_order, int write_state,
+              float *ws, hipStream_t s) {
+    int nch = 1;
+    for (int i = 0; i < L.n; ++i) nch = std::max(nch, (L.s[i].rows + kGcC - 1) / kGcC);
+    GcArgs A{conv, b, a, ssm_a, dt, ws, key_heads, value_heads, vd, head_order, 0, std::min(gc_round(L.n), nch), eps};
+    float *const tmp = ws + static_cast<size_t>(L.n) * A.cr * value_heads * GcSlot::floats;
+    for (; A.c0 < nch; A.c0 += A.cr) {
+        gd_prep_kernel<<<dim3(value_heads, std::min(A.cr, nch - A.c0), L.n), 256, 0, s>>>(A, L);
+        gd_chunk_kernel<ST><<<dim3(value_heads * (vd / kGcCols), L.n), 256, 0, s>>>(A, L, state, tmp, out, write_state);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return status_of(e);
+    }
+    return VQ_OK;
+}
+
+}  // namespace

@@ -31,6 +31,12 @@ __device__ __forceinline__ void dma16s(const void *base, uint32_t voff, void *ds
     asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %1, %0" ::"s"(base), "v"(voff), "s"(lds_addr(dst)), "s"(dst)
                  : "memory", "m0");
 }
+// The same with the destination as an LDS byte address inside the __shared__ object `whole` (the operand that tells the
+// compiler what the asm writes): for destinations computed from loop counters.
+__device__ __forceinline__ void dma16u(const void *base, uint32_t voff, uint32_t lds, void *whole) {
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %1, %0" ::"s"(base), "v"(voff), "s"(lds), "s"(whole)
+                 : "memory", "m0");
+}
 template <int N>
 __device__ __forceinline__ void wait_vm() {
     static_assert(N >= 0 && N < 64, "vmcnt range");

@@ -1518,6 +1518,12 @@ __global__ __launch_bounds__(64 * NW) void gated_delta4_kernel(const float *__re
     }
 }
 
+}  // namespace
+
+#include "vq_gdelta_impl.h"
+
+namespace {
+
 // ---- host launchers --------------------------------------------------------------------------------------
 
 int launch_rope(float *x, const SegTable &T, int heads, int hd, int rot, double base, hipStream_t s) {
@@ -1788,12 +1794,32 @@ void gd4_dispatch(int R, dim3 grid, hipStream_t s, const float *conv, const floa
 
 int launch_gated_delta(const float *conv, const float *b, const float *a, const float *ssm_a, const float *dt,
                        void *state, int state_elem, float *out, int kh, int vh, int kd, int vd, float eps,
-                       int head_order, const SegTable &T, float *snap, int write_state, hipStream_t s) {
+                       int head_order, const SegTable &T, float *snap, int write_state, hipStream_t s,
+                       void *ws = nullptr, size_t ws_bytes = 0) {
     if (!conv || !b || !a || !ssm_a || !dt || !state || !out || (state_elem != 4 && state_elem != 2)) return VQ_ERR_ARG;
     if (kh < 1 || vh < kh || vh % kh || kd < 1 || kd > kGdMaxKd || vd < 1 || (head_order != 0 && head_order != 1) ||
         !(eps >= 0.0f))
         return VQ_ERR_SHAPE;
     if (snap != nullptr && (T.n != 1 || state_elem != 4)) return VQ_ERR_ARG;
+    if (ws != nullptr && snap == nullptr && (reinterpret_cast<uintptr_t>(conv) & 15) == 0) {
+        // With a workspace: the segments long enough for it in chunks on MFMA, each by its own row count (a segment's
+        // result does not depend on what else is in the pass); the others token by token below.
+        const size_t need = gc_ws_bytes(T, kh, vh, kd, vd);
+        if (need != 0) {
+            if (ws_bytes < need || (reinterpret_cast<uintptr_t>(ws) & 15)) return VQ_ERR_WORKSPACE;
+            SegTable L, H;
+            gc_segments(T, &L, &H);
+            float *const wf = static_cast<float *>(ws);
+            const int st = state_elem == 4
+                               ? gc_launch(L, conv, b, a, ssm_a, dt, static_cast<float *>(state), out, kh, vh, vd, eps,
+                                           head_order, write_state, wf, s)
+                               : gc_launch(L, conv, b, a, ssm_a, dt, static_cast<_Float16 *>(state), out, kh, vh, vd, eps,
+                                           head_order, write_state, wf, s);
+            if (st != VQ_OK || H.n == 0) return st;
+            return launch_gated_delta(conv, b, a, ssm_a, dt, state, state_elem, out, kh, vh, kd, vd, eps, head_order, H,
+                                      nullptr, write_state, s);
+        }
+    }
     const int R = kd <= 4 * kGdGroups ? 4 : kd <= 8 * kGdGroups ? 8 : kd <= 16 * kGdGroups ? 16 : 32;
     const uintptr_t align = reinterpret_cast<uintptr_t>(state) | reinterpret_cast<uintptr_t>(conv) |
                             reinterpret_cast<uintptr_t>(out) | (snap ? reinterpret_cast<uintptr_t>(snap) : 0);
@@ -2048,6 +2074,23 @@ int vq_gated_delta_seg(const float *conv, const float *b, const float *a, const 
     return st != VQ_OK ? st
                        : launch_gated_delta(conv, b, a, ssm_a, dt, state, state_elem, out, key_heads, value_heads, kd,
                                             vd, eps, head_order, T, snap, write_state, static_cast<hipStream_t>(stream));
+}
+
+size_t vq_gated_delta_seg_workspace_bytes(const int32_t *segs, int nseg, int key_heads, int value_heads, int kd, int vd) {
+    SegTable T;
+    return make_table(segs, nseg, T, nullptr) == VQ_OK ? gc_ws_bytes(T, key_heads, value_heads, kd, vd) : 0;
+}
+
+int vq_gated_delta_seg_ws(const float *conv, const float *b, const float *a, const float *ssm_a, const float *dt,
+                          void *state, int state_elem, float *out, int key_heads, int value_heads, int kd, int vd,
+                          float eps, int head_order, const int32_t *segs, int nseg, float *snap, int write_state,
+                          void *workspace, size_t workspace_bytes, void *stream) {
+    SegTable T;
+    const int st = make_table(segs, nseg, T, nullptr);
+    return st != VQ_OK ? st
+                       : launch_gated_delta(conv, b, a, ssm_a, dt, state, state_elem, out, key_heads, value_heads, kd,
+                                            vd, eps, head_order, T, snap, write_state, static_cast<hipStream_t>(stream),
+                                            workspace, workspace_bytes);
 }
 
 }  // extern "C"

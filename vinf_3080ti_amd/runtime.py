@@ -110,7 +110,7 @@ class Runtime:
         self.tensors: dict[str, _Tensor] = {}
         self.buffers: dict[str, _Buffer] = {}
         self._argmax_out = torch.empty(MAX_ARGMAX_ROWS, dtype=torch.int32, device=self.device)
-        self._ws = torch.empty(0, dtype=torch.uint8, device=self.device)
+        self._ws: dict[int, torch.Tensor] = {}  # per stream: calls on different streams may overlap
         self.gemm_min_rows = 0
         self.batch_invariant = False
         self.gemm_f16_activations = False
@@ -125,13 +125,17 @@ class Runtime:
 
     # ---- helpers ----------------------------------------------------------------------------------
     def _stream(self) -> int:
-        return torch.cuda.current_stream(self.device).cuda_stream
+        # torch.cuda.current_stream(device).cuda_stream without the Stream object (0.9 us less on every call)
+        return torch._C._cuda_getCurrentRawStream(self.device.index)
 
     def _workspace(self, nbytes: int) -> torch.Tensor:
-        """Device scratch for packed activations / argmax keys, grown on demand and reused (stream-ordered)."""
-        if self._ws.numel() < nbytes:
-            self._ws = torch.empty(max(nbytes, 2 * self._ws.numel()), dtype=torch.uint8, device=self.device)
-        return self._ws
+        """Device scratch of the calls on the current stream, grown on demand and reused (stream-ordered)."""
+        stream = self._stream()
+        ws = self._ws.get(stream)
+        if ws is None or ws.numel() < nbytes:
+            size = nbytes if ws is None else max(nbytes, 2 * ws.numel())
+            ws = self._ws[stream] = torch.empty(size, dtype=torch.uint8, device=self.device)
+        return ws
 
     def _logits_scratch(self, n: int) -> torch.Tensor:
         """fp32 logits of the batch-invariant argmax when the caller keeps none: grown on demand and reused
@@ -307,7 +311,7 @@ class Runtime:
         total = sum(g.data.numel() for g in self._groups)
         total += self._arena.data.numel() if self._arena is not None else 0
         total += sum(t.data.numel() for t in self.tensors.values() if t.home == "own")
-        return total + self.buffer_bytes() + self._ws.numel()
+        return total + self.buffer_bytes() + sum(w.numel() for w in self._ws.values())
 
     def buffer_bytes(self) -> int:
         return sum(b.data.numel() * b.elem for b in self.buffers.values())
@@ -617,10 +621,21 @@ class Runtime:
         sb, ob = self._f32_buffer(state, state_n), self._f32_buffer(out, value_heads * vd * ntok)
         sa, dtt = self._f32_weight(ssm_a, value_heads), self._f32_weight(dt, value_heads)
         snp = self._f32_buffer(snap, state_n * (ntok - 1)).data_ptr() if snap is not None else None
-        _lib.check(self._lib.vq_gated_delta(cb.data_ptr(), bb.data_ptr(), ab.data_ptr(), sa.data_ptr(), dtt.data_ptr(),
-                                            sb.data_ptr(), 4, ob.data_ptr(), key_heads, value_heads, kd, vd, float(eps),
-                                            int(head_order), ntok, snp, int(bool(write_state)), self._stream()),
-                   "gated_delta")
+        seg = (ctypes.c_int32 * 4)(0, 0, ntok, 0)
+        ws, nws = self._gated_delta_ws(seg, 1, ntok, key_heads, value_heads, kd, vd, snp)
+        _lib.check(self._lib.vq_gated_delta_seg_ws(cb.data_ptr(), bb.data_ptr(), ab.data_ptr(), sa.data_ptr(),
+                                                   dtt.data_ptr(), sb.data_ptr(), 4, ob.data_ptr(), key_heads,
+                                                   value_heads, kd, vd, float(eps), int(head_order), seg, 1, snp,
+                                                   int(bool(write_state)), ws, nws, self._stream()), "gated_delta")
+
+    def _gated_delta_ws(self, segs, nseg: int, rows: int, key_heads: int, value_heads: int, kd: int, vd: int,
+                        snap: int | None) -> tuple[int | None, int]:
+        """Workspace (address, bytes) of the chunked gated delta kernels: none for decode-length passes, snapshot
+        passes, and batch-invariant mode (a token's sums then do not depend on where its prompt was cut into passes)."""
+        if snap is not None or rows <= MAX_TOKENS or self.batch_invariant:
+            return None, 0
+        nws = self._lib.vq_gated_delta_seg_workspace_bytes(segs, nseg, key_heads, value_heads, kd, vd)
+        return (self._workspace(nws).data_ptr() if nws else None), nws
 
     def concat_rows(self, dst: str, a: str, b: str, rows: int, width: int) -> None:
         """dst[r] = [a[r] | b[r]] for rows of width floats (Runtime_concat_rows, qwen_runtime.cu:2567-2587)."""
@@ -792,11 +807,14 @@ class Runtime:
             if len(segs) != 1:
                 raise ValueError("snapshots need a single-segment pass")
             snp = self._f32_buffer(snap, state_n * (ntok - 1)).data_ptr()
+        rows = max(r for _, _, r, _ in segs)
         for arr, n in self._seg_chunks():
-            _lib.check(self._lib.vq_gated_delta_seg(cb.data_ptr(), bb.data_ptr(), ab.data_ptr(), sa.data_ptr(),
-                                                    dtt.data_ptr(), sbuf.data.data_ptr(), sbuf.elem, ob.data_ptr(),
-                                                    key_heads, value_heads, kd, vd, float(eps), int(head_order), arr, n,
-                                                    snp, int(bool(write_state)), self._stream()), "gated_delta_seg")
+            ws, nws = self._gated_delta_ws(arr, n, rows, key_heads, value_heads, kd, vd, snp)
+            _lib.check(self._lib.vq_gated_delta_seg_ws(cb.data_ptr(), bb.data_ptr(), ab.data_ptr(), sa.data_ptr(),
+                                                       dtt.data_ptr(), sbuf.data.data_ptr(), sbuf.elem, ob.data_ptr(),
+                                                       key_heads, value_heads, kd, vd, float(eps), int(head_order), arr,
+                                                       n, snp, int(bool(write_state)), ws, nws, self._stream()),
+                       "gated_delta_seg")
 
     def copy(self, dst: str, dst_off: int, src: str, src_off: int, n: int) -> None:
         """dst[dst_off:+n] = src[src_off:+n] in elements, buffers of one precision (Runtime_copy,
