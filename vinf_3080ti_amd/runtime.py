@@ -42,6 +42,9 @@ class _Tensor:
     home: str = "own"  # where the bytes live: "own" allocation, "arena", or "group:<id>"
     streamed: bool = False  # uploaded with resident=False (served from HBM all the same)
 
+    def __post_init__(self) -> None:
+        self.ptr = self.data.data_ptr()  # data lives as long as this entry; asking torch costs 0.2 us per use
+
 
 @dataclass
 class _Region:
@@ -67,6 +70,9 @@ WEIGHT_GRANULE = 2 << 20
 class _Buffer:
     data: torch.Tensor  # float32 or float16
     elem: int
+
+    def __post_init__(self) -> None:
+        self.ptr, self.n = self.data.data_ptr(), self.data.numel()
 
 
 def _check_upload_args(name: str, nbytes_given: int, type_id: int, cols: int, rows: int) -> tuple[int, int]:
@@ -114,8 +120,10 @@ class Runtime:
         self.gemm_min_rows = 0
         self.batch_invariant = False
         self.gemm_f16_activations = False
-        self._paging: tuple[torch.Tensor, int, int, int] | None = None
+        self._paging: tuple[_Buffer, int, int, int] | None = None
         self._segments: list[tuple[int, int, int, int]] = []
+        self._seg_tables: list[tuple[ctypes.Array, int]] = []  # the same as int32 tables of one launch each
+        self._seg_span = self._seg_longest = 0
         # Resident-weight memory: an optional arena and the executor's per-layer weight groups. Nothing streams
         # over PCIe here, so the stream order only records which uploads were requested as streamed.
         self._arena: _Region | None = None
@@ -157,14 +165,16 @@ class Runtime:
             raise KeyError(f"device buffer {name} is not allocated")
         return b
 
-    def _f32_buffer(self, name: str, min_n: int) -> torch.Tensor:
+    def _f32_buffer(self, name: str, min_n: int) -> _Buffer:
         """find_buffer (qwen_runtime.cu:1206-1223)."""
-        b = self._any_buffer(name)
+        b = self.buffers.get(name)
+        if b is None:
+            raise KeyError(f"device buffer {name} is not allocated")
         if b.elem != 4:
             raise TypeError(f"device buffer {name} is fp16 (KV cache), not fp32")
-        if b.data.numel() < min_n:
-            raise ValueError(f"device buffer {name} has {b.data.numel()} floats, need {min_n}")
-        return b.data
+        if b.n < min_n:
+            raise ValueError(f"device buffer {name} has {b.n} floats, need {min_n}")
+        return b
 
     # ---- weights ----------------------------------------------------------------------------------
     def upload(self, name: str, data, type_id: int, cols: int, rows: int, resident: bool = True, group: int = -1) -> None:
@@ -385,7 +395,7 @@ class Runtime:
 
     def buffer_ptr(self, name: str) -> tuple[int, int]:
         b = self._f32_buffer(name, 0)
-        return (b.data_ptr(), b.numel())
+        return (b.ptr, b.n)
 
     def buffer_elem(self, name: str) -> int:
         return self._any_buffer(name).elem
@@ -403,7 +413,7 @@ class Runtime:
         _check_qmv_args(weight, t.cols, ntok)
         xb = self._f32_buffer(x, t.cols * ntok)
         yb = self._f32_buffer(y, t.rows * ntok)
-        self._qmv_ptrs(t, xb.data_ptr(), yb.data_ptr(), ntok)
+        self._qmv_ptrs(t, xb.ptr, yb.ptr, ntok)
 
     def _qmv_ptrs(self, t: _Tensor, x_ptr: int, y_ptr: int, ntok: int) -> None:
         if t.type not in (0, 1) and self.gemm_min_rows > 0 and ntok >= self.gemm_min_rows:
@@ -415,7 +425,7 @@ class Runtime:
             if self.gemm_f16_activations and ng:
                 # The reference's own numerics: fp32 activations rounded to f16 inside the call.
                 buf = self._workspace(ng)
-                st = self._lib.vq_qgemm_f16x_ws(t.type, t.data.data_ptr(), t.rows, t.cols, x_ptr, ntok, y_ptr,
+                st = self._lib.vq_qgemm_f16x_ws(t.type, t.ptr, t.rows, t.cols, x_ptr, ntok, y_ptr,
                                                 buf.data_ptr(), ng, flags, self._stream())
                 _lib.check(st, "qgemm launch")
                 return
@@ -423,7 +433,7 @@ class Runtime:
             buf = self._workspace(nx + ng)
             xp = buf.data_ptr()
             _lib.check(self._lib.vq_pack_x(x_ptr, ntok, t.cols, xp, self._stream()), "pack_x")
-            st = self._lib.vq_qgemm_ws_ex(t.type, t.data.data_ptr(), t.rows, t.cols, xp, ntok, y_ptr,
+            st = self._lib.vq_qgemm_ws_ex(t.type, t.ptr, t.rows, t.cols, xp, ntok, y_ptr,
                                           (xp + nx) if ng else None, ng, flags, self._stream())
             _lib.check(st, "qgemm launch")
             return
@@ -433,7 +443,7 @@ class Runtime:
         else:
             nws = self._lib.vq_qmv_workspace_bytes_for(t.type, t.rows, t.cols, ntok)
             ws = self._workspace(nws).data_ptr() if nws else None
-        st = self._lib.vq_qmv(t.type, t.data.data_ptr(), t.rows, t.cols, x_ptr, ntok, y_ptr, ws, nws, self._stream())
+        st = self._lib.vq_qmv(t.type, t.ptr, t.rows, t.cols, x_ptr, ntok, y_ptr, ws, nws, self._stream())
         _lib.check(st, "qmv launch")
 
     def qmv_staged(self, weight: str, x: str, y: str, ntok: int = 1, *, x2: str | None = None,
@@ -456,32 +466,32 @@ class Runtime:
         x2p = nwp = None
         if x2 is not None:
             flags |= _lib.VQ_QMV_SILU_MUL
-            x2p = self._f32_buffer(x2, t.cols * ntok).data_ptr()
+            x2p = self._f32_buffer(x2, t.cols * ntok).ptr
         if norm is not None:
             flags |= _lib.VQ_QMV_NORM
             if norm in self.tensors:
                 nt = self._tensor(norm)
                 if nt.type != 0 or nt.rows * nt.cols != t.cols:
                     raise ValueError(f"{norm}: norm weights must be an F32 tensor of {t.cols} values")
-                nwp = nt.data.data_ptr()
+                nwp = nt.ptr
             else:
-                nwp = self._f32_buffer(norm, t.cols).data_ptr()
+                nwp = self._f32_buffer(norm, t.cols).ptr
         # 5-16 tokens of the f16 small-batch types stage inside that kernel (vq_qmv_staged_ws, with the RMS
         # prepass and partial sums in the runtime's workspace); other calls stream (vq_qmv_staged).
         nws = self._lib.vq_qmv_staged_workspace_bytes(t.type, t.rows, t.cols, ntok)
         ws = self._workspace(nws) if nws else None
-        st = self._lib.vq_qmv_staged_ws(t.type, t.data.data_ptr(), t.rows, t.cols, xb.data_ptr(), x2p, nwp,
-                                        float(eps), flags, ntok, yb.data_ptr(), ws.data_ptr() if ws is not None else None,
+        st = self._lib.vq_qmv_staged_ws(t.type, t.ptr, t.rows, t.cols, xb.ptr, x2p, nwp,
+                                        float(eps), flags, ntok, yb.ptr, ws.data_ptr() if ws is not None else None,
                                         nws, self._stream())
         _lib.check(st, "qmv_staged launch")
 
     # ---- ops around the matvec (the reference runtime's elementwise / norm ops) ------------------------------
-    def _f32_weight(self, name: str, n: int) -> torch.Tensor:
+    def _f32_weight(self, name: str, n: int) -> _Tensor:
         """find_f32_weight: an uploaded F32 tensor of n values."""
         t = self._tensor(name)
         if t.type != 0 or t.rows * t.cols != n:
             raise ValueError(f"{name}: expected an F32 tensor of {n} values")
-        return t.data
+        return t
 
     def rmsnorm(self, x: str, w: str, y: str, n: int, eps: float = 1e-6, groups: int = 1) -> None:
         """y[g] = x[g] * rsqrt(mean(x[g]^2) + eps) * w for each of `groups` rows of n (Runtime_rmsnorm,
@@ -490,7 +500,7 @@ class Runtime:
             raise ValueError("n and groups must be positive")
         xb, yb = self._f32_buffer(x, n * groups), self._f32_buffer(y, n * groups)
         wt = self._f32_weight(w, n)
-        _lib.check(self._lib.vq_rmsnorm(xb.data_ptr(), wt.data_ptr(), None, yb.data_ptr(), n, groups, float(eps),
+        _lib.check(self._lib.vq_rmsnorm(xb.ptr, wt.ptr, None, yb.ptr, n, groups, float(eps),
                                         self._stream()), "rmsnorm")
 
     def gated_rmsnorm(self, x: str, w: str, z: str, y: str, n: int, eps: float, groups: int) -> None:
@@ -500,7 +510,7 @@ class Runtime:
         xb, zb = self._f32_buffer(x, n * groups), self._f32_buffer(z, n * groups)
         yb = self._f32_buffer(y, n * groups)
         wt = self._f32_weight(w, n)
-        _lib.check(self._lib.vq_rmsnorm(xb.data_ptr(), wt.data_ptr(), zb.data_ptr(), yb.data_ptr(), n, groups,
+        _lib.check(self._lib.vq_rmsnorm(xb.ptr, wt.ptr, zb.ptr, yb.ptr, n, groups,
                                         float(eps), self._stream()), "gated_rmsnorm")
 
     def _binary(self, op: int, a: str, b: str, out: str, n: int) -> None:
@@ -508,7 +518,7 @@ class Runtime:
         if n < 0:
             raise ValueError("n must be non-negative")
         ab, bb, ob = self._f32_buffer(a, n), self._f32_buffer(b, n), self._f32_buffer(out, n)
-        _lib.check(self._lib.vq_binary(op, ab.data_ptr(), bb.data_ptr(), ob.data_ptr(), n, self._stream()),
+        _lib.check(self._lib.vq_binary(op, ab.ptr, bb.ptr, ob.ptr, n, self._stream()),
                    "elementwise")
 
     def add(self, a: str, b: str, out: str, n: int) -> None:
@@ -526,7 +536,7 @@ class Runtime:
             raise ValueError("heads and hd must be positive")
         n = heads * hd
         rb, qb, gb = self._f32_buffer(raw, 2 * n), self._f32_buffer(q, n), self._f32_buffer(gate, n)
-        _lib.check(self._lib.vq_split_gated_q(rb.data_ptr(), qb.data_ptr(), gb.data_ptr(), heads, hd, self._stream()),
+        _lib.check(self._lib.vq_split_gated_q(rb.ptr, qb.ptr, gb.ptr, heads, hd, self._stream()),
                    "split_gated_q")
 
     def rope(self, x: str, heads: int, hd: int, rot: int, pos: int, base: float = 10000.0, ntok: int = 1) -> None:
@@ -539,7 +549,7 @@ class Runtime:
         if heads < 1 or pos < 0:
             raise ValueError("heads must be positive and pos non-negative")
         xb = self._f32_buffer(x, heads * hd * ntok)
-        _lib.check(self._lib.vq_rope(xb.data_ptr(), ntok, heads, hd, rot, pos, float(base), self._stream()), "rope")
+        _lib.check(self._lib.vq_rope(xb.ptr, ntok, heads, hd, rot, pos, float(base), self._stream()), "rope")
 
     def kv_append(self, k: str, v: str, kc: str, vc: str, kv_heads: int, max_seq: int, hd: int, pos: int,
                   ntok: int = 1) -> None:
@@ -551,11 +561,11 @@ class Runtime:
         kb, vb = self._f32_buffer(k, n), self._f32_buffer(v, n)
         kcb, vcb = self._any_buffer(kc), self._any_buffer(vc)
         for name, b in ((kc, kcb), (vc, vcb)):
-            if b.data.numel() < cache:
-                raise ValueError(f"device buffer {name} has {b.data.numel()} values, need {cache}")
+            if b.n < cache:
+                raise ValueError(f"device buffer {name} has {b.n} values, need {cache}")
         if kcb.elem != vcb.elem:
             raise TypeError("K and V caches differ in precision")
-        _lib.check(self._lib.vq_kv_append(kb.data_ptr(), vb.data_ptr(), kcb.data.data_ptr(), vcb.data.data_ptr(),
+        _lib.check(self._lib.vq_kv_append(kb.ptr, vb.ptr, kcb.ptr, vcb.ptr,
                                           kcb.elem, ntok, kv_heads, max_seq, hd, pos, self._stream()), "kv_append")
 
     def attention(self, q: str, kc: str, vc: str, out: str, heads: int, kv_heads: int, hd: int, max_seq: int,
@@ -571,19 +581,19 @@ class Runtime:
         qb = self._f32_buffer(q, n)
         kcb, vcb = self._any_buffer(kc), self._any_buffer(vc)
         for name, b in ((kc, kcb), (vc, vcb)):
-            if b.data.numel() < cache:
-                raise ValueError(f"device buffer {name} has {b.data.numel()} values, need {cache}")
+            if b.n < cache:
+                raise ValueError(f"device buffer {name} has {b.n} values, need {cache}")
         ob = self._f32_buffer(out, n)
         if kcb.elem != vcb.elem:
             raise TypeError("K and V caches differ in precision")
         if self._tiled_attention(ntok):
-            _lib.check(self._lib.vq_attention_tiled(qb.data_ptr(), kcb.data.data_ptr(), vcb.data.data_ptr(),
-                                                    ob.data_ptr(), kcb.elem, heads, kv_heads, hd, max_seq, seq_len, ntok,
+            _lib.check(self._lib.vq_attention_tiled(qb.ptr, kcb.ptr, vcb.ptr,
+                                                    ob.ptr, kcb.elem, heads, kv_heads, hd, max_seq, seq_len, ntok,
                                                     int(bidirectional), int(window), self._stream()), "attention")
             return
         nws = self._lib.vq_attention_workspace_bytes(heads, kv_heads, hd, seq_len, ntok, int(window))
         ws = self._workspace(nws).data_ptr() if nws else None
-        _lib.check(self._lib.vq_attention_ws(qb.data_ptr(), kcb.data.data_ptr(), vcb.data.data_ptr(), ob.data_ptr(),
+        _lib.check(self._lib.vq_attention_ws(qb.ptr, kcb.ptr, vcb.ptr, ob.ptr,
                                              kcb.elem, heads, kv_heads, hd, max_seq, seq_len, ntok, int(bidirectional),
                                              int(window), ws, nws, self._stream()), "attention")
 
@@ -598,10 +608,10 @@ class Runtime:
         sb = self._f32_buffer(state, channels * K)
         ob = self._f32_buffer(out, channels * ntok)
         wt = self._f32_weight(w, channels * K)
-        snp = self._f32_buffer(snap, channels * K * (ntok - 1)).data_ptr() if snap is not None else None
+        snp = self._f32_buffer(snap, channels * K * (ntok - 1)).ptr if snap is not None else None
         if K > _lib.VQ_CONV_MAX_K:
             raise ValueError(f"conv kernel size {K} > {_lib.VQ_CONV_MAX_K}")
-        _lib.check(self._lib.vq_conv_update(xb.data_ptr(), sb.data_ptr(), wt.data_ptr(), ob.data_ptr(), channels, K,
+        _lib.check(self._lib.vq_conv_update(xb.ptr, sb.ptr, wt.ptr, ob.ptr, channels, K,
                                             ntok, snp, int(bool(write_state)), self._stream()), "conv_update")
 
     def gated_delta(self, conv: str, b: str, a: str, ssm_a: str, dt: str, state: str, out: str, key_heads: int,
@@ -620,11 +630,11 @@ class Runtime:
         bb, ab = self._f32_buffer(b, value_heads * ntok), self._f32_buffer(a, value_heads * ntok)
         sb, ob = self._f32_buffer(state, state_n), self._f32_buffer(out, value_heads * vd * ntok)
         sa, dtt = self._f32_weight(ssm_a, value_heads), self._f32_weight(dt, value_heads)
-        snp = self._f32_buffer(snap, state_n * (ntok - 1)).data_ptr() if snap is not None else None
+        snp = self._f32_buffer(snap, state_n * (ntok - 1)).ptr if snap is not None else None
         seg = (ctypes.c_int32 * 4)(0, 0, ntok, 0)
         ws, nws = self._gated_delta_ws(seg, 1, ntok, key_heads, value_heads, kd, vd, snp)
-        _lib.check(self._lib.vq_gated_delta_seg_ws(cb.data_ptr(), bb.data_ptr(), ab.data_ptr(), sa.data_ptr(),
-                                                   dtt.data_ptr(), sb.data_ptr(), 4, ob.data_ptr(), key_heads,
+        _lib.check(self._lib.vq_gated_delta_seg_ws(cb.ptr, bb.ptr, ab.ptr, sa.ptr,
+                                                   dtt.ptr, sb.ptr, 4, ob.ptr, key_heads,
                                                    value_heads, kd, vd, float(eps), int(head_order), seg, 1, snp,
                                                    int(bool(write_state)), ws, nws, self._stream()), "gated_delta")
 
@@ -643,15 +653,15 @@ class Runtime:
             raise ValueError("rows and width must be non-negative")
         n = rows * width
         ab, bb, db = self._f32_buffer(a, n), self._f32_buffer(b, n), self._f32_buffer(dst, 2 * n)
-        _lib.check(self._lib.vq_concat_rows(db.data_ptr(), ab.data_ptr(), bb.data_ptr(), rows, width, self._stream()),
+        _lib.check(self._lib.vq_concat_rows(db.ptr, ab.ptr, bb.ptr, rows, width, self._stream()),
                    "concat_rows")
 
     def zero_range(self, name: str, offset: int, n: int) -> None:
         """Clear n elements of a buffer from offset (Runtime_zero_range, qwen_runtime.cu:2589-2600)."""
         buf = self._any_buffer(name)
-        if offset < 0 or n < 0 or offset + n > buf.data.numel():
+        if offset < 0 or n < 0 or offset + n > buf.n:
             raise ValueError("zero_range out of bounds")
-        _lib.check(self._lib.vq_zero(buf.data.data_ptr() + offset * buf.elem, n * buf.elem, self._stream()),
+        _lib.check(self._lib.vq_zero(buf.ptr + offset * buf.elem, n * buf.elem, self._stream()),
                    "zero_range")
 
     # ---- multi-sequence passes (paged KV caches, per-slot recurrent state) --------------------------------------
@@ -685,6 +695,13 @@ class Runtime:
         if not table:
             raise ValueError("no segments")
         self._segments = table
+        # Built once for the pass: every layer's *_seg ops read them.
+        self._seg_tables = []
+        for i in range(0, len(table), _lib.VQ_MAX_SEGMENTS):
+            part = table[i:i + _lib.VQ_MAX_SEGMENTS]
+            self._seg_tables.append(((ctypes.c_int32 * (4 * len(part)))(*[v for sg in part for v in sg]), len(part)))
+        self._seg_span = max(r0 + n for _, _, n, r0 in table)
+        self._seg_longest = max(n for _, _, n, _ in table)
         return row0
 
     def _seg_ready(self) -> list[tuple[int, int, int, int]]:
@@ -693,21 +710,19 @@ class Runtime:
         return self._segments
 
     def _seg_rows(self) -> int:
-        return max(r0 + n for _, _, n, r0 in self._seg_ready())
+        self._seg_ready()
+        return self._seg_span
 
-    def _seg_chunks(self):
+    def _seg_chunks(self) -> list[tuple[ctypes.Array, int]]:
         """The segment table as int32 arrays of at most VQ_MAX_SEGMENTS segments (one launch each)."""
-        segs = self._seg_ready()
-        for i in range(0, len(segs), _lib.VQ_MAX_SEGMENTS):
-            part = segs[i:i + _lib.VQ_MAX_SEGMENTS]
-            yield (ctypes.c_int32 * (4 * len(part)))(*[v for sg in part for v in sg]), len(part)
+        return self._seg_tables
 
     def _kv_pair(self, kc: str, vc: str, min_n: int) -> tuple[_Buffer, _Buffer]:
         """find_kv_buffer for a K/V cache pair of one precision (qwen_runtime.cu:1226-1248)."""
         kcb, vcb = self._any_buffer(kc), self._any_buffer(vc)
         for name, buf in ((kc, kcb), (vc, vcb)):
-            if buf.data.numel() < min_n:
-                raise ValueError(f"device buffer {name} has {buf.data.numel()} values, need {min_n}")
+            if buf.n < min_n:
+                raise ValueError(f"device buffer {name} has {buf.n} values, need {min_n}")
         if kcb.elem != vcb.elem:
             raise TypeError("K and V caches differ in precision")
         return kcb, vcb
@@ -719,7 +734,7 @@ class Runtime:
             raise ValueError(f"invalid rotary dim {rot}")
         xb = self._f32_buffer(x, heads * hd * self._seg_rows())
         for arr, n in self._seg_chunks():
-            _lib.check(self._lib.vq_rope_seg(xb.data_ptr(), arr, n, heads, hd, rot, float(base), self._stream()),
+            _lib.check(self._lib.vq_rope_seg(xb.ptr, arr, n, heads, hd, rot, float(base), self._stream()),
                        "rope_seg")
 
     def kv_append_seg(self, k: str, v: str, kc: str, vc: str, kv_heads: int, hd: int) -> None:
@@ -731,8 +746,8 @@ class Runtime:
         kcb, vcb = self._kv_pair(kc, vc, rowsz)
         pt, page, pps, _ = self._paging
         for arr, n in self._seg_chunks():
-            _lib.check(self._lib.vq_kv_append_seg(kb.data_ptr(), vb.data_ptr(), kcb.data.data_ptr(), vcb.data.data_ptr(),
-                                                  kcb.elem, arr, n, kv_heads, hd, pt.data_ptr(), page, pps,
+            _lib.check(self._lib.vq_kv_append_seg(kb.ptr, vb.ptr, kcb.ptr, vcb.ptr,
+                                                  kcb.elem, arr, n, kv_heads, hd, pt.ptr, page, pps,
                                                   self._stream()), "kv_append_seg")
 
     def attention_seg(self, q: str, kc: str, vc: str, out: str, heads: int, kv_heads: int, hd: int) -> None:
@@ -746,18 +761,18 @@ class Runtime:
         kcb, vcb = self._kv_pair(kc, vc, 1)
         ob = self._f32_buffer(out, rowsz * self._seg_rows())
         pt, page, pps, _ = self._paging
-        tiled = self._tiled_attention(max(r for _, _, r, _ in self._segments))
+        tiled = self._tiled_attention(self._seg_longest)
         for arr, n in self._seg_chunks():
             if tiled:  # prompt rows in the pass, or batch-invariant mode
-                _lib.check(self._lib.vq_attention_seg_tiled(qb.data_ptr(), kcb.data.data_ptr(), vcb.data.data_ptr(),
-                                                            ob.data_ptr(), kcb.elem, arr, n, heads, kv_heads, hd,
-                                                            pt.data_ptr(), page, pps, self._stream()), "attention_seg")
+                _lib.check(self._lib.vq_attention_seg_tiled(qb.ptr, kcb.ptr, vcb.ptr,
+                                                            ob.ptr, kcb.elem, arr, n, heads, kv_heads, hd,
+                                                            pt.ptr, page, pps, self._stream()), "attention_seg")
                 continue
             nws = self._lib.vq_attention_seg_workspace_bytes(arr, n, heads, kv_heads, hd)
             ws = self._workspace(nws).data_ptr() if nws else None
-            _lib.check(self._lib.vq_attention_seg_ws(qb.data_ptr(), kcb.data.data_ptr(), vcb.data.data_ptr(),
-                                                     ob.data_ptr(), kcb.elem, arr, n, heads, kv_heads, hd,
-                                                     pt.data_ptr(), page, pps, ws, nws, self._stream()),
+            _lib.check(self._lib.vq_attention_seg_ws(qb.ptr, kcb.ptr, vcb.ptr,
+                                                     ob.ptr, kcb.elem, arr, n, heads, kv_heads, hd,
+                                                     pt.ptr, page, pps, ws, nws, self._stream()),
                        "attention_seg")
 
     def conv_update_seg(self, x: str, state: str, w: str, out: str, channels: int, K: int, snap: str | None = None,
@@ -776,9 +791,9 @@ class Runtime:
         if snap is not None:
             if len(segs) != 1:
                 raise ValueError("snapshots need a single-segment pass")
-            snp = self._f32_buffer(snap, stride * (ntok - 1)).data_ptr()
+            snp = self._f32_buffer(snap, stride * (ntok - 1)).ptr
         for arr, n in self._seg_chunks():
-            _lib.check(self._lib.vq_conv_update_seg(xb.data_ptr(), sb.data_ptr(), wt.data_ptr(), ob.data_ptr(), channels,
+            _lib.check(self._lib.vq_conv_update_seg(xb.ptr, sb.ptr, wt.ptr, ob.ptr, channels,
                                                     K, arr, n, snp, int(bool(write_state)), self._stream()),
                        "conv_update_seg")
 
@@ -796,8 +811,8 @@ class Runtime:
         cb = self._f32_buffer(conv, conv_dim * ntok)
         bb, ab = self._f32_buffer(b, value_heads * ntok), self._f32_buffer(a, value_heads * ntok)
         sbuf = self._any_buffer(state)
-        if sbuf.data.numel() < state_n * self._paging[3]:
-            raise ValueError(f"device buffer {state} has {sbuf.data.numel()} values, need {state_n * self._paging[3]}")
+        if sbuf.n < state_n * self._paging[3]:
+            raise ValueError(f"device buffer {state} has {sbuf.n} values, need {state_n * self._paging[3]}")
         ob = self._f32_buffer(out, value_heads * vd * ntok)
         sa, dtt = self._f32_weight(ssm_a, value_heads), self._f32_weight(dt, value_heads)
         snp = None
@@ -806,12 +821,12 @@ class Runtime:
                 raise ValueError("fp16 SSM state does not support snapshots")
             if len(segs) != 1:
                 raise ValueError("snapshots need a single-segment pass")
-            snp = self._f32_buffer(snap, state_n * (ntok - 1)).data_ptr()
-        rows = max(r for _, _, r, _ in segs)
+            snp = self._f32_buffer(snap, state_n * (ntok - 1)).ptr
+        rows = self._seg_longest
         for arr, n in self._seg_chunks():
             ws, nws = self._gated_delta_ws(arr, n, rows, key_heads, value_heads, kd, vd, snp)
-            _lib.check(self._lib.vq_gated_delta_seg_ws(cb.data_ptr(), bb.data_ptr(), ab.data_ptr(), sa.data_ptr(),
-                                                       dtt.data_ptr(), sbuf.data.data_ptr(), sbuf.elem, ob.data_ptr(),
+            _lib.check(self._lib.vq_gated_delta_seg_ws(cb.ptr, bb.ptr, ab.ptr, sa.ptr,
+                                                       dtt.ptr, sbuf.ptr, sbuf.elem, ob.ptr,
                                                        key_heads, value_heads, kd, vd, float(eps), int(head_order), arr,
                                                        n, snp, int(bool(write_state)), ws, nws, self._stream()),
                        "gated_delta_seg")
@@ -824,7 +839,7 @@ class Runtime:
         db, sb = self._any_buffer(dst), self._any_buffer(src)
         if db.elem != sb.elem:
             raise TypeError("copy between buffers of different precision")
-        if dst_off + n > db.data.numel() or src_off + n > sb.data.numel():
+        if dst_off + n > db.n or src_off + n > sb.n:
             raise ValueError(f"copy out of bounds ({dst} <- {src})")
         if n:
             db.data[dst_off:dst_off + n].copy_(sb.data[src_off:src_off + n], non_blocking=True)
@@ -850,19 +865,19 @@ class Runtime:
         xb = self._f32_buffer(x, t0.cols * ntok)
         yb = [self._f32_buffer(y, t.rows * ntok) for y, t in zip(ys, ts)]
         n = len(ts)
-        wa = (ctypes.c_void_p * n)(*[t.data.data_ptr() for t in ts])
+        wa = (ctypes.c_void_p * n)(*[t.ptr for t in ts])
         ra = (ctypes.c_int * n)(*[t.rows for t in ts])
-        ya = (ctypes.c_void_p * n)(*[b.data_ptr() for b in yb])
+        ya = (ctypes.c_void_p * n)(*[b.ptr for b in yb])
         if any(t.type != t0.type for t in ts):
             # Mixed types (Q5_K projections with Q8_0 small tensors, or Q5_K with Q6_K): one launch.
             ta = (ctypes.c_int * n)(*[t.type for t in ts])
-            st = self._lib.vq_qmv_group_mixed_f32(n, ta, wa, ra, ya, t0.cols, xb.data_ptr(), ntok, self._stream())
+            st = self._lib.vq_qmv_group_mixed_f32(n, ta, wa, ra, ya, t0.cols, xb.ptr, ntok, self._stream())
         else:
             # One type: the streaming group launch, or for small batches the MFMA paths qmv would take (5-16
             # tokens of Q3_K..Q6_K as one launch over all the matrices).
             nws = self._lib.vq_qmv_group_workspace_bytes(t0.type, n, ra, t0.cols, ntok)
             ws = self._workspace(nws).data_ptr() if nws else None
-            st = self._lib.vq_qmv_group_ws(t0.type, n, wa, ra, ya, t0.cols, xb.data_ptr(), ntok, ws, nws,
+            st = self._lib.vq_qmv_group_ws(t0.type, n, wa, ra, ya, t0.cols, xb.ptr, ntok, ws, nws,
                                            self._stream())
         _lib.check(st, "qmv_group launch")
 
@@ -879,16 +894,16 @@ class Runtime:
         _check_qmv_args(weight, t.cols, ntok)
         xb = self._f32_buffer(x, t.cols * ntok)
         if self.batch_invariant:  # the matvec on the invariant path, then the row argmax
-            yt = (self._f32_buffer(logits, t.rows * ntok) if logits is not None
-                  else self._logits_scratch(t.rows * ntok))
-            self._qmv_ptrs(t, xb.data_ptr(), yt.data_ptr(), ntok)
-            _lib.check(self._lib.vq_argmax_rows(yt.data_ptr(), t.rows, ntok, self._argmax_out.data_ptr(),
+            yp = (self._f32_buffer(logits, t.rows * ntok).ptr if logits is not None
+                  else self._logits_scratch(t.rows * ntok).data_ptr())
+            self._qmv_ptrs(t, xb.ptr, yp, ntok)
+            _lib.check(self._lib.vq_argmax_rows(yp, t.rows, ntok, self._argmax_out.data_ptr(),
                                                 self._stream()), "argmax_rows")
             return [int(v) for v in self._argmax_out[:ntok].tolist()]
-        lp = self._f32_buffer(logits, t.rows * ntok).data_ptr() if logits is not None else None
+        lp = self._f32_buffer(logits, t.rows * ntok).ptr if logits is not None else None
         nws = self._lib.vq_lmhead_argmax_workspace_bytes(t.type, t.rows, t.cols, ntok)
         ws = self._workspace(nws)
-        st = self._lib.vq_lmhead_argmax(t.type, t.data.data_ptr(), t.rows, t.cols, xb.data_ptr(), ntok,
+        st = self._lib.vq_lmhead_argmax(t.type, t.ptr, t.rows, t.cols, xb.ptr, ntok,
                                         self._argmax_out.data_ptr(), lp, ws.data_ptr(), nws, self._stream())
         _lib.check(st, "lmhead_argmax")
         return [int(v) for v in self._argmax_out[:ntok].tolist()]
@@ -926,7 +941,7 @@ class Runtime:
     def argmax(self, name: str, n: int) -> int:
         """Index of the largest of the first n floats; ties -> lowest index (Runtime_argmax, :2167-2179)."""
         xb = self._f32_buffer(name, n)
-        _lib.check(self._lib.vq_argmax_rows(xb.data_ptr(), n, 1, self._argmax_out.data_ptr(), self._stream()), "argmax")
+        _lib.check(self._lib.vq_argmax_rows(xb.ptr, n, 1, self._argmax_out.data_ptr(), self._stream()), "argmax")
         return int(self._argmax_out[0].item())
 
     def argmax_rows(self, name: str, n: int, ntok: int) -> list[int]:
@@ -934,7 +949,7 @@ class Runtime:
         if ntok < 1 or ntok > MAX_ARGMAX_ROWS:
             raise ValueError(f"ntok must be in [1, {MAX_ARGMAX_ROWS}]")
         xb = self._f32_buffer(name, n * ntok)
-        _lib.check(self._lib.vq_argmax_rows(xb.data_ptr(), n, ntok, self._argmax_out.data_ptr(), self._stream()),
+        _lib.check(self._lib.vq_argmax_rows(xb.ptr, n, ntok, self._argmax_out.data_ptr(), self._stream()),
                    "argmax_rows")
         return [int(v) for v in self._argmax_out[:ntok].tolist()]
 
