@@ -205,3 +205,30 @@ def test_gated_delta_chunks_keep_causality(rt, oracle_mod, what):
     if what == "v":
         rest = np.arange(vd) != 3
         assert np.abs(out[:, 0, rest] - clean[:, 0, rest]).max() <= 2e-6 * np.abs(clean).max()
+
+
+# Key blocks of 32 in two parities, 16-row tiles, three or four heads of a kv head per workgroup.
+@pytest.mark.parametrize("heads,kvh,hd", [(6, 1, 256), (5, 1, 64), (6, 2, 128), (9, 1, 64), (2, 2, 256)])
+@pytest.mark.parametrize("ntok,seq_len,window", [(9, 1, 0), (9, 24, 0), (16, 49, 0), (17, 48, 0), (33, 1, 5),
+                                                 (20, 97, 40), (18, 64, 32)])
+def test_prompt_attention_f16_blocks(rt, oracle_mod, heads, kvh, hd, ntok, seq_len, window):
+    """The last key just before, on and after a block's and a step's edge, one parity without a key, windows that
+    begin inside a block. Bar: that of the prompt attention tests (fp32 products and sums; splitting the keys in two
+    shortens each chain of sums). A row's bits do not depend on the rows before it in the pass."""
+    rng = np.random.default_rng(1000 * heads + hd + ntok + seq_len)
+    max_seq = seq_len + ntok
+    q = rng.standard_normal((ntok, heads, hd)).astype(np.float32)
+    kc = (rng.standard_normal((kvh, max_seq, hd)) * 0.3).astype(np.float16)
+    vc = rng.standard_normal((kvh, max_seq, hd)).astype(np.float16)
+    put(rt, "pq", q)
+    put(rt, "po", np.full(q.size, np.nan))
+    put(rt, "pkc", kc, 2)
+    put(rt, "pvc", vc, 2)
+    rt.attention("pq", "pkc", "pvc", "po", heads, kvh, hd, max_seq, seq_len, ntok, 0, window)
+    got = get(rt, "po", q.shape)
+    ref = oracle_mod.attention(q, kc, vc, heads, kvh, seq_len, False, window)
+    assert np.allclose(got, ref, rtol=2e-5, atol=2e-5)
+    skip = ntok - 9
+    put(rt, "pq", q[skip:])
+    rt.attention("pq", "pkc", "pvc", "po", heads, kvh, hd, max_seq, seq_len + skip, 9, 0, window)
+    assert np.array_equal(get(rt, "po", q.shape)[:9], got[skip:])

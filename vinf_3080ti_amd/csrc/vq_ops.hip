@@ -81,8 +81,13 @@ struct KvMap {
     // keep the loads that follow in flight (a load under a branch makes it wait for every outstanding load).
     template <bool PAGED>
     __device__ __forceinline__ size_t row_t(int slot, int kvh, int pos) const {
+        return row_in<PAGED>(PAGED ? page_of(slot, pos) : 0, kvh, pos);
+    }
+    // The lookup in two parts, for a caller with other work between the page's load and its use.
+    __device__ __forceinline__ int page_of(int slot, int pos) const { return pt[slot * pps + pos / page]; }
+    template <bool PAGED>
+    __device__ __forceinline__ size_t row_in(int pg, int kvh, int pos) const {
         if constexpr (!PAGED) return static_cast<size_t>(kvh) * max_seq + pos;
-        const int pg = pt[slot * pps + pos / page];
         return (static_cast<size_t>(pg) * kv_heads + kvh) * page + pos % page;
     }
 };
@@ -764,6 +769,21 @@ __device__ __forceinline__ void fa16_issue(const _Float16 *__restrict__ kc, cons
     }
 }
 
+// Order of a run of N LDS reads that feed two MFMAs each: kFaAhead reads in flight ahead of the products. Left alone
+// the compiler reads two, waits for them and multiplies: a read's latency for every four products.
+constexpr int kFaAhead = 4;
+template <int N>
+__device__ __forceinline__ void fa16_ahead() {
+    constexpr int kMfma = 0x8, kDsRead = 0x100;
+    __builtin_amdgcn_sched_group_barrier(kDsRead, kFaAhead, 0);
+#pragma unroll
+    for (int i = 0; i < N - kFaAhead; ++i) {
+        __builtin_amdgcn_sched_group_barrier(kMfma, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(kMfma, 2 * kFaAhead, 0);
+}
+
 // Online softmax over the S^T values of block [kb, kb + 32) (s[h][r]: key kb + 16 h + 4 g + r, query column c sees
 // keys [qs, qe), keys at or past k_hi masked), then O^T += V^T P^T from the block's V^T in LDS (vt, read at rows
 // 16 b + c, positions 8 g ..). The caller makes vt visible first.
@@ -773,22 +793,25 @@ __device__ __forceinline__ void fa16_softmax_pv(const fa4 (&s)[2], int kb, int k
     const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
     float v[8], bm = -INFINITY;
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int j = 0; j < 8; ++j) v[j] = s[j >> 2][j & 3];
+    if (__any(kb < qs || kb + 32 > min(qe, k_hi))) {  // a block that some query's range cuts
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int p = kb + 16 * h + 4 * g + r;
-            v[4 * h + r] = p >= qs && p < qe && p < k_hi ? s[h][r] : -INFINITY;
-            bm = fmaxf(bm, v[4 * h + r]);
+        for (int j = 0; j < 8; ++j) {
+            const int p = kb + 16 * (j >> 2) + 4 * g + (j & 3);
+            v[j] = p >= qs && p < qe && p < k_hi ? v[j] : -INFINITY;
         }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) bm = fmaxf(bm, v[j]);
     bm = xor16_max(bm);
     bm = xor32_max(bm);
-    const float mn = fmaxf(m, bm);
-    const float alpha = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
+    const float mn = fmaxf(m, bm), ms = mn == -INFINITY ? 0.0f : mn;  // ms: exp2(-inf - ms) is 0 also before any key
+    const float alpha = __builtin_amdgcn_exp2f(m - ms);
     fh8 ph, pl;
     float ps = 0.0f;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-        const float p = v[j] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(v[j] - mn);
+        const float p = __builtin_amdgcn_exp2f(v[j] - ms);
         ps += p;
         _Float16 hh, ll;
         split_h(p, hh, ll);
@@ -799,13 +822,17 @@ __device__ __forceinline__ void fa16_softmax_pv(const fa4 (&s)[2], int kb, int k
     ps = xor32_add(ps);
     l = l * alpha + ps;
     m = mn;
+    if (__any(alpha != 1.0f)) {  // the maximum of most blocks after the first few is an earlier block's
+#pragma unroll
+        for (int b = 0; b < HD / 16; ++b) o[b] *= alpha;
+    }
 #pragma unroll
     for (int b = 0; b < HD / 16; ++b) {
         const fh8 a = *reinterpret_cast<const fh8 *>(vt + fa16_vt(16 * b + c, 8 * g));
-        fa4 ob = o[b] * alpha;
-        ob = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, ph, ob, 0, 0, 0);
-        o[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, pl, ob, 0, 0, 0);
+        o[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, ph, o[b], 0, 0, 0);
+        o[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, pl, o[b], 0, 0, 0);
     }
+    fa16_ahead<HD / 16>();
 }
 
 // V unit (key quad qd, 16-byte chunk dc) of a block into V^T: eight 8-byte writes (four keys of one dim at
@@ -854,31 +881,46 @@ __device__ __forceinline__ void fa16_consume(const Fa16Raw<HD> &rw, int kb, int 
 }
 
 // Prompt passes on fp16 caches: a workgroup takes 16 query rows of one segment and up to four query heads of one kv
-// head (one wave each). Its 256 threads stage each 32-key block once for all four: K row-major [32][HD + 8] f16
-// (the S^T A fragments are 16-byte reads, rows 528 bytes apart for HD 256: no two of a read's 16 rows share banks),
-// V^T as in the decode kernel; the next two blocks' loads are in flight while one is used.
+// head. Wave w takes head w >> 1 and every second 32-key block (the blocks of parity w & 1) with its own online softmax;
+// the two waves of a head are combined through LDS at the end. Blocks start at multiples of 32 keys whatever the rows
+// of the tile, so a row's sums do not depend on the other rows of its pass.
+// Each step (64 keys, one block per parity): all 512 threads load the next step's K and V into registers, the waves
+// consume the present one from LDS, the registers go to the other LDS buffer: one barrier per step. The loads are
+// issued after the S products, which would otherwise wait behind them in the address unit. K is [32][HD + 16] f16
+// (the S^T A fragments are 16-byte reads; 95 us against 96 with rows of HD + 8), V^T as in the decode kernel. The cache
+// rows of a step's keys are looked up once per workgroup, two steps ahead.
+// Why: one wave per SIMD (290 registers, two blocks in flight) left every read, conversion and barrier exposed, and
+// three heads for each half of the waves keep all 256 CUs at work where four and two did not. 512 rows over 2048 keys,
+// 24 heads of 256 on 4 kv heads: 167 -> 76 us (45 GFLOP issued, 590 TFLOP/s). Two waves of a SIMD need 2090 cycles of
+// matrix products and 1900 of other vector instructions per step and do both in step; giving one of them priority
+// changed nothing.
 template <int HD, bool PAGED>
-__global__ __launch_bounds__(256) void attention_prompt16_kernel(const float *__restrict__ q,
+__global__ __launch_bounds__(512) void attention_prompt16_kernel(const float *__restrict__ q,
                                                                  const _Float16 *__restrict__ kc,
                                                                  const _Float16 *__restrict__ vc, float *__restrict__ out,
                                                                  SegTable T, KvMap M, int heads, int bidirectional,
-                                                                 int window, int chunks) {
-    constexpr int CR = HD / 8, LDK = HD + 8;
-    constexpr int KU = 32 * CR / 256;  // K chunks per thread per block
-    constexpr int VU = 8 * CR / 256;   // V units per thread per block (HD 64: half the threads take one)
-    __shared__ __align__(16) _Float16 ks[32 * LDK];
-    __shared__ __align__(16) _Float16 vts[HD * 32];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int c = lane & 15, g = lane >> 4;
-    int tb = blockIdx.x, si = 0;
+                                                                 int window, int chunks, int hpw) {
+    constexpr int CR = HD / 8, LDK = HD + 16;
+    constexpr int KU = 32 * CR / 256;                  // K chunks per thread per block
+    constexpr int VU = 8 * CR / 256 > 0 ? 8 * CR / 256 : 1;  // V units (HD 64: half the threads take one)
+    constexpr int KB = 32 * LDK, VB = HD * 32;         // f16 elements of a staged block
+    __shared__ __align__(16) _Float16 kv[2][2][KB + VB];  // [buffer][parity]
+    __shared__ __align__(16) size_t rowtab[2][64];     // first element of the cache row of a step's keys
+    __shared__ float sml[4][2][16];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int c = lane & 15, g = lane >> 4, par = wv & 1;
+    // Consecutive workgroups take the kv heads in turn (with 8 (kv head, chunk) pairs each XCD's L2 holds one kv head),
+    // the last tiles, which see the most keys, first.
+    const int per = M.kv_heads * chunks, kvc = blockIdx.x % per, kvh = kvc / chunks, gi0 = (kvc - kvh * chunks) * hpw;
+    int tb = gridDim.x / per - 1 - blockIdx.x / per, si = 0;
     while (si + 1 < T.n && tb >= (T.s[si].rows + 15) / 16) {
         tb -= (T.s[si].rows + 15) / 16;
         ++si;
     }
     const Seg &s = T.s[si];
     const int G = heads / M.kv_heads;
-    const int kvh = blockIdx.y / chunks, gi = (blockIdx.y - kvh * chunks) * 4 + wv;
-    const bool wave_on = gi < G;
+    const int gi = gi0 + (wv >> 1);
+    const bool wave_on = (wv >> 1) < hpw && gi < G;
     const int h = kvh * G + (wave_on ? gi : 0);
     const int t0 = 16 * tb, nq = min(16, s.rows - t0);
     const int seq_len0 = s.pos0 + 1;
@@ -887,81 +929,119 @@ __global__ __launch_bounds__(256) void attention_prompt16_kernel(const float *__
     const int tq = t0 + min(c, nq - 1);  // this lane's query row (rows past nq repeat the last; not written)
     const int qs = q_start(tq), qe = q_end(tq);
     const int k_lo = q_start(t0), k_hi = q_end(t0 + nq - 1);
+    const int k0 = k_lo & ~63, steps = (k_hi - k0 + 63) / 64;
+    // Keys outside [k_lo, k_hi) read the nearest key of the range (they are masked).
+    auto key_of = [&](int step) { return min(max(k0 + 64 * step + lane, k_lo), k_hi - 1); };
+    if (wv < 2) rowtab[wv][lane] = M.row_t<PAGED>(s.slot, kvh, key_of(wv)) * HD;
     float4 qr[HD / 16];
     fa16_q_load<HD>(q + (static_cast<size_t>(s.row0 + tq) * heads + h) * HD, qr);
-    // Block loads of this thread: K chunks i = tid + 256 k (key i / CR, chunk i % CR); V unit tid (key quad tid & 7,
-    // chunk tid >> 3).
-    // Two blocks are in flight ahead of the one being used (register buffers A and B).
-    struct Buf {
-        fh8 k[KU];
-        fh8 v[VU > 0 ? VU : 1][4];
-    };
-    auto row_of = [&](int key) { return M.row_t<PAGED>(s.slot, kvh, min(key, k_hi - 1)); };
-    auto issue = [&](Buf &bf, int kb) {
+    __syncthreads();
+    // Half sp of the threads stages the block of parity sp: K chunks i = st + 256 k (key i / CR, chunk i % CR), V units
+    // st + 256 k (key quad & 7, chunk >> 3).
+    const int sp = tid >> 8, st = tid & 255;
+    fh8 rk[KU], rv[VU][4];
+    auto issue_k = [&](int step) {
+        const size_t *rt = rowtab[step & 1] + 32 * sp;
 #pragma unroll
         for (int k = 0; k < KU; ++k) {
-            const int i = threadIdx.x + 256 * k;
-            bf.k[k] = ld_h8(kc + row_of(kb + i / CR) * HD + 8 * (i % CR));
-        }
-#pragma unroll
-        for (int k = 0; k < (VU > 0 ? VU : 1); ++k) {
-            const int i = threadIdx.x + 256 * k;
-            if (i < 8 * CR)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) bf.v[k][j] = ld_h8(vc + row_of(kb + 4 * (i & 7) + j) * HD + 8 * (i >> 3));
+            const int i = st + 256 * k;
+            rk[k] = ld_h8(kc + rt[i / CR] + 8 * (i % CR));
         }
     };
-    Buf ba, bb;
-    if (k_lo < k_hi) issue(ba, k_lo);
-    if (k_lo + 32 < k_hi) issue(bb, k_lo + 32);
+    auto issue_v = [&](int step) {
+        const size_t *rt = rowtab[step & 1] + 32 * sp;
+#pragma unroll
+        for (int k = 0; k < VU; ++k) {
+            const int i = (st + 256 * k) % (8 * CR);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) rv[k][j] = ld_h8(vc + rt[4 * (i & 7) + j] + 8 * (i >> 3));
+        }
+    };
+    auto stage = [&](int step) {
+        _Float16 *kd = kv[step & 1][sp], *vd = kd + KB;
+#pragma unroll
+        for (int k = 0; k < KU; ++k) {
+            const int i = st + 256 * k;
+            *reinterpret_cast<fh8 *>(kd + (i / CR) * LDK + 8 * (i % CR)) = rk[k];
+        }
+#pragma unroll
+        for (int k = 0; k < VU; ++k) {
+            const int i = st + 256 * k;
+            if (i < 8 * CR) fa16_put_vt<HD>(vd, i & 7, i >> 3, rv[k]);
+        }
+    };
+    issue_k(0);
+    issue_v(0);
     fh8 qh[HD / 32], ql[HD / 32];
     const float sinv = fa16_q_split<HD>(qr, 1.0f / sqrtf(static_cast<float>(HD)), qh, ql);
     float m = -INFINITY, l = 0.0f;
     fa4 o[HD / 16];
 #pragma unroll
     for (int b = 0; b < HD / 16; ++b) o[b] = fa4{0.f, 0.f, 0.f, 0.f};
-    auto consume = [&](Buf &bf, int kb) {
-        __syncthreads();  // the previous block is consumed
-#pragma unroll
-        for (int k = 0; k < KU; ++k) {
-            const int i = threadIdx.x + 256 * k;
-            *reinterpret_cast<fh8 *>(ks + (i / CR) * LDK + 8 * (i % CR)) = bf.k[k];
+    stage(0);
+    __syncthreads();
+    for (int step = 0; step < steps; ++step) {
+        const bool more = step + 1 < steps;
+        const int nkey = key_of(step + 2);
+        int npage = 0;
+        if (PAGED && wv == 7) npage = M.page_of(s.slot, nkey);
+        if (!wave_on) {
+            issue_k(step + 1);
+            issue_v(step + 1);
         }
+        if (wave_on) {
+            const _Float16 *ks = kv[step & 1][par], *vts = ks + KB;
+            fa4 sc[2];
 #pragma unroll
-        for (int k = 0; k < (VU > 0 ? VU : 1); ++k) {
-            const int i = threadIdx.x + 256 * k;
-            if (i < 8 * CR) fa16_put_vt<HD>(vts, i & 7, i >> 3, bf.v[k]);
-        }
-        __syncthreads();
-        if (kb + 64 < k_hi) issue(bf, kb + 64);
-        if (!wave_on) return;
-        fa4 sc[2];
+            for (int hh = 0; hh < 2; ++hh) {
+                fa4 a0{0.f, 0.f, 0.f, 0.f}, a1{0.f, 0.f, 0.f, 0.f};
+                const _Float16 *kp = ks + (16 * hh + c) * LDK + 8 * g;
 #pragma unroll
-        for (int hh = 0; hh < 2; ++hh) {
-            fa4 a0{0.f, 0.f, 0.f, 0.f}, a1{0.f, 0.f, 0.f, 0.f};
-            const _Float16 *kp = ks + (16 * hh + c) * LDK + 8 * g;
-#pragma unroll
-            for (int u = 0; u < HD / 32; ++u) {
-                const fh8 a = *reinterpret_cast<const fh8 *>(kp + 32 * u);
-                a0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qh[u], a0, 0, 0, 0);
-                a1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, ql[u], a1, 0, 0, 0);
+                for (int u = 0; u < HD / 32; ++u) {
+                    const fh8 a = *reinterpret_cast<const fh8 *>(kp + 32 * u);
+                    a0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qh[u], a0, 0, 0, 0);
+                    a1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, ql[u], a1, 0, 0, 0);
+                }
+                sc[hh] = (a0 + a1) * sinv;
             }
-            sc[hh] = (a0 + a1) * sinv;
+            fa16_ahead<HD / 16>();
+            __builtin_amdgcn_sched_barrier(0);
+            issue_k(step + 1);
+            issue_v(step + 1);
+            fa16_softmax_pv<HD>(sc, k0 + 64 * step + 32 * par, k_hi, qs, qe, vts, m, l, o);
         }
-        fa16_softmax_pv<HD>(sc, kb, k_hi, qs, qe, vts, m, l, o);
-    };
-    for (int kb = k_lo; kb < k_hi; kb += 64) {
-        consume(ba, kb);
-        if (kb + 32 < k_hi) consume(bb, kb + 32);
+        if (more) stage(step + 1);
+        if (wv == 7) rowtab[step & 1][lane] = M.row_in<PAGED>(npage, kvh, nkey) * HD;
+        __syncthreads();
     }
-    // o[b][r]: head dim 16 b + 4 g + r of query row tq
-    if (wave_on && c < nq) {
-        float *orow = out + (static_cast<size_t>(s.row0 + t0 + c) * heads + h) * HD;
-        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    // Wave 2 i + 1 hands its sums to wave 2 i (same lane layout): 16 query vectors x HD fp32 per head.
+    float *oh = reinterpret_cast<float *>(&kv[0][0][0]) + (wv >> 1) * 16 * HD;
+    if (par == 1) {
 #pragma unroll
-        for (int b = 0; b < HD / 16; ++b)
-            *reinterpret_cast<float4 *>(orow + 16 * b + 4 * g) =
-                float4{o[b][0] * inv, o[b][1] * inv, o[b][2] * inv, o[b][3] * inv};
+        for (int b = 0; b < HD / 16; ++b) *reinterpret_cast<fa4 *>(oh + 256 * b + 4 * lane) = o[b];
+        if (g == 0) {
+            sml[wv >> 1][0][c] = m;
+            sml[wv >> 1][1][c] = l;
+        }
+    }
+    __syncthreads();
+    // o[b][r]: head dim 16 b + 4 g + r of query row tq
+    if (wave_on && par == 0 && c < nq) {
+        float *orow = out + (static_cast<size_t>(s.row0 + t0 + c) * heads + h) * HD;
+        const float m1 = sml[wv >> 1][0][c], l1 = sml[wv >> 1][1][c];
+        const float mx = fmaxf(m, m1);
+        const float f0 = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mx);
+        const float f1 = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m1 - mx);
+        const float lt = fmaf(l1, f1, l * f0);
+        const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
+#pragma unroll
+        for (int b = 0; b < HD / 16; ++b) {
+            const fa4 o1 = *reinterpret_cast<const fa4 *>(oh + 256 * b + 4 * lane);
+            float r[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) r[j] = fmaf(o1[j], f1, o[b][j] * f0) * inv;
+            *reinterpret_cast<float4 *>(orow + 16 * b + 4 * g) = float4{r[0], r[1], r[2], r[3]};
+        }
     }
 }
 
@@ -1569,15 +1649,18 @@ void launch_mfma_hd(bool fast, dim3 grid, hipStream_t s, const float *q, const C
                                                                 chunks);
 }
 
+// Query heads per workgroup: a kv head's heads dealt evenly over as few workgroups as four heads each allow (6: 3 + 3).
 template <bool PAGED>
-void launch_prompt16(dim3 grid, hipStream_t s, const float *q, const _Float16 *kc, const _Float16 *vc, float *out,
+void launch_prompt16(int tiles, hipStream_t s, const float *q, const _Float16 *kc, const _Float16 *vc, float *out,
                      const SegTable &T, const KvMap &M, int heads, int hd, int bidirectional, int window, int chunks) {
+    const int G = heads / M.kv_heads, hpw = (G + chunks - 1) / chunks;
+    const dim3 grid(static_cast<unsigned>(tiles) * M.kv_heads * chunks);
     if (hd == 64)
-        attention_prompt16_kernel<64, PAGED><<<grid, 256, 0, s>>>(q, kc, vc, out, T, M, heads, bidirectional, window, chunks);
+        attention_prompt16_kernel<64, PAGED><<<grid, 512, 0, s>>>(q, kc, vc, out, T, M, heads, bidirectional, window, chunks, hpw);
     else if (hd == 128)
-        attention_prompt16_kernel<128, PAGED><<<grid, 256, 0, s>>>(q, kc, vc, out, T, M, heads, bidirectional, window, chunks);
+        attention_prompt16_kernel<128, PAGED><<<grid, 512, 0, s>>>(q, kc, vc, out, T, M, heads, bidirectional, window, chunks, hpw);
     else
-        attention_prompt16_kernel<256, PAGED><<<grid, 256, 0, s>>>(q, kc, vc, out, T, M, heads, bidirectional, window, chunks);
+        attention_prompt16_kernel<256, PAGED><<<grid, 512, 0, s>>>(q, kc, vc, out, T, M, heads, bidirectional, window, chunks, hpw);
 }
 
 // fp16 caches with hd 64, 128 or 256 and 16-byte aligned q, K, V and out: the f16 MFMA kernels.
@@ -1596,8 +1679,8 @@ void launch_attention_mfma(const float *q, const C *kc, const C *vc, float *out,
     const dim3 grid(tiles, M.kv_heads * chunks);
     if constexpr (sizeof(C) == 2) {
         if (fa16_ok(q, kc, vc, out, hd)) {
-            if (M.pt != nullptr) launch_prompt16<true>(grid, s, q, kc, vc, out, T, M, heads, hd, bidirectional, window, chunks);
-            else launch_prompt16<false>(grid, s, q, kc, vc, out, T, M, heads, hd, bidirectional, window, chunks);
+            if (M.pt != nullptr) launch_prompt16<true>(tiles, s, q, kc, vc, out, T, M, heads, hd, bidirectional, window, chunks);
+            else launch_prompt16<false>(tiles, s, q, kc, vc, out, T, M, heads, hd, bidirectional, window, chunks);
             return;
         }
     }
