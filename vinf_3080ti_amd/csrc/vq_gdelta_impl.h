@@ -9,17 +9,20 @@
 //   S_C = G_C S0 + sum_i D(C - 1, i) k_i d_i^T
 // so with T = (I + L)^-1 everything that meets the state is a matrix product:
 //   d = T (b V - (b G) K S0),   o = G (Q S0) + P d,   S_C = G_C S0 + (D(C - 1, .) K)^T d.
-// All of it in fp32 (v_mfma_f32_16x16x4_f32, fp32 operands and sums, long sums in four chains): against float64 at 512
-// tokens rel-L2 1.6e-7 (outputs) and 1.7e-7 (state); the per-token kernel 1.4e-7 and 1.6e-7.
+// All of it in fp32 (v_mfma_f32_16x16x4_f32, fp32 operands and sums), with care for the roundings in a row: long sums in
+// eight chains, the sums over a chunk's tokens from zero, decays, pair factors and the diagonal blocks of T in fp64 and
+// rounded once. Against float64 at 512 tokens rel-L2 1.4-1.5e-7 (outputs) and 1.5-1.7e-7 (state) over three inputs; the
+// per-token kernel 1.4e-7 and 1.4-1.7e-7. In four chains, with fp32 decays, it was 1.65e-7 (and 54.5 us for the walk).
 //
 // Two launches. gd_prep_kernel, one workgroup per (chunk, value head), all chunks at once: T and P into the workspace in
 // MFMA operand order, and the tokens' scales. gd_chunk_kernel, one workgroup per (value head, 32 state columns), walks
 // the chunks with its part of the state in accumulators, the chunk's K, Q, V rows and T, P reaching LDS by DMA a chunk
 // ahead: 116-120 MFMAs per wave and two barriers per 32 tokens, instead of 32 serial tokens of two barriers each. What bounds
-// it: the serial chunk walk's MFMA issue (33 cycles each, 1.9 us of a chunk's 3.3, on 192 of 256 CUs). Operands prepared in full
+// it: the serial chunk walk's MFMA issue (33 cycles each, 1.9 us of a chunk's 3.7, on 192 of 256 CUs). Operands prepared in full
 // (W = T diag(b G) K, scaled Q and K in operand order, read straight into registers) moved 55 KB per chunk and
 // workgroup through L2 twice and took 28 + 56 us. Measured at 16 key and 48 value heads, kd = vd = 128, 512 tokens:
-// 13.8 + 54.5 us against 358 us token by token. Of a chunk's 6800 cycles the K S0 and Q S0 products take 3500 (their
+// 15.4 + 59.6 us against 358 us token by token. Before the eight chains, of a chunk's 6800 cycles the K S0 and Q S0
+// products took 3500 (their
 // 64 MFMAs 2100; the rest are the copies and LDS reads of the one wave per SIMD), T R 690, the state update 1720; eight
 // waves of 32 rows measured 62 us (more operand reads and a four-way exchange), one copy per four MFMAs 57 us.
 //
@@ -71,8 +74,9 @@ __device__ __forceinline__ gc_f4 gc_ld(const float *p) { return *reinterpret_cas
 __global__ __launch_bounds__(256) void gd_prep_kernel(GcArgs A, SegTable T) {
     constexpr int RS = kGcKd + 4;  // LDS row pitch (floats)
     __shared__ __align__(16) float sK[kGcC][RS], sQ[kGcC][RS];
-    __shared__ __align__(16) float sL[kGcC][36], sT[kGcC][36], sD[kGcC][33];
-    __shared__ float sB[kGcC], sG[kGcC], sGt[kGcC], sQs[kGcC], sKs[kGcC];
+    __shared__ __align__(16) float sL[kGcC][36], sT[kGcC][36];
+    __shared__ double sD[kGcC][33], sGt[kGcC];
+    __shared__ float sB[kGcC], sG[kGcC], sQs[kGcC], sKs[kGcC];
     __shared__ int s_bad;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, lr = lane & 15, lk = lane >> 4;
     const int h = blockIdx.x, c = A.c0 + blockIdx.y;
@@ -131,16 +135,18 @@ __global__ __launch_bounds__(256) void gd_prep_kernel(GcArgs A, SegTable T) {
     if (bad) s_bad = 1;
     __syncthreads();
     // 3. Decays of the pairs: lane i of wave 0 walks D(t, i) down its column; lane 32 the decay since the chunk's start.
-    // The other waves meanwhile start on their products.
+    // The other waves meanwhile start on their products. The running products and the pairs' factors are fp64, rounded
+    // once where they become operands.
     if (tid < kGcC) {
-        float d = 1.0f;
+        double d = 1.0;
 #pragma unroll
         for (int t = 0; t < kGcC; ++t) {
-            d = t <= tid ? 1.0f : d * sG[t];
-            sD[t][tid] = t < tid ? 0.0f : d;
+            d = t <= tid ? 1.0 : d * sG[t];
+            sD[t][tid] = t < tid ? 0.0 : d;
         }
     } else if (tid == kGcC) {
-        float d = 1.0f, grow = 1.0f;
+        double d = 1.0;
+        float grow = 1.0f;
 #pragma unroll
         for (int t = 0; t < kGcC; ++t) {
             d *= sG[t];
@@ -151,51 +157,57 @@ __global__ __launch_bounds__(256) void gd_prep_kernel(GcArgs A, SegTable T) {
     }
     // 4. Wave (jt, ji): the 16 x 16 tiles L (rows t, columns i) and P^T (rows i, columns t); nothing above the diagonal.
     const int jt = wv >> 1, ji = wv & 1;
-    gc_f4 kk = {0.f, 0.f, 0.f, 0.f}, kq = kk, kc4[4] = {kk, kk, kk, kk}, qc4[4] = {kk, kk, kk, kk};
-    if (ji <= jt) {  // four chains each, as in the walk
+    gc_f4 kk = {0.f, 0.f, 0.f, 0.f}, kq = kk, kc8[8], qc8[8];
+    if (ji <= jt) {  // eight chains each
+#pragma unroll
+        for (int q = 0; q < 8; ++q) kc8[q] = qc8[q] = kk;
 #pragma unroll
         for (int cc = 0; cc < kGcKd / 16; ++cc) {
             const gc_f4 kt = gc_ld(&sK[16 * jt + lr][16 * cc + 4 * lk]), ki = gc_ld(&sK[16 * ji + lr][16 * cc + 4 * lk]),
                         qt = gc_ld(&sQ[16 * jt + lr][16 * cc + 4 * lk]);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                kc4[q] = gc_mfma(kt[q], ki[q], kc4[q]);
-                qc4[q] = gc_mfma(ki[q], qt[q], qc4[q]);
+                const int e = 4 * (cc & 1) + q;
+                kc8[e] = gc_mfma(kt[q], ki[q], kc8[e]);
+                qc8[e] = gc_mfma(ki[q], qt[q], qc8[e]);
             }
         }
-        kk = (kc4[0] + kc4[1]) + (kc4[2] + kc4[3]);
-        kq = (qc4[0] + qc4[1]) + (qc4[2] + qc4[3]);
+        kk = ((kc8[0] + kc8[1]) + (kc8[2] + kc8[3])) + ((kc8[4] + kc8[5]) + (kc8[6] + kc8[7]));
+        kq = ((qc8[0] + qc8[1]) + (qc8[2] + qc8[3])) + ((qc8[4] + qc8[5]) + (qc8[6] + qc8[7]));
     }
     __syncthreads();
     gc_f4 p;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         const int t = 16 * jt + 4 * lk + q, i = 16 * ji + lr;
-        sL[t][i] = i < t ? sB[t] * sD[t][i] * (sKs[t] * sKs[i]) * kk[q] : 0.0f;
+        const double ks = sKs[t], qs = sQs[16 * jt + lr];
+        sL[t][i] = i < t ? static_cast<float>(sB[t] * sD[t][i] * (ks * sKs[i]) * kk[q]) : 0.0f;
         const int pt = 16 * jt + lr, pi = 16 * ji + 4 * lk + q;
-        p[q] = pi <= pt ? sD[pt][pi] * (sQs[pt] * sKs[pi]) * kq[q] : 0.0f;
+        p[q] = pi <= pt ? static_cast<float>(sD[pt][pi] * (qs * sKs[pi]) * kq[q]) : 0.0f;
     }
     *reinterpret_cast<gc_f4 *>(ws + GcSlot::P + ((jt * 2 + ji) * 64 + lane) * 4) = p;
     if (tid < kGcC) {
         float *const sc = ws + GcSlot::SC;
-        sc[GcSlot::KW + tid] = sB[tid] * sGt[tid] * sKs[tid];
+        const double ks = sKs[tid];
+        const float gc = static_cast<float>(sGt[kGcC - 1]);
+        sc[GcSlot::KW + tid] = static_cast<float>(sB[tid] * sGt[tid] * ks);
         sc[GcSlot::B + tid] = sB[tid];
-        sc[GcSlot::KC + tid] = sD[kGcC - 1][tid] * sKs[tid];
-        sc[GcSlot::QG + tid] = sGt[tid] * sQs[tid];
-        if (tid == 0) sc[GcSlot::GC] = sGt[kGcC - 1], sc[GcSlot::BAD] = s_bad || gc_bad(sGt[kGcC - 1]) ? 1.0f : 0.0f;
+        sc[GcSlot::KC + tid] = static_cast<float>(sD[kGcC - 1][tid] * ks);
+        sc[GcSlot::QG + tid] = static_cast<float>(sGt[tid] * sQs[tid]);
+        if (tid == 0) sc[GcSlot::GC] = gc, sc[GcSlot::BAD] = s_bad || gc_bad(gc) ? 1.0f : 0.0f;
     }
     __syncthreads();
     // 5. T = (I + L)^-1: the two diagonal blocks by forward substitution (lane = column), then T21 = -T22 (L21 T11).
     if (wv < 2 && lane < 16) {
         const int o = 16 * wv;
-        float x[16];
+        double x[16];
 #pragma unroll
         for (int t = 0; t < 16; ++t) {
-            float v = t == lane ? 1.0f : 0.0f;
+            double v = t == lane ? 1.0 : 0.0;
 #pragma unroll
-            for (int i = 0; i < t; ++i) v = fmaf(-sL[o + t][o + i], x[i], v);
+            for (int i = 0; i < t; ++i) v = fma(-static_cast<double>(sL[o + t][o + i]), x[i], v);
             x[t] = v;
-            sT[o + t][o + lane] = v;
+            sT[o + t][o + lane] = static_cast<float>(v);
         }
     }
     __syncthreads();
@@ -320,15 +332,20 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
 #pragma unroll
         for (int i = 0; i < 4; ++i) qa[0][i] = a_row(f.q, 0, i), qa[1][i] = a_row(f.q, 1, i);
         VQ_GC_FENCE();
-        // Four chains per tile: a quarter of the length, half the rounding of a 64-term sum in order.
-        gc_f4 xc[2][4], oc[2][4];
+        // Eight sums of eight terms per tile, added pairwise: twelve roundings in a row, not 64. The first half's are added
+        // while the second half's products run.
+        gc_f4 xc[2][2][4], oc[2][2][4], xs[2][2], os[2][2];
+        auto part_sum = [&](int i) {
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) xc[t][e] = oc[t][e] = gc_f4{0.f, 0.f, 0.f, 0.f};
+            for (int t = 0; t < 2; ++t) {
+                const gc_f4 *const a = xc[i][t], *const b = oc[i][t];
+                xs[t][i] = (a[0] + a[1]) + (a[2] + a[3]);
+                os[t][i] = (b[0] + b[1]) + (b[2] + b[3]);
+            }
+        };
         gc_f4 kw[2], bs[2], kc[2], vv[2], tt[3], pp[2], qg;
         float gc;
-        // K S0 and Q S0: four chains of MFMAs (a dependent one waits 8-12 cycles past its 32), in four parts that also
+        // K S0 and Q S0: chains of MFMAs (a dependent one waits 8-12 cycles past its 32), in four parts that also
         // read what the second half of the chunk needs and start the next chunk's DMA.
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -355,17 +372,20 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
             for (int q = 0; q < 4; ++q) {
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
-                    xc[t][q] = gc_mfma(ka[t][i][q], st[i][q], xc[t][q]);
-                    oc[t][q] = gc_mfma(qa[t][i][q], st[i][q], oc[t][q]);
+                    const gc_f4 z = {0.f, 0.f, 0.f, 0.f};
+                    xc[i >> 1][t][q] = gc_mfma(ka[t][i][q], st[i][q], i & 1 ? xc[i >> 1][t][q] : z);
+                    oc[i >> 1][t][q] = gc_mfma(qa[t][i][q], st[i][q], i & 1 ? oc[i >> 1][t][q] : z);
                 }
             }
+            if (i == 2) part_sum(0);
             if (i < 3 && c + 1 < cb) issue(c + 1, i);
             VQ_GC_FENCE();
         }
+        part_sum(1);
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            x[t] = (xc[t][0] + xc[t][1]) + (xc[t][2] + xc[t][3]);
-            o[t] = (oc[t][0] + oc[t][1]) + (oc[t][2] + oc[t][3]);
+            x[t] = xs[t][0] + xs[t][1];
+            o[t] = os[t][0] + os[t][1];
         }
         ex[wv][0][lane] = x[0];
         ex[wv][1][lane] = x[1];
@@ -374,8 +394,6 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
         const int pw = wv ^ 2;
         gc_f4 xp[2] = {ex[pw][0][lane], ex[pw][1][lane]};
         const gc_f4 op = ex[pw][2][lane];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) st[i] *= gc;
         // R = b V - (b G) K S0, then d = T R
         gc_f4 r[2], d[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, d1 = d[0];
 #pragma unroll
@@ -390,16 +408,24 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
         }
         d[1] += d1;
         // S = G_C S + K^T (D(C - 1, .) d),  o = G (Q S0) + P d (the tile of P above the diagonal is zero)
-        gc_f4 y = ((kh == 0 ? o[0] : o[1]) + op) * qg;
+        // The sums over the chunk's tokens start from zero and meet the larger terms once, in one fma.
+        gc_f4 y = {0.f, 0.f, 0.f, 0.f}, up[4] = {y, y, y, y};
+        const gc_f4 qs0 = (kh == 0 ? o[0] : o[1]) + op;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             const gc_f4 kd = d[t] * kc[t];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) st[i] = gc_mfma(kt[t][q][i], kd[q], st[i]);
+                for (int i = 0; i < 4; ++i) up[i] = gc_mfma(kt[t][q][i], kd[q], up[i]);
                 y = gc_mfma(pp[t][q], d[t][q], y);
             }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            y[q] = fmaf(qs0[q], qg[q], y[q]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) st[i][q] = fmaf(st[i][q], gc, up[i][q]);
         }
 #undef VQ_GC_FENCE
         vq::wait_vm<0>();  // the next chunk's operands (not the stores that follow)
