@@ -125,7 +125,7 @@ def gated_delta_inputs(rng, n, kh, vh, kd, vd, slots):
                 state=(0.1 * rng.standard_normal((slots, vh, kd, vd))).astype(np.float32))
 
 
-def run_gated_delta(rt, inp, segs, shape, elem, order, write):
+def run_gated_delta(rt, inp, segs, shape, elem, order, write, eps=1e-6):
     kh, vh, kd, vd = shape
     n = inp["conv"].shape[0]
     for name in ("ssm_a", "dt"):
@@ -135,7 +135,7 @@ def run_gated_delta(rt, inp, segs, shape, elem, order, write):
     put(rt, "g.s", inp["state"], elem)
     put(rt, "g.o", np.zeros((n, vh, vd)))
     rt.set_segments(segs)
-    rt.gated_delta_seg("g.conv", "g.b", "g.a", "g.ssm_a", "g.dt", "g.s", "g.o", kh, vh, kd, vd, 1e-6, order, None, write)
+    rt.gated_delta_seg("g.conv", "g.b", "g.a", "g.ssm_a", "g.dt", "g.s", "g.o", kh, vh, kd, vd, eps, order, None, write)
     return get(rt, "g.o", (n, vh, vd)), get(rt, "g.s", inp["state"].shape)
 
 
@@ -205,6 +205,47 @@ def test_gated_delta_chunks_keep_causality(rt, oracle_mod, what):
     if what == "v":
         rest = np.arange(vd) != 3
         assert np.abs(out[:, 0, rest] - clean[:, 0, rest]).max() <= 2e-6 * np.abs(clean).max()
+
+
+@pytest.mark.parametrize("what", ["keys", "keys and queries", "keys, eps 0", "state", "values"])
+def test_gated_delta_chunks_fp32_range(rt, oracle_mod, what):
+    """Finite inputs whose norms, products with the state or sums leave the fp32 range behave as token by token: a key
+    whose squares overflow has weight zero, and a state or value at the edge of the range reaches no earlier token of its
+    chunk. Same finite elements as the per-token kernel's, those within 5e-6 of the column's largest: the state of that
+    kernel is rounded once per token, 80 halves of 2^-23."""
+    shape = kh, vh, kd, vd = 1, 2, 128, 64
+    rng = np.random.default_rng(6)
+    n, k0, eps = 80, kh * kd, 0.0 if what == "keys, eps 0" else 1e-6
+    rt.alloc("pt", 64)
+    rt.set_paging("pt", 64, 16, 1)
+    inp = gated_delta_inputs(rng, n, kh, vh, kd, vd, 1)
+    segs = [(0, 0, n, 0)]
+    if what.startswith("keys"):  # sum of squares 1e42, with eps 0 1e-34
+        inp["conv"][[20, 25], k0:k0 + kd] *= np.float32(1e20 if eps else 1e-18)
+        if what == "keys and queries":
+            inp["conv"][[20, 25], :kd] *= np.float32(1e20)
+    elif what == "state":  # S^T k overflows at token 20 in column 3 of head 0, and nowhere before
+        inp["ssm_a"][:], inp["b"][:] = -1e-6, -20.0
+        inp["state"][0, 0, 5, 3] = 2.5e38
+        inp["conv"][:, [5, k0 + 5]] = 0.01
+        inp["conv"][20, k0 + 5] = 4.0
+    else:  # d overflows at token 26 in column 3 of head 0
+        inp["b"][:] = 20.0
+        inp["conv"][26, k0:k0 + kd] = -inp["conv"][25, k0:k0 + kd]
+        inp["conv"][[25, 26], 2 * kh * kd + 3] = 3e38
+        inp["conv"][[25, 26], :kd] *= np.float32(0.01)  # (S^T q of the token before does not)
+    out, st = run_gated_delta(rt, inp, segs, shape, 4, 0, 1, eps)
+    rt.set_batch_invariant(True)
+    want, fin = run_gated_delta(rt, inp, segs, shape, 4, 0, 1, eps)
+    rt.set_batch_invariant(False)
+    assert np.isfinite(want[:20]).all() and np.isfinite(want[:, 1]).all()
+    for got, ref in ((out, want), (st[0], fin[0])):
+        ok = np.isfinite(ref)
+        assert np.array_equal(np.isfinite(got), ok)
+        diff, size = np.where(ok, np.abs(np.where(ok, got, 0) - np.where(ok, ref, 0)), 0), np.where(ok, np.abs(ref), 0)
+        if ref is want:
+            assert (diff[:20].max((0, 1)) <= 5e-6 * size[:20].max((0, 1))).all()  # before the large value
+        assert (diff.max((0, 1)) <= 5e-6 * size.max((0, 1))).all()
 
 
 # Key blocks of 32 in two parities, 16-row tiles, three or four heads of a kv head per workgroup.

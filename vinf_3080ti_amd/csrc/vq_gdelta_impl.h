@@ -30,8 +30,10 @@
 // element is free as long as A and B agree, so step q of a 16-deep block takes k = 4 lk + q: an accumulator tile is then
 // a B operand as it stands, and an A operand is one float4 of a row.
 //
-// Inputs that are not finite (or whose norms or decays are not) would meet zeros of T and P in these products and reach
-// tokens before their own; the prep kernel flags such chunks and the walk takes them token by token.
+// A value that is not finite, given or arising on the way, would meet zeros of T and P in these products and reach tokens
+// before its own. Chunks that could hold one are taken token by token: the prep kernel flags those whose inputs or norms
+// lie past kGcHuge or whose scales past kGcScale, the walk those whose (b G) K S0 does. Below these bounds T's entries
+// stay near one (decays of at most one) and no product or sum of a chunk leaves the fp32 range.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stddef.h>
@@ -48,6 +50,8 @@ constexpr int kGcC = 32, kGcKd = 128, kGcMaxVd = 128, kGcCols = 32;
 constexpr int kGcMinRows = 24;
 constexpr int kGcRound = 16;  // chunks per segment and launch pair at one segment (bounds the workspace)
 static_assert(kGcRound <= 64, "one lane per chunk reads the non-finite flags");
+
+constexpr float kGcHuge = 1e30f, kGcScale = 1e15f;
 
 typedef float gc_f4 __attribute__((ext_vector_type(4)));
 
@@ -89,7 +93,7 @@ __global__ __launch_bounds__(256) void gd_prep_kernel(GcArgs A, SegTable T) {
     const size_t row0 = static_cast<size_t>(s.row0) + t0;
     float *const ws = A.ws + ((static_cast<size_t>(blockIdx.z) * A.cr + blockIdx.y) * vh + h) * GcSlot::floats;
 
-    // 1. The chunk's q, k rows (zeros past the segment); v only to see that it is finite.
+    // 1. The chunk's q, k rows (zeros past the segment); v only to see that it is in range.
     if (tid == 0) s_bad = 0;
     bool bad = false;
 #pragma unroll
@@ -103,7 +107,7 @@ __global__ __launch_bounds__(256) void gd_prep_kernel(GcArgs A, SegTable T) {
             if (e < vd) v = gc_ld(src + static_cast<size_t>(2) * A.key_heads * kGcKd + static_cast<size_t>(h) * vd + e);
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) bad |= gc_bad(q[j]) || gc_bad(k[j]) || gc_bad(v[j]);
+        for (int j = 0; j < 4; ++j) bad |= !(fabsf(v[j]) < kGcHuge);
         *reinterpret_cast<gc_f4 *>(&sQ[r][e]) = q;
         *reinterpret_cast<gc_f4 *>(&sK[r][e]) = k;
     }
@@ -128,7 +132,8 @@ __global__ __launch_bounds__(256) void gd_prep_kernel(GcArgs A, SegTable T) {
             const float qs = in ? rkd / sqrtf(qq + A.eps) : 0.0f, ks = in ? 1.0f / sqrtf(kk + A.eps) : 0.0f;
             const float g = in ? expf(sa * (xa > 20.0f ? xa : log1pf(expf(xa)))) : 1.0f;
             const float b = in ? sigmoid_ieee(xb) : 0.0f;
-            bad |= gc_bad(qs) || gc_bad(ks) || gc_bad(g) || gc_bad(b);
+            // The sums themselves: one that overflowed leaves a finite scale (zero).
+            bad |= !(qq < kGcHuge) || !(kk < kGcHuge) || !(qs < kGcScale) || !(ks < kGcScale) || gc_bad(g) || gc_bad(b);
             sQs[t] = qs, sKs[t] = ks, sG[t] = g, sB[t] = b;
         }
     }
@@ -242,6 +247,7 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
     __shared__ __align__(1024) Buf buf[2];
     __shared__ __align__(16) gc_f4 ex[4][3][64];  // [wave][tile][lane]
     __shared__ float red[2][4][3][16];            // token-by-token chunks: [wave][sum][column]
+    __shared__ __align__(16) int huge[4];         // [wave]: its part of the present chunk's (b G) K S0 is out of range
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lk = lane >> 4;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), n = wv & 1, kh = wv >> 1;
     const int vh = A.value_heads, vd = A.vd, tiles = vd / kGcCols;
@@ -308,7 +314,8 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
     float *const orow = out + (static_cast<size_t>(s.row0) * vh + h) * vd + col;
     const size_t ostep = static_cast<size_t>(vh) * vd;
 
-    // One chunk from its operands (landed; all waves past the barrier that says so).
+    // One chunk from its operands (landed; all waves past the barrier that says so). False (for all waves alike), with
+    // the state as it was, when (b G) K S0 is out of range.
     auto chunk = [&](int c) {
         const Buf &f = buf[c & 1];
         auto a_row = [&](const float *m, int t, int i) {  // A operand: rows 16 t + lr, columns 64 kh + 16 i + 4 lk ..
@@ -390,7 +397,18 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
         ex[wv][0][lane] = x[0];
         ex[wv][1][lane] = x[1];
         ex[wv][2][lane] = kh == 0 ? o[1] : o[0];  // the partner's output rows
+        float mag = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) mag = fmaf(fabsf(kw[t][q]), fabsf(x[t][q]), mag);
+        const int far = __any(!(mag < kGcHuge));
+        if (lane == 0) huge[wv] = far;
         __syncthreads();
+        if (__builtin_amdgcn_readfirstlane(huge[0] | huge[1] | huge[2] | huge[3])) {
+            vq::wait_vm<0>();
+            return false;
+        }
         const int pw = wv ^ 2;
         gc_f4 xp[2] = {ex[pw][0][lane], ex[pw][1][lane]};
         const gc_f4 op = ex[pw][2][lane];
@@ -434,8 +452,9 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
             const int t = c * kGcC + 16 * kh + 4 * lk + q;
             if (t < s.rows) orow[t * ostep] = y[q];
         }
+        return true;
     };
-    // One chunk token by token (an input is not finite): the rule as the per-token kernel computes it.
+    // One chunk token by token (a value is out of range): the rule as the per-token kernel computes it.
     auto serial = [&](int c) {
         const float rkd = 1.0f / sqrtf(static_cast<float>(kGcKd));
         // Column sums over all rows: the lane groups, then the two waves of the column tile.
@@ -492,12 +511,15 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
     vq::wait_vm<0>();
     for (int c = ca; c < cb; ++c) {
         __syncthreads();  // chunk c landed for every wave; every wave is done with chunk c - 1's buffer
+        bool done = false;
         if ((bad >> (c - ca) & 1) == 0) {
-            chunk(c);
+            done = chunk(c);
         } else {
 #pragma unroll
             for (int part = 0; part < 3; ++part)
                 if (c + 1 < cb) issue(c + 1, part);
+        }
+        if (!done) {
             serial(c);
             vq::wait_vm<0>();
         }
