@@ -207,6 +207,24 @@ def test_gated_delta_chunks_keep_causality(rt, oracle_mod, what):
         assert np.abs(out[:, 0, rest] - clean[:, 0, rest]).max() <= 2e-6 * np.abs(clean).max()
 
 
+@pytest.mark.parametrize("g", [1.1, 1.3])
+def test_gated_delta_chunks_decay_above_one(rt, oracle_mod, g):
+    """Equal keys, each token replacing what the one before wrote: token by token nothing grows, while the products of a
+    chunk's decays reach 1.3^32 = 4400. Bound as above, 2e-6 of the largest value."""
+    shape = kh, vh, kd, vd = 1, 2, 128, 64
+    rng = np.random.default_rng(8)
+    rt.alloc("pt", 64)
+    rt.set_paging("pt", 64, 16, 1)
+    inp = gated_delta_inputs(rng, 64, kh, vh, kd, vd, 1)
+    inp["conv"][:, :2 * kh * kd] = np.tile(rng.standard_normal(kd), 2)
+    inp["a"][:], inp["dt"][:], inp["b"][:], inp["state"][:] = 0.0, 0.0, 6.0, 0.0
+    inp["ssm_a"][:] = np.log(g) / np.log(2.0)
+    segs = [(0, 0, 64, 0)]
+    expect, _ = gated_delta_rows(oracle_mod, inp, segs, inp["state"], kh, vh, kd, vd, 0)
+    out, _ = run_gated_delta(rt, inp, segs, shape, 4, 0, 1)
+    assert np.abs(out - expect).max() <= 2e-6 * np.abs(expect).max()
+
+
 @pytest.mark.parametrize("what", ["keys", "keys and queries", "keys, eps 0", "state", "values"])
 def test_gated_delta_chunks_fp32_range(rt, oracle_mod, what):
     """Finite inputs whose norms, products with the state or sums leave the fp32 range behave as token by token: a key
