@@ -2,37 +2,40 @@
 //
 // The rule per token t (k, q normalised, g the decay, b = beta):
 //   S <- g_t S;  d_t = b_t (v_t - S^T k_t);  S <- S + k_t d_t^T;  o_t = S^T q_t.
-// Over a chunk that starts from state S0, with D(t, i) = g_{i+1} ... g_t (running products, so that a pair's decay
-// carries only its own roundings) and G_t = D(t, -1):
+// Over a chunk that starts from state S0, with D(t, i) = g_{i+1} ... g_t (running products) and G_t = D(t, -1):
 //   d_t = b_t (v_t - G_t S0^T k_t) - sum_{i<t} L(t, i) d_i,   L(t, i) = b_t D(t, i) (k_i . k_t)
 //   o_t = G_t S0^T q_t + sum_{i<=t} P(t, i) d_i,              P(t, i) = D(t, i) (k_i . q_t)
 //   S_C = G_C S0 + sum_i D(C - 1, i) k_i d_i^T
 // so with T = (I + L)^-1 everything that meets the state is a matrix product:
-//   d = T (b V - (b G) K S0),   o = G (Q S0) + P d,   S_C = G_C S0 + (D(C - 1, .) K)^T d.
-// All of it in fp32 (v_mfma_f32_16x16x4_f32, fp32 operands and sums), with care for the roundings in a row: long sums in
-// eight chains, the sums over a chunk's tokens from zero, decays, pair factors and the diagonal blocks of T in fp64 and
-// rounded once. Against float64 at 512 tokens rel-L2 1.4-1.5e-7 (outputs) and 1.5-1.7e-7 (state) over three inputs; the
-// per-token kernel 1.4e-7 and 1.4-1.7e-7. In four chains, with fp32 decays, it was 1.65e-7 (and 54.5 us for the walk).
+//   d = T b (V - G K S0),   o = G (Q S0) + P d,   S_C = G_C S0 + (D(C - 1, .) K)^T d.
+// The 1 / |k| of the last two's k and the b go into T, so that the walk's products are of the rows as given.
+// What meets the state is fp32 (v_mfma_f32_16x16x4_f32, fp32 operands and sums), with care for the roundings in a row: long
+// sums in eight chains, the sums over a chunk's tokens from zero. What does not (the pairs' products, decays and factors,
+// T) is fp64 on v_mfma_f64_16x16x4_f64 and rounded once into an operand. Rel-L2 error against float64 as a multiple of the
+// per-token kernel's, 24 to 512 tokens, independent keys: outputs 0.83-0.90 (1.1-1.6e-7), state 0.8-1.13 (1.0-2.2e-7); with
+// the pairs' products in fp32 the outputs stood at 0.9-1.12, and at 1.3-1.4 (now 1.0-1.1) for keys that share a
+// direction. Equal keys, beta near one: 1.3-1.6; there each update of the per-token rule corrects the one before it.
 //
 // Two launches. gd_prep_kernel, one workgroup per (chunk, value head), all chunks at once: T and P into the workspace in
-// MFMA operand order, and the tokens' scales. gd_chunk_kernel, one workgroup per (value head, 32 state columns), walks
+// MFMA operand order, and the tokens' scales. It leaves V alone (the walk reads and checks it), which pays for the fp64
+// products: 15.9 us, as with fp32 ones. gd_chunk_kernel, one workgroup per (value head, 32 state columns), walks
 // the chunks with its part of the state in accumulators, the chunk's K, Q, V rows and T, P reaching LDS by DMA a chunk
-// ahead: 116-120 MFMAs per wave and two barriers per 32 tokens, instead of 32 serial tokens of two barriers each. What bounds
-// it: the serial chunk walk's MFMA issue (33 cycles each, 1.9 us of a chunk's 3.7, on 192 of 256 CUs). Operands prepared in full
-// (W = T diag(b G) K, scaled Q and K in operand order, read straight into registers) moved 55 KB per chunk and
+// ahead: 116 MFMAs per wave and two barriers per 32 tokens, instead of 32 serial tokens of two barriers each. What bounds
+// it: the serial chunk walk's MFMA issue (33 cycles each, 1.6 us of a chunk's 3.7, on 192 of 256 CUs). Operands prepared
+// in full (W = T diag(b G) K, scaled Q and K in operand order, read straight into registers) moved 55 KB per chunk and
 // workgroup through L2 twice and took 28 + 56 us. Measured at 16 key and 48 value heads, kd = vd = 128, 512 tokens:
-// 15.4 + 59.6 us against 358 us token by token. Before the eight chains, of a chunk's 6800 cycles the K S0 and Q S0
-// products took 3500 (their
-// 64 MFMAs 2100; the rest are the copies and LDS reads of the one wave per SIMD), T R 690, the state update 1720; eight
-// waves of 32 rows measured 62 us (more operand reads and a four-way exchange), one copy per four MFMAs 57 us.
+// 15.9 + 60.3 us against 358 us token by token. With four chains (54.5 us), of a chunk's 6800 cycles the K S0 and Q S0
+// products took 3500 (their 64 MFMAs 2100; the rest are the copies and LDS reads of the one wave per SIMD), T R 690, the
+// state update 1720; eight waves of 32 rows measured 62 us (more operand reads and a four-way exchange), one copy per four
+// MFMAs 57 us.
 //
 // MFMA layouts used below (lane = 16 lk + lr): C/D element q is row 4 lk + q, column lr; the k index of an operand
 // element is free as long as A and B agree, so step q of a 16-deep block takes k = 4 lk + q: an accumulator tile is then
 // a B operand as it stands, and an A operand is one float4 of a row.
 //
 // A value that is not finite, given or arising on the way, would meet zeros of T and P in these products and reach tokens
-// before its own. Chunks that could hold one are taken token by token: the prep kernel flags those whose inputs or norms
-// lie past kGcHuge or whose scales past kGcScale, the walk those whose (b G) K S0 does. Below these bounds no product or
+// before its own. Chunks that could hold one are taken token by token: the prep kernel flags those whose sums
+// of squares lie past kGcHuge or whose scales past kGcScale, the walk those whose V or G K S0 does. Below these bounds no product or
 // sum of a chunk leaves the fp32 range. So are chunks whose decays above one multiply to kGcGrow or more: the entries of T
 // reach that product (one otherwise), and with it the rounding of d. Equal keys, beta 0.9975, against float64: decays of
 // 1.1 1.3e-6 (token by token 1.2e-7), of 1.3 1.4e-4.
@@ -53,14 +56,15 @@ constexpr int kGcMinRows = 24;
 constexpr int kGcRound = 16;  // chunks per segment and launch pair at one segment (bounds the workspace)
 static_assert(kGcRound <= 64, "one lane per chunk reads the non-finite flags");
 
-constexpr float kGcHuge = 1e30f, kGcScale = 1e15f, kGcGrow = 1.0625f;
+constexpr float kGcHuge = 1e30f, kGcScale = 1e6f, kGcGrow = 1.0625f;
 
 typedef float gc_f4 __attribute__((ext_vector_type(4)));
+typedef double gc_d4 __attribute__((ext_vector_type(4)));
 
 // Workspace of one (chunk, value head), in floats: T and P as A operands [t tile 2][i tile 2][lane][4], then the tokens'
-// scales (32 each: b G / |k|, b, D(C - 1, .) / |k|, G / (|q| sqrt(kd))), G_C and the non-finite flag.
+// scales (32 each: G / |k|, D(C - 1, .), G / (|q| sqrt(kd))), G_C and the flag of a chunk to take token by token.
 struct GcSlot {
-    static constexpr int T = 0, P = 1024, SC = 2048, KW = 0, B = 32, KC = 64, QG = 96, GC = 128, BAD = 129;
+    static constexpr int T = 0, P = 1024, SC = 2048, KG = 0, DC = 32, QG = 64, GC = 96, BAD = 97;
     static constexpr size_t floats = 2304;
 };
 
@@ -75,13 +79,19 @@ struct GcArgs {
 
 __device__ __forceinline__ bool gc_bad(float v) { return (__float_as_uint(v) & 0x7F800000u) == 0x7F800000u; }
 __device__ __forceinline__ gc_f4 gc_mfma(float a, float b, gc_f4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ gc_d4 gc_mfma64(double a, double b, gc_d4 c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ gc_f4 gc_ld(const float *p) { return *reinterpret_cast<const gc_f4 *>(p); }
 
 __global__ __launch_bounds__(256) void gd_prep_kernel(GcArgs A, SegTable T) {
     constexpr int RS = kGcKd + 4;  // LDS row pitch (floats)
-    __shared__ __align__(16) float sK[kGcC][RS], sQ[kGcC][RS];
-    __shared__ __align__(16) float sL[kGcC][36], sT[kGcC][36];
-    __shared__ double sD[kGcC][33], sGt[kGcC];
+    // K and Q until their products are made, then L and T in their place.
+    __shared__ __align__(16) float sKQ[2][kGcC][RS];
+    static_assert(2 * kGcC * 34 * sizeof(double) <= sizeof(sKQ));
+    auto &sK = sKQ[0], &sQ = sKQ[1];
+    double(&sL)[kGcC][34] = reinterpret_cast<double(&)[kGcC][34]>(sKQ[0]);
+    double(&sT)[kGcC][34] = *(&sL + 1);
+    __shared__ double sD[kGcC][kGcC + 1];  // [t][i + 1]: D(t, i); [t][0]: G_t
+    __shared__ double sH[3][4][64];  // the second halves of the three tiles of P^T
     __shared__ float sB[kGcC], sG[kGcC], sQs[kGcC], sKs[kGcC];
     __shared__ int s_bad;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, lr = lane & 15, lk = lane >> 4;
@@ -95,21 +105,18 @@ __global__ __launch_bounds__(256) void gd_prep_kernel(GcArgs A, SegTable T) {
     const size_t row0 = static_cast<size_t>(s.row0) + t0;
     float *const ws = A.ws + ((static_cast<size_t>(blockIdx.z) * A.cr + blockIdx.y) * vh + h) * GcSlot::floats;
 
-    // 1. The chunk's q, k rows (zeros past the segment); v only to see that it is in range.
+    // 1. The chunk's q, k rows (zeros past the segment).
     if (tid == 0) s_bad = 0;
     bool bad = false;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int r = (tid >> 5) + 8 * i, e = 4 * (tid & 31);
-        gc_f4 q = {0.f, 0.f, 0.f, 0.f}, k = q, v = q;
+        gc_f4 q = {0.f, 0.f, 0.f, 0.f}, k = q;
         if (r < nt) {
             const float *src = A.conv + (row0 + r) * cdim;
             q = gc_ld(src + static_cast<size_t>(kh) * kGcKd + e);
             k = gc_ld(src + static_cast<size_t>(A.key_heads + kh) * kGcKd + e);
-            if (e < vd) v = gc_ld(src + static_cast<size_t>(2) * A.key_heads * kGcKd + static_cast<size_t>(h) * vd + e);
         }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) bad |= !(fabsf(v[j]) < kGcHuge);
         *reinterpret_cast<gc_f4 *>(&sQ[r][e]) = q;
         *reinterpret_cast<gc_f4 *>(&sK[r][e]) = k;
     }
@@ -141,71 +148,78 @@ __global__ __launch_bounds__(256) void gd_prep_kernel(GcArgs A, SegTable T) {
     }
     if (bad) s_bad = 1;
     __syncthreads();
-    // 3. Decays of the pairs: lane i of wave 0 walks D(t, i) down its column; lane 32 the decay since the chunk's start.
-    // The other waves meanwhile start on their products. The running products and the pairs' factors are fp64, rounded
-    // once where they become operands.
-    if (tid < kGcC) {
-        double d = 1.0;
-#pragma unroll
-        for (int t = 0; t < kGcC; ++t) {
-            d = t <= tid ? 1.0 : d * sG[t];
-            sD[t][tid] = t < tid ? 0.0 : d;
-        }
-    } else if (tid == kGcC) {
-        double d = 1.0;
-        float grow = 1.0f;
-#pragma unroll
-        for (int t = 0; t < kGcC; ++t) {
-            d *= sG[t];
-            grow *= fmaxf(sG[t], 1.0f);
-            sGt[t] = d;
-        }
-        // Decays above one: T's entries grow with their products while the d_t that the sums leave stay as they were.
-        if (!(grow < kGcGrow)) s_bad = 1;
-    }
+    // 3. Wave 1, which has no tile below, walks the decays of the pairs down their columns: lane 0 those since the chunk's
+    // start (G_t), lane i + 1 the D(t, i). The running products and the pairs' factors are fp64, rounded once where they
+    // become operands.
     // 4. Wave (jt, ji): the 16 x 16 tiles L (rows t, columns i) and P^T (rows i, columns t); nothing above the diagonal.
+    // D element q of the fp64 MFMA: row 4 q + lk, column lr.
     const int jt = wv >> 1, ji = wv & 1;
-    gc_f4 kk = {0.f, 0.f, 0.f, 0.f}, kq = kk, kc8[8], qc8[8];
-    if (ji <= jt) {  // eight chains each
+    gc_d4 kk = {0.0, 0.0, 0.0, 0.0}, kq = kk;
+    if (wv == 1) {
+        if (lane <= kGcC) {
+            double d = 1.0;
+            float grow = 1.0f;
 #pragma unroll
-        for (int q = 0; q < 8; ++q) kc8[q] = qc8[q] = kk;
+            for (int t = 0; t < kGcC; ++t) {
+                d = t < lane ? 1.0 : d * sG[t];
+                sD[t][lane] = t + 1 < lane ? 0.0 : d;
+                grow *= fmaxf(sG[t], 1.0f);
+            }
+            // Decays above one: T's entries grow with their products while the d_t that the sums leave stay as they were.
+            if (!(grow < kGcGrow)) s_bad = 1;
+        }
+        gc_d4 h[3] = {kk, kk, kk};
+#pragma unroll
+        for (int cc = kGcKd / 32; cc < kGcKd / 16; ++cc) {
+            const gc_f4 k0 = gc_ld(&sK[lr][16 * cc + 4 * lk]), k1 = gc_ld(&sK[16 + lr][16 * cc + 4 * lk]),
+                        q0 = gc_ld(&sQ[lr][16 * cc + 4 * lk]), q1 = gc_ld(&sQ[16 + lr][16 * cc + 4 * lk]);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                h[0] = gc_mfma64(k0[q], q0[q], h[0]);
+                h[1] = gc_mfma64(k0[q], q1[q], h[1]);
+                h[2] = gc_mfma64(k1[q], q1[q], h[2]);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 3; ++t)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) sH[t][q][lane] = h[t][q];
+    } else {
 #pragma unroll
         for (int cc = 0; cc < kGcKd / 16; ++cc) {
             const gc_f4 kt = gc_ld(&sK[16 * jt + lr][16 * cc + 4 * lk]), ki = gc_ld(&sK[16 * ji + lr][16 * cc + 4 * lk]),
                         qt = gc_ld(&sQ[16 * jt + lr][16 * cc + 4 * lk]);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const int e = 4 * (cc & 1) + q;
-                kc8[e] = gc_mfma(kt[q], ki[q], kc8[e]);
-                qc8[e] = gc_mfma(ki[q], qt[q], qc8[e]);
+                kk = gc_mfma64(kt[q], ki[q], kk);
+                if (cc < kGcKd / 32) kq = gc_mfma64(ki[q], qt[q], kq);
             }
         }
-        kk = ((kc8[0] + kc8[1]) + (kc8[2] + kc8[3])) + ((kc8[4] + kc8[5]) + (kc8[6] + kc8[7]));
-        kq = ((qc8[0] + qc8[1]) + (qc8[2] + qc8[3])) + ((qc8[4] + qc8[5]) + (qc8[6] + qc8[7]));
     }
     __syncthreads();
-    gc_f4 p;
+    if (wv != 1) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) kq[q] += sH[jt + ji][q][lane];
+    }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        const int t = 16 * jt + 4 * lk + q, i = 16 * ji + lr;
-        const double ks = sKs[t], qs = sQs[16 * jt + lr];
-        sL[t][i] = i < t ? static_cast<float>(sB[t] * sD[t][i] * (ks * sKs[i]) * kk[q]) : 0.0f;
-        const int pt = 16 * jt + lr, pi = 16 * ji + 4 * lk + q;
-        p[q] = pi <= pt ? static_cast<float>(sD[pt][pi] * (qs * sKs[pi]) * kq[q]) : 0.0f;
+        const int e = 4 * q + lk, t = 16 * jt + e, i = 16 * ji + lr;
+        const double ks = sKs[t];
+        sL[t][i] = i < t ? sB[t] * sD[t][i + 1] * (ks * sKs[i]) * kk[q] : 0.0;
+        const int pt = 16 * jt + lr, pi = 16 * ji + e;
+        ws[GcSlot::P + ((jt * 2 + ji) * 64 + 16 * q + lr) * 4 + lk] =
+            pi <= pt ? static_cast<float>(sD[pt][pi + 1] * sQs[pt] * kq[q]) : 0.0f;
     }
-    *reinterpret_cast<gc_f4 *>(ws + GcSlot::P + ((jt * 2 + ji) * 64 + lane) * 4) = p;
     if (tid < kGcC) {
         float *const sc = ws + GcSlot::SC;
-        const double ks = sKs[tid];
-        const float gc = static_cast<float>(sGt[kGcC - 1]);
-        sc[GcSlot::KW + tid] = static_cast<float>(sB[tid] * sGt[tid] * ks);
-        sc[GcSlot::B + tid] = sB[tid];
-        sc[GcSlot::KC + tid] = static_cast<float>(sD[kGcC - 1][tid] * ks);
-        sc[GcSlot::QG + tid] = static_cast<float>(sGt[tid] * sQs[tid]);
+        const float gc = static_cast<float>(sD[kGcC - 1][0]);
+        sc[GcSlot::KG + tid] = static_cast<float>(sD[tid][0] * sKs[tid]);
+        sc[GcSlot::DC + tid] = static_cast<float>(sD[kGcC - 1][tid + 1]);
+        sc[GcSlot::QG + tid] = static_cast<float>(sD[tid][0] * sQs[tid]);
         if (tid == 0) sc[GcSlot::GC] = gc, sc[GcSlot::BAD] = s_bad || gc_bad(gc) ? 1.0f : 0.0f;
     }
     __syncthreads();
-    // 5. T = (I + L)^-1: the two diagonal blocks by forward substitution (lane = column), then T21 = -T22 (L21 T11).
+    // 5. (I + L)^-1: the two diagonal blocks by forward substitution (lane = column), then T21 = -T22 (L21 T11).
     if (wv < 2 && lane < 16) {
         const int o = 16 * wv;
         double x[16];
@@ -213,26 +227,32 @@ __global__ __launch_bounds__(256) void gd_prep_kernel(GcArgs A, SegTable T) {
         for (int t = 0; t < 16; ++t) {
             double v = t == lane ? 1.0 : 0.0;
 #pragma unroll
-            for (int i = 0; i < t; ++i) v = fma(-static_cast<double>(sL[o + t][o + i]), x[i], v);
+            for (int i = 0; i < t; ++i) v = fma(-sL[o + t][o + i], x[i], v);
             x[t] = v;
-            sT[o + t][o + lane] = static_cast<float>(v);
+            sT[o + t][o + lane] = v;
         }
     }
     __syncthreads();
     if (wv == 0) {
-        gc_f4 m = {0.f, 0.f, 0.f, 0.f}, x = m;
-        const gc_f4 l = gc_ld(&sL[16 + lr][4 * lk]), t22 = gc_ld(&sT[16 + lr][16 + 4 * lk]);
+        gc_d4 m = {0.0, 0.0, 0.0, 0.0}, x = m;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) m = gc_mfma(l[q], sT[4 * lk + q][lr], m);
+        for (int q = 0; q < 4; ++q) m = gc_mfma64(sL[16 + lr][4 * q + lk], sT[4 * q + lk][lr], m);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) x = gc_mfma(t22[q], m[q], x);
+        for (int q = 0; q < 4; ++q) x = gc_mfma64(sT[16 + lr][16 + 4 * q + lk], m[q], x);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) sT[16 + 4 * lk + q][lr] = -x[q];
+        for (int q = 0; q < 4; ++q) sT[16 + 4 * q + lk][lr] = -x[q];
     }
     __syncthreads();
-    if (ji <= jt)
-        *reinterpret_cast<gc_f4 *>(ws + GcSlot::T + ((jt * 2 + ji) * 64 + lane) * 4) =
-            gc_ld(&sT[16 * jt + lr][16 * ji + 4 * lk]);
+    if (ji <= jt) {
+        const int t = 16 * jt + lr;
+        gc_f4 v;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int i = 16 * ji + 4 * lk + q;
+            v[q] = static_cast<float>(sKs[t] * sT[t][i] * sB[i]);
+        }
+        *reinterpret_cast<gc_f4 *>(ws + GcSlot::T + ((jt * 2 + ji) * 64 + lane) * 4) = v;
+    }
 }
 
 // The chunk walk. Wave w of a workgroup: column tile n = w & 1 (16 of the 32 columns), state rows 64 kh .. +64 with
@@ -250,7 +270,7 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
     __shared__ __align__(1024) Buf buf[2];
     __shared__ __align__(16) gc_f4 ex[4][3][64];  // [wave][tile][lane]
     __shared__ float red[2][4][3][16];            // token-by-token chunks: [wave][sum][column]
-    __shared__ __align__(16) int huge[4];         // [wave]: its part of the present chunk's (b G) K S0 is out of range
+    __shared__ __align__(16) int huge[4];         // [wave]: its part of the present chunk's V and G K S0 is out of range
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lk = lane >> 4;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), n = wv & 1, kh = wv >> 1;
     const int vh = A.value_heads, vd = A.vd, tiles = vd / kGcCols;
@@ -318,7 +338,7 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
     const size_t ostep = static_cast<size_t>(vh) * vd;
 
     // One chunk from its operands (landed; all waves past the barrier that says so). False (for all waves alike), with
-    // the state as it was, when (b G) K S0 is out of range.
+    // the state as it was, when V or G K S0 is out of range.
     auto chunk = [&](int c) {
         const Buf &f = buf[c & 1];
         auto a_row = [&](const float *m, int t, int i) {  // A operand: rows 16 t + lr, columns 64 kh + 16 i + 4 lk ..
@@ -353,7 +373,7 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
                 os[t][i] = (b[0] + b[1]) + (b[2] + b[3]);
             }
         };
-        gc_f4 kw[2], bs[2], kc[2], vv[2], tt[3], pp[2], qg;
+        gc_f4 kg[2], dc[2], vv[2], tt[3], pp[2], qg;
         float gc;
         // K S0 and Q S0: chains of MFMAs (a dependent one waits 8-12 cycles past its 32), in four parts that also
         // read what the second half of the chunk needs and start the next chunk's DMA.
@@ -363,9 +383,8 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
                 read_kt(i);
             } else {
                 const int t = i - 2;
-                kw[t] = gc_ld(f.sc + GcSlot::KW + 16 * t + 4 * lk);
-                bs[t] = gc_ld(f.sc + GcSlot::B + 16 * t + 4 * lk);
-                kc[t] = gc_ld(f.sc + GcSlot::KC + 16 * t + 4 * lk);
+                kg[t] = gc_ld(f.sc + GcSlot::KG + 16 * t + 4 * lk);
+                dc[t] = gc_ld(f.sc + GcSlot::DC + 16 * t + 4 * lk);
                 pp[t] = gc_ld(f.p + 4 * ((2 * kh + t) * 64 + lane));
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
@@ -400,27 +419,26 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
         ex[wv][0][lane] = x[0];
         ex[wv][1][lane] = x[1];
         ex[wv][2][lane] = kh == 0 ? o[1] : o[0];  // the partner's output rows
-        float mag = 0.0f;
+        gc_f4 mag;
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) mag = fmaf(fabsf(kw[t][q]), fabsf(x[t][q]), mag);
-        const int far = __any(!(mag < kGcHuge));
+        for (int q = 0; q < 4; ++q)
+            mag[q] = fmaf(fabsf(kg[0][q]), fabsf(x[0][q]), fmaf(fabsf(kg[1][q]), fabsf(x[1][q]), fabsf(vv[0][q]) + fabsf(vv[1][q])));
+        const int far = __any(!((mag[0] + mag[1]) + (mag[2] + mag[3]) < kGcHuge));
         if (lane == 0) huge[wv] = far;
         __syncthreads();
-        if (__builtin_amdgcn_readfirstlane(huge[0] | huge[1] | huge[2] | huge[3])) {
+        const int pw = wv ^ 2;
+        const gc_f4 xp[2] = {ex[pw][0][lane], ex[pw][1][lane]}, op = ex[pw][2][lane];
+        const int4 any = *reinterpret_cast<const int4 *>(huge);
+        if (__builtin_amdgcn_readfirstlane(any.x | any.y | any.z | any.w)) {
             vq::wait_vm<0>();
             return false;
         }
-        const int pw = wv ^ 2;
-        gc_f4 xp[2] = {ex[pw][0][lane], ex[pw][1][lane]};
-        const gc_f4 op = ex[pw][2][lane];
-        // R = b V - (b G) K S0, then d = T R
+        // R = V - G K S0, then d / |k| = T R
         gc_f4 r[2], d[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, d1 = d[0];
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) r[t][q] = fmaf(-kw[t][q], x[t][q] + xp[t][q], bs[t][q] * vv[t][q]);
+            for (int q = 0; q < 4; ++q) r[t][q] = fmaf(-kg[t][q], x[t][q] + xp[t][q], vv[t][q]);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             d[0] = gc_mfma(tt[0][q], r[0][q], d[0]);
@@ -434,7 +452,7 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
         const gc_f4 qs0 = (kh == 0 ? o[0] : o[1]) + op;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            const gc_f4 kd = d[t] * kc[t];
+            const gc_f4 kd = d[t] * dc[t];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
 #pragma unroll
