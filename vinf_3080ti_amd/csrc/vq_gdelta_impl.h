@@ -24,7 +24,7 @@
 // it: the serial chunk walk's MFMA issue (33 cycles each, 1.6 us of a chunk's 3.7, on 192 of 256 CUs). Operands prepared
 // in full (W = T diag(b G) K, scaled Q and K in operand order, read straight into registers) moved 55 KB per chunk and
 // workgroup through L2 twice and took 28 + 56 us. Measured at 16 key and 48 value heads, kd = vd = 128, 512 tokens:
-// 15.9 + 60.3 us against 358 us token by token. With four chains (54.5 us), of a chunk's 6800 cycles the K S0 and Q S0
+// 15.9 + 59.5 us against 358 us token by token. With four chains (54.5 us), of a chunk's 6800 cycles the K S0 and Q S0
 // products took 3500 (their 64 MFMAs 2100; the rest are the copies and LDS reads of the one wave per SIMD), T R 690, the
 // state update 1720; eight waves of 32 rows measured 62 us (more operand reads and a four-way exchange), one copy per four
 // MFMAs 57 us.
@@ -34,9 +34,9 @@
 // a B operand as it stands, and an A operand is one float4 of a row.
 //
 // A value that is not finite, given or arising on the way, would meet zeros of T and P in these products and reach tokens
-// before its own. Chunks that could hold one are taken token by token: the prep kernel flags those whose sums
-// of squares lie past kGcHuge or whose scales past kGcScale, the walk those whose V or G K S0 does. Below these bounds no product or
-// sum of a chunk leaves the fp32 range. So are chunks whose decays above one multiply to kGcGrow or more: the entries of T
+// before its own. Chunks that could hold one are taken token by token: the prep kernel flags those
+// whose sums of squares lie past kGcSquare or whose scales past kGcScale, the walk those whose V or S0 lies past kGcHuge.
+// Below these bounds no product or sum of a chunk leaves the fp32 range. So are chunks whose decays above one multiply to kGcGrow or more: the entries of T
 // reach that product (one otherwise), and with it the rounding of d. Equal keys, beta 0.9975, against float64: decays of
 // 1.1 1.3e-6 (token by token 1.2e-7), of 1.3 1.4e-4.
 #pragma once
@@ -56,7 +56,7 @@ constexpr int kGcMinRows = 24;
 constexpr int kGcRound = 16;  // chunks per segment and launch pair at one segment (bounds the workspace)
 static_assert(kGcRound <= 64, "one lane per chunk reads the non-finite flags");
 
-constexpr float kGcHuge = 1e30f, kGcScale = 1e6f, kGcGrow = 1.0625f;
+constexpr float kGcHuge = 1e28f, kGcSquare = 1e18f, kGcScale = 1e6f, kGcGrow = 1.0625f;
 
 typedef float gc_f4 __attribute__((ext_vector_type(4)));
 typedef double gc_d4 __attribute__((ext_vector_type(4)));
@@ -142,7 +142,7 @@ __global__ __launch_bounds__(256) void gd_prep_kernel(GcArgs A, SegTable T) {
             const float g = in ? expf(sa * (xa > 20.0f ? xa : log1pf(expf(xa)))) : 1.0f;
             const float b = in ? sigmoid_ieee(xb) : 0.0f;
             // The sums themselves: one that overflowed leaves a finite scale (zero).
-            bad |= !(qq < kGcHuge) || !(kk < kGcHuge) || !(qs < kGcScale) || !(ks < kGcScale) || gc_bad(g) || gc_bad(b);
+            bad |= !(qq < kGcSquare) || !(kk < kGcSquare) || !(qs < kGcScale) || !(ks < kGcScale) || gc_bad(g) || gc_bad(b);
             sQs[t] = qs, sKs[t] = ks, sG[t] = g, sB[t] = b;
         }
     }
@@ -270,7 +270,7 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
     __shared__ __align__(1024) Buf buf[2];
     __shared__ __align__(16) gc_f4 ex[4][3][64];  // [wave][tile][lane]
     __shared__ float red[2][4][3][16];            // token-by-token chunks: [wave][sum][column]
-    __shared__ __align__(16) int huge[4];         // [wave]: its part of the present chunk's V and G K S0 is out of range
+    __shared__ __align__(16) int huge[4];         // [wave]: its part of the present chunk's V and S0 is out of range
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lk = lane >> 4;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), n = wv & 1, kh = wv >> 1;
     const int vh = A.value_heads, vd = A.vd, tiles = vd / kGcCols;
@@ -337,8 +337,18 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
     float *const orow = out + (static_cast<size_t>(s.row0) * vh + h) * vd + col;
     const size_t ostep = static_cast<size_t>(vh) * vd;
 
+    auto state_mag = [&] {  // of the lane's state elements; taken where they are made, off the walk's chain
+        gc_f4 m = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) m[i] += fabsf(st[i][q]);
+        return (m[0] + m[1]) + (m[2] + m[3]);
+    };
+    float st_mag;
+
     // One chunk from its operands (landed; all waves past the barrier that says so). False (for all waves alike), with
-    // the state as it was, when V or G K S0 is out of range.
+    // the state as it was, when V or S0 is out of range.
     auto chunk = [&](int c) {
         const Buf &f = buf[c & 1];
         auto a_row = [&](const float *m, int t, int i) {  // A operand: rows 16 t + lr, columns 64 kh + 16 i + 4 lk ..
@@ -419,20 +429,15 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
         ex[wv][0][lane] = x[0];
         ex[wv][1][lane] = x[1];
         ex[wv][2][lane] = kh == 0 ? o[1] : o[0];  // the partner's output rows
-        gc_f4 mag;
+        float mag = st_mag;
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            mag[q] = fmaf(fabsf(kg[0][q]), fabsf(x[0][q]), fmaf(fabsf(kg[1][q]), fabsf(x[1][q]), fabsf(vv[0][q]) + fabsf(vv[1][q])));
-        const int far = __any(!((mag[0] + mag[1]) + (mag[2] + mag[3]) < kGcHuge));
+        for (int q = 0; q < 4; ++q) mag += fabsf(vv[0][q]) + fabsf(vv[1][q]);
+        const int far = __any(!(mag < kGcHuge));
         if (lane == 0) huge[wv] = far;
         __syncthreads();
         const int pw = wv ^ 2;
         const gc_f4 xp[2] = {ex[pw][0][lane], ex[pw][1][lane]}, op = ex[pw][2][lane];
         const int4 any = *reinterpret_cast<const int4 *>(huge);
-        if (__builtin_amdgcn_readfirstlane(any.x | any.y | any.z | any.w)) {
-            vq::wait_vm<0>();
-            return false;
-        }
         // R = V - G K S0, then d / |k| = T R
         gc_f4 r[2], d[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, d1 = d[0];
 #pragma unroll
@@ -448,7 +453,7 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
         d[1] += d1;
         // S = G_C S + K^T (D(C - 1, .) d),  o = G (Q S0) + P d (the tile of P above the diagonal is zero)
         // The sums over the chunk's tokens start from zero and meet the larger terms once, in one fma.
-        gc_f4 y = {0.f, 0.f, 0.f, 0.f}, up[4] = {y, y, y, y};
+        gc_f4 y = {0.f, 0.f, 0.f, 0.f}, up[4] = {y, y, y, y}, next[4];
         const gc_f4 qs0 = (kh == 0 ? o[0] : o[1]) + op;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
@@ -464,10 +469,15 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
         for (int q = 0; q < 4; ++q) {
             y[q] = fmaf(qs0[q], qg[q], y[q]);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) st[i][q] = fmaf(st[i][q], gc, up[i][q]);
+            for (int i = 0; i < 4; ++i) next[i][q] = fmaf(st[i][q], gc, up[i][q]);
         }
 #undef VQ_GC_FENCE
         vq::wait_vm<0>();  // the next chunk's operands (not the stores that follow)
+        // Only now: a branch among the products cost 2.1 us of the walk's 60.
+        if (__builtin_amdgcn_readfirstlane(any.x | any.y | any.z | any.w)) return false;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) st[i] = next[i];
+        st_mag = state_mag();
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int t = c * kGcC + 16 * kh + 4 * lk + q;
@@ -530,6 +540,7 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
     const bool flagged = lane < cb - ca && slot0[lane * cstep + GcSlot::SC + GcSlot::BAD] != 0.0f;
     const uint64_t bad = __ballot(flagged);  // chunk ca + i of this launch: bit i
     vq::wait_vm<0>();
+    st_mag = state_mag();
     for (int c = ca; c < cb; ++c) {
         __syncthreads();  // chunk c landed for every wave; every wave is done with chunk c - 1's buffer
         bool done = false;
@@ -542,6 +553,7 @@ __global__ __launch_bounds__(256, 1) void gd_chunk_kernel(GcArgs A, SegTable T, 
         }
         if (!done) {
             serial(c);
+            st_mag = state_mag();
             vq::wait_vm<0>();
         }
     }
