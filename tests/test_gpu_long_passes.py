@@ -208,6 +208,38 @@ def test_gated_delta_chunks_keep_causality(rt, oracle_mod, what):
         assert np.abs(out[:, 0, rest] - clean[:, 0, rest]).max() <= 2e-6 * np.abs(clean).max()
 
 
+@pytest.mark.parametrize("elem", [4, 2])
+def test_gated_delta_many_long_segments(rt, oracle_mod, elem):
+    """A pass of twenty segments of 7 to 1100 rows: several groups of long ones, some of them over several launches, and
+    short ones. Every segment's bits are those of a pass of its own; the longest and the shortest long one are right."""
+    shape = kh, vh, kd, vd = 4, 48, 128, 32
+    rng = np.random.default_rng(9)
+    rows = [24, 1100, 40, 7, 513, 24, 90, 31, 32, 33, 64, 300, 24, 65, 25, 520, 128, 23, 48, 1]
+    slots = len(rows)
+    rt.alloc("pt", slots)
+    rt.set_paging("pt", 2048, 1, slots)
+    starts = np.cumsum([0] + rows)
+    inp = gated_delta_inputs(rng, int(starts[-1]), kh, vh, kd, vd, slots)
+    if elem == 2:
+        inp["state"] = inp["state"].astype(np.float16).astype(np.float32)
+    segs = [(slots - 1 - i, 0, n, int(starts[i])) for i, n in enumerate(rows)]
+    out, st = run_gated_delta(rt, inp, segs, shape, elem, 0, 1)
+    for i, n in enumerate(rows):
+        part = dict(inp, **{k: inp[k][starts[i]:starts[i + 1]] for k in ("conv", "b", "a")})
+        alone, fin = run_gated_delta(rt, part, [(slots - 1 - i, 0, n, 0)], shape, elem, 0, 1)
+        assert np.array_equal(alone, out[starts[i]:starts[i + 1]]), n
+        assert np.array_equal(fin[slots - 1 - i], st[slots - 1 - i]), n
+    head = dict(inp, conv=np.concatenate([inp["conv"][:, :kd], inp["conv"][:, kh * kd:(kh + 1) * kd],
+                                          inp["conv"][:, 2 * kh * kd:2 * kh * kd + vd]], 1), b=inp["b"][:, :1],
+                a=inp["a"][:, :1], ssm_a=inp["ssm_a"][:1], dt=inp["dt"][:1])  # head 0 by itself
+    for i in (0, 1):
+        expect, fin = gated_delta_rows(oracle_mod, head, segs[i:i + 1], inp["state"][:, :1], 1, 1, kd, vd, 0)
+        at = slice(starts[i], starts[i + 1])
+        assert np.abs(out[at, :1] - expect[at]).max() <= 2e-6 * np.abs(expect).max()
+        slot = segs[i][0]
+        assert np.abs(st[slot, :1] - fin[slot]).max() <= (2e-6 if elem == 4 else 5e-4) * np.abs(fin[slot]).max()
+
+
 # Largest error of the outputs and of the state, as a multiple of the per-token kernel's (measured: independent keys 0.85
 # and 0.8-1.1, correlated ones 1.1 and 1.1, equal ones 1.3-1.6 and 1.4-1.8).
 @pytest.mark.parametrize("keys,out_bound,state_bound", [("independent", 1.0, 1.25), ("correlated", 1.3, 1.3),

@@ -49,11 +49,17 @@
 namespace {
 
 constexpr int kGcC = 32, kGcKd = 128, kGcMaxVd = 128, kGcCols = 32;
-// Segments of at least this many rows take the chunks. Measured at 48 value heads, us token by token / in chunks: one
-// sequence of 16 rows 15.3 / 15.8, 24 rows 21.7 / 16.0, 64 rows 47.6 / 19.1; four of 16 rows 23.0 / 25.9, 24 rows
-// 32.2 / 26.6.
+// Segments of at least this many rows take the chunks. Measured at 48 value heads of 128, us token by token / in chunks:
+// one sequence of 16 rows 15.3 / 15.8, 24 rows 22.3 / 17.7, 512 rows 360 / 75; four of 24 rows 33.5 / 29.5; 16 of 24 rows
+// 93 / 89, 64 rows 223 / 142, 512 rows 1656 / 895; 64 of 24 rows 335 / 369 (the one loss: 32 rows 418 / 376, 512 rows
+// 6113 / 3570). The rule looks at a segment's own rows alone, so that its bits do not depend on the others of a pass.
 constexpr int kGcMinRows = 24;
-constexpr int kGcRound = 16;  // chunks per segment and launch pair at one segment (bounds the workspace)
+// Chunks of a segment per launch pair, and the bytes of a launch pair's chunk operands, which the segments of a group
+// share. With one launch pair for all long segments at 16 / n chunks each, every 32 tokens of nine and more took a pair of
+// launches and the state's way through memory: 64 segments of 512 rows 5919 us and 230 MB of workspace, now 3570 and 28;
+// 16 of 64 rows 178 -> 142; 64 of 512 rows, four heads of 64, 426 (403 token by token) -> 243.
+constexpr int kGcRound = 16;
+constexpr size_t kGcGroupBytes = size_t{32} << 20;
 static_assert(kGcRound <= 64, "one lane per chunk reads the non-finite flags");
 
 constexpr float kGcHuge = 1e28f, kGcSquare = 1e18f, kGcScale = 1e6f, kGcGrow = 1.0625f;
@@ -573,7 +579,7 @@ bool gc_shape(int key_heads, int value_heads, int kd, int vd) {
     return kd == kGcKd && vd % kGcCols == 0 && vd <= kGcMaxVd && key_heads >= 1 && value_heads >= key_heads &&
            value_heads % key_heads == 0;
 }
-// ... for these segments of a pass; chunks per launch and segment, and workspace bytes (0: no such segment).
+// ... for these segments of a pass (the longest first), which run in groups.
 int gc_segments(const SegTable &T, SegTable *longs, SegTable *shorts) {
     SegTable L{}, H{};
     for (int i = 0; i < T.n; ++i) {
@@ -581,36 +587,55 @@ int gc_segments(const SegTable &T, SegTable *longs, SegTable *shorts) {
         d.s[d.n++] = T.s[i];
         d.total += T.s[i].rows;
     }
+    std::stable_sort(L.s, L.s + L.n, [](const Seg &x, const Seg &y) { return x.rows > y.rows; });
     if (longs) *longs = L;
     if (shorts) *shorts = H;
     return L.n;
 }
-int gc_round(int nlong) { return nlong >= kGcRound ? 1 : kGcRound / nlong; }
+// The group that starts at segment i: its segments, the chunks of its longest one and those of a launch pair.
+struct GcGroup {
+    int n, chunks, cr;
+    size_t slots(int value_heads) const { return static_cast<size_t>(n) * cr * value_heads * GcSlot::floats; }
+};
+GcGroup gc_group(const SegTable &L, int i, int value_heads) {
+    const size_t budget = std::max<size_t>(1, kGcGroupBytes / (value_heads * GcSlot::floats * sizeof(float)));
+    GcGroup g;
+    g.chunks = (L.s[i].rows + kGcC - 1) / kGcC;
+    g.cr = static_cast<int>(std::min<size_t>(std::min(g.chunks, kGcRound), budget));
+    g.n = std::min(std::max(1, static_cast<int>(budget / g.cr)), L.n - i);
+    return g;
+}
 size_t gc_ws_bytes(const SegTable &T, int key_heads, int value_heads, int kd, int vd) {
     if (!gc_shape(key_heads, value_heads, kd, vd)) return 0;
     SegTable L;
-    const int n = gc_segments(T, &L, nullptr);
-    if (n == 0) return 0;
-    int nch = 1;
-    for (int i = 0; i < n; ++i) nch = std::max(nch, (L.s[i].rows + kGcC - 1) / kGcC);
-    const size_t slots = static_cast<size_t>(n) * std::min(gc_round(n), nch) * value_heads * GcSlot::floats;
-    const size_t copy = nch > gc_round(n) ? static_cast<size_t>(n) * value_heads * kGcKd * vd : 0;
-    return (slots + copy) * sizeof(float);
+    gc_segments(T, &L, nullptr);
+    size_t floats = 0;
+    for (int i = 0; i < L.n;) {
+        const GcGroup g = gc_group(L, i, value_heads);
+        const size_t copy = g.chunks > g.cr ? static_cast<size_t>(g.n) * value_heads * kGcKd * vd : 0;
+        floats = std::max(floats, g.slots(value_heads) + copy);
+        i += g.n;
+    }
+    return floats * sizeof(float);
 }
 
 template <typename ST>
 int gc_launch(const SegTable &L, const float *conv, const float *b, const float *a, const float *ssm_a, const float *dt,
               ST *state, float *out, int key_heads, int value_heads, int vd, float eps, int head_order, int write_state,
               float *ws, hipStream_t s) {
-    int nch = 1;
-    for (int i = 0; i < L.n; ++i) nch = std::max(nch, (L.s[i].rows + kGcC - 1) / kGcC);
-    GcArgs A{conv, b, a, ssm_a, dt, ws, key_heads, value_heads, vd, head_order, 0, std::min(gc_round(L.n), nch), eps};
-    float *const tmp = ws + static_cast<size_t>(L.n) * A.cr * value_heads * GcSlot::floats;
-    for (; A.c0 < nch; A.c0 += A.cr) {
-        gd_prep_kernel<<<dim3(value_heads, std::min(A.cr, nch - A.c0), L.n), 256, 0, s>>>(A, L);
-        gd_chunk_kernel<ST><<<dim3(value_heads * (vd / kGcCols), L.n), 256, 0, s>>>(A, L, state, tmp, out, write_state);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return status_of(e);
+    for (int i = 0; i < L.n;) {
+        const GcGroup g = gc_group(L, i, value_heads);
+        SegTable T{};
+        for (T.n = 0; T.n < g.n; ++T.n) T.s[T.n] = L.s[i + T.n];
+        i += g.n;
+        GcArgs A{conv, b, a, ssm_a, dt, ws, key_heads, value_heads, vd, head_order, 0, g.cr, eps};
+        float *const tmp = ws + g.slots(value_heads);
+        for (; A.c0 < g.chunks; A.c0 += A.cr) {
+            gd_prep_kernel<<<dim3(value_heads, std::min(A.cr, g.chunks - A.c0), T.n), 256, 0, s>>>(A, T);
+            gd_chunk_kernel<ST><<<dim3(value_heads * (vd / kGcCols), T.n), 256, 0, s>>>(A, T, state, tmp, out, write_state);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return status_of(e);
+        }
     }
     return VQ_OK;
 }
