@@ -331,7 +331,7 @@ def test_gated_delta_chunks_fp32_range(rt, oracle_mod, what):
         assert (diff.max((0, 1)) <= 5e-6 * size.max((0, 1))).all()
 
 
-# Key blocks of 32 in two parities, 16-row tiles, three or four heads of a kv head per workgroup.
+# Key blocks of 32 in two parities, 16-row tiles, two to four heads of a kv head per workgroup.
 @pytest.mark.parametrize("heads,kvh,hd", [(6, 1, 256), (5, 1, 64), (6, 2, 128), (9, 1, 64), (2, 2, 256)])
 @pytest.mark.parametrize("ntok,seq_len,window", [(9, 1, 0), (9, 24, 0), (16, 49, 0), (17, 48, 0), (33, 1, 5),
                                                  (20, 97, 40), (18, 64, 32)])
@@ -356,3 +356,68 @@ def test_prompt_attention_f16_blocks(rt, oracle_mod, heads, kvh, hd, ntok, seq_l
     put(rt, "pq", q[skip:])
     rt.attention("pq", "pkc", "pvc", "po", heads, kvh, hd, max_seq, seq_len + skip, 9, 0, window)
     assert np.array_equal(get(rt, "po", q.shape)[:9], got[skip:])
+
+
+# More workgroups than CUs over long contexts: a head's two parities in one wave. Passes of a few rows: in two waves.
+@pytest.mark.parametrize("G,hd", [(3, 64), (4, 128), (7, 64), (5, 128)])
+@pytest.mark.parametrize("window,bidirectional", [(0, 0), (33, 0), (300, 0), (0, 1)])
+def test_prompt_attention_f16_whole_heads(rt, oracle_mod, G, hd, window, bidirectional):
+    """Both forms give the same bits: a pass of 530 rows against passes of 64 rows of it, and rows at the tiles' edges
+    against the oracle (bar of the prompt attention tests)."""
+    rng = np.random.default_rng(hd + G + window)
+    kvh, ntok, before = 8, 530, 1200
+    heads, keys = G * kvh, before + ntok
+    print(f"whole heads G {G} hd {hd} window {window} bidirectional {bidirectional}", flush=True)
+    q = rng.standard_normal((ntok, heads, hd)).astype(np.float32)
+    kc = (rng.standard_normal((kvh, keys, hd)) * 0.3).astype(np.float16)
+    vc = rng.standard_normal((kvh, keys, hd)).astype(np.float16)
+    put(rt, "wk", kc, 2)
+    put(rt, "wv", vc, 2)
+    put(rt, "wq", q)
+    put(rt, "wo", np.full(q.size, np.nan))
+    rt.set_gemm_min_rows(9)
+    rt.attention("wq", "wk", "wv", "wo", heads, kvh, hd, keys, before + 1, ntok, bidirectional, window)
+    got = get(rt, "wo", q.shape)
+    if not bidirectional:
+        for r in (0, 64, ntok - 64):
+            put(rt, "wq", q[r:r + 64])
+            put(rt, "wo", np.full(q[:64].size, np.nan))
+            rt.attention("wq", "wk", "wv", "wo", heads, kvh, hd, keys, before + 1 + r, 64, 0, window)
+            assert np.array_equal(get(rt, "wo", q[:64].shape), got[r:r + 64]), r
+    rt.set_gemm_min_rows(0)
+    for r in (0, 15, 16, 511, ntok - 1):
+        seq = keys if bidirectional else before + 1 + r
+        ref = oracle_mod.attention(q[r:r + 1], kc, vc, heads, kvh, seq, False, window)
+        assert np.allclose(got[r:r + 1], ref, rtol=2e-5, atol=2e-5), r
+
+
+def test_prompt_attention_f16_whole_heads_paged(rt, oracle_mod):
+    """The same over pages: more than 256 workgroups in a pass of 48 sequences, each sequence's rows as in a
+    pass of its own."""
+    rng = np.random.default_rng(12)
+    heads, kvh, hd, page, pps, slots = 24, 8, 128, 64, 20, 48
+    pages = rng.permutation(pps * slots).astype(np.int32)
+    rt.alloc("wpt", pages.size)
+    rt.write("wpt", pages.tobytes())
+    rt.set_paging("wpt", page, pps, slots)
+    pool = (rng.standard_normal((pps * slots, kvh, page, hd)) * 0.3).astype(np.float16)
+    put(rt, "wk", pool, 2)
+    put(rt, "wv", pool[::-1], 2)
+    rows = [1 + 5 * (i % 4) for i in range(slots)]
+    starts = np.cumsum([0] + rows)
+    q = rng.standard_normal((int(starts[-1]), heads, hd)).astype(np.float32)
+    put(rt, "wq", q)
+    put(rt, "wo", np.full(q.size, np.nan))
+    rt.set_batch_invariant(True)
+    segs = [(slots - 1 - i, 1264 - 20 * i, n, int(starts[i])) for i, n in enumerate(rows)]
+    rt.set_segments(segs)
+    rt.attention_seg("wq", "wk", "wv", "wo", heads, kvh, hd)
+    got = get(rt, "wo", q.shape)
+    for i in (0, 1, 23, 47):
+        part = q[starts[i]:starts[i + 1]]
+        put(rt, "wq", part)
+        put(rt, "wo", np.full(part.size, np.nan))
+        rt.set_segments([segs[i][:3] + (0,)])
+        rt.attention_seg("wq", "wk", "wv", "wo", heads, kvh, hd)
+        assert np.array_equal(get(rt, "wo", part.shape), got[starts[i]:starts[i + 1]]), i
+    rt.set_batch_invariant(False)

@@ -880,35 +880,40 @@ __device__ __forceinline__ void fa16_consume(const Fa16Raw<HD> &rw, int kb, int 
     __builtin_amdgcn_wave_barrier();
 }
 
-// Prompt passes on fp16 caches: a workgroup takes 16 query rows of one segment and up to four query heads of one kv
-// head. Wave w takes head w >> 1 and every second 32-key block (the blocks of parity w & 1) with its own online softmax;
-// the two waves of a head are combined through LDS at the end. Blocks start at multiples of 32 keys whatever the rows
-// of the tile, so a row's sums do not depend on the other rows of its pass.
-// Each step (64 keys, one block per parity): all 512 threads load the next step's K and V into registers, the waves
-// consume the present one from LDS, the registers go to the other LDS buffer: one barrier per step. The loads are
-// issued after the S products, which would otherwise wait behind them in the address unit. K is [32][HD + 16] f16
-// (the S^T A fragments are 16-byte reads; 95 us against 96 with rows of HD + 8), V^T as in the decode kernel. The cache
-// rows of a step's keys are looked up once per workgroup, two steps ahead.
-// Why: one wave per SIMD (290 registers, two blocks in flight) left every read, conversion and barrier exposed, and
-// three heads for each half of the waves keep all 256 CUs at work where four and two did not. 512 rows over 2048 keys,
-// 24 heads of 256 on 4 kv heads: 167 -> 76 us (45 GFLOP issued, 590 TFLOP/s). Two waves of a SIMD need 2090 cycles of
-// matrix products and 1900 of other vector instructions per step and do both in step; giving one of them priority
-// changed nothing.
-template <int HD, bool PAGED>
-__global__ __launch_bounds__(512) void attention_prompt16_kernel(const float *__restrict__ q,
+// Prompt passes on fp16 caches: a workgroup of NW waves takes 16 query rows of one segment and up to NW / PH query heads of
+// one kv head. The 32-key blocks of each parity have an online softmax of their own, and the two are combined at the end:
+// PH 2, a head's two waves take a parity each and meet in LDS; PH 1, one wave takes both. The same sums either way. Blocks
+// start at multiples of 32 keys whatever the rows of the tile, so a row's sums do not depend on the other rows of its pass.
+// Each step (64 keys, one block per parity): all threads load the next step's K and V into registers, the waves consume the
+// present one from LDS, the registers go to the other LDS buffer: one barrier per step. The loads are issued after the S
+// products, which would otherwise wait behind them in the address unit. K is [32][HD + 16] f16 (the S^T A fragments are
+// 16-byte reads; 95 us against 96 with rows of HD + 8), V^T as in the decode kernel. The cache rows of a step's keys are
+// looked up once per workgroup, two steps ahead.
+// Why: hd 256, one wave per SIMD (290 registers, two blocks in flight) left every read, conversion and barrier exposed, and
+// three heads for each half of the waves keep all 256 CUs at work where four and two did not. 512 rows over 2048 keys, 24
+// heads of 256 on 4 kv heads: 167 -> 76 us (45 GFLOP issued, 590 TFLOP/s). Two waves of a SIMD need 2090 cycles of matrix
+// products and 1900 of other vector instructions per step and do both in step; giving one of them priority changed nothing.
+// For hd 64 and 128, see launch_prompt16.
+template <int HD, bool PAGED, int NW, int PH>
+__global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attention_prompt16_kernel(const float *__restrict__ q,
                                                                  const _Float16 *__restrict__ kc,
                                                                  const _Float16 *__restrict__ vc, float *__restrict__ out,
                                                                  SegTable T, KvMap M, int heads, int bidirectional,
                                                                  int window, int chunks, int hpw) {
     constexpr int CR = HD / 8, LDK = HD + 16;
-    constexpr int KU = 32 * CR / 256;                  // K chunks per thread per block
-    constexpr int VU = 8 * CR / 256 > 0 ? 8 * CR / 256 : 1;  // V units (HD 64: half the threads take one)
+    constexpr int ST = 32 * NW;                        // threads that stage a block
+    constexpr int KU = 32 * CR / ST;                   // K chunks per thread per block
+    constexpr int VU = 8 * CR > ST ? 8 * CR / ST : 1;  // V units (fewer units than threads: some take none)
+    constexpr int NP = 2 / PH;                         // parities of a wave
+    // Steps from the first block that holds a key, blocks past the last key skipped, nothing loaded in the last step: where
+    // workgroups queue for the CUs (2048 rows, windows of 256: 41 -> 39 us; the other forms lose 2 % to the branches).
+    constexpr bool TIGHT = PH == 1;
     constexpr int KB = 32 * LDK, VB = HD * 32;         // f16 elements of a staged block
     __shared__ __align__(16) _Float16 kv[2][2][KB + VB];  // [buffer][parity]
     __shared__ __align__(16) size_t rowtab[2][64];     // first element of the cache row of a step's keys
-    __shared__ float sml[4][2][16];
+    __shared__ float sml[NW / 2][2][16];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int c = lane & 15, g = lane >> 4, par = wv & 1;
+    const int c = lane & 15, g = lane >> 4, hw = wv / PH, par = wv % PH;
     // Consecutive workgroups take the kv heads in turn (with 8 (kv head, chunk) pairs each XCD's L2 holds one kv head),
     // the last tiles, which see the most keys, first.
     const int per = M.kv_heads * chunks, kvc = blockIdx.x % per, kvh = kvc / chunks, gi0 = (kvc - kvh * chunks) * hpw;
@@ -919,8 +924,8 @@ __global__ __launch_bounds__(512) void attention_prompt16_kernel(const float *__
     }
     const Seg &s = T.s[si];
     const int G = heads / M.kv_heads;
-    const int gi = gi0 + (wv >> 1);
-    const bool wave_on = (wv >> 1) < hpw && gi < G;
+    const int gi = gi0 + hw;
+    const bool wave_on = hw < hpw && gi < G;
     const int h = kvh * G + (wave_on ? gi : 0);
     const int t0 = 16 * tb, nq = min(16, s.rows - t0);
     const int seq_len0 = s.pos0 + 1;
@@ -929,22 +934,23 @@ __global__ __launch_bounds__(512) void attention_prompt16_kernel(const float *__
     const int tq = t0 + min(c, nq - 1);  // this lane's query row (rows past nq repeat the last; not written)
     const int qs = q_start(tq), qe = q_end(tq);
     const int k_lo = q_start(t0), k_hi = q_end(t0 + nq - 1);
-    const int k0 = k_lo & ~63, steps = (k_hi - k0 + 63) / 64;
+    const int k0 = k_lo & (TIGHT ? ~31 : ~63), steps = (k_hi - k0 + 63) / 64;
+    const int flip = TIGHT ? k0 >> 5 & 1 : 0;  // a step's first block is of this parity
     // Keys outside [k_lo, k_hi) read the nearest key of the range (they are masked).
     auto key_of = [&](int step) { return min(max(k0 + 64 * step + lane, k_lo), k_hi - 1); };
     if (wv < 2) rowtab[wv][lane] = M.row_t<PAGED>(s.slot, kvh, key_of(wv)) * HD;
     float4 qr[HD / 16];
     fa16_q_load<HD>(q + (static_cast<size_t>(s.row0 + tq) * heads + h) * HD, qr);
     __syncthreads();
-    // Half sp of the threads stages the block of parity sp: K chunks i = st + 256 k (key i / CR, chunk i % CR), V units
-    // st + 256 k (key quad & 7, chunk >> 3).
-    const int sp = tid >> 8, st = tid & 255;
+    // Half sp of the threads stages the block of parity sp: K chunks i = st + ST k (key i / CR, chunk i % CR), V units
+    // st + ST k (key quad & 7, chunk >> 3).
+    const int sp = tid / ST, st = tid % ST;
     fh8 rk[KU], rv[VU][4];
     auto issue_k = [&](int step) {
         const size_t *rt = rowtab[step & 1] + 32 * sp;
 #pragma unroll
         for (int k = 0; k < KU; ++k) {
-            const int i = st + 256 * k;
+            const int i = st + ST * k;
             rk[k] = ld_h8(kc + rt[i / CR] + 8 * (i % CR));
         }
     };
@@ -952,7 +958,7 @@ __global__ __launch_bounds__(512) void attention_prompt16_kernel(const float *__
         const size_t *rt = rowtab[step & 1] + 32 * sp;
 #pragma unroll
         for (int k = 0; k < VU; ++k) {
-            const int i = (st + 256 * k) % (8 * CR);
+            const int i = (st + ST * k) % (8 * CR);
 #pragma unroll
             for (int j = 0; j < 4; ++j) rv[k][j] = ld_h8(vc + rt[4 * (i & 7) + j] + 8 * (i >> 3));
         }
@@ -961,12 +967,12 @@ __global__ __launch_bounds__(512) void attention_prompt16_kernel(const float *__
         _Float16 *kd = kv[step & 1][sp], *vd = kd + KB;
 #pragma unroll
         for (int k = 0; k < KU; ++k) {
-            const int i = st + 256 * k;
+            const int i = st + ST * k;
             *reinterpret_cast<fh8 *>(kd + (i / CR) * LDK + 8 * (i % CR)) = rk[k];
         }
 #pragma unroll
         for (int k = 0; k < VU; ++k) {
-            const int i = st + 256 * k;
+            const int i = st + ST * k;
             if (i < 8 * CR) fa16_put_vt<HD>(vd, i & 7, i >> 3, rv[k]);
         }
     };
@@ -974,72 +980,86 @@ __global__ __launch_bounds__(512) void attention_prompt16_kernel(const float *__
     issue_v(0);
     fh8 qh[HD / 32], ql[HD / 32];
     const float sinv = fa16_q_split<HD>(qr, 1.0f / sqrtf(static_cast<float>(HD)), qh, ql);
-    float m = -INFINITY, l = 0.0f;
-    fa4 o[HD / 16];
+    float m[NP], l[NP];
+    fa4 o[NP][HD / 16];
 #pragma unroll
-    for (int b = 0; b < HD / 16; ++b) o[b] = fa4{0.f, 0.f, 0.f, 0.f};
+    for (int p = 0; p < NP; ++p) {
+        m[p] = -INFINITY, l[p] = 0.0f;
+#pragma unroll
+        for (int b = 0; b < HD / 16; ++b) o[p][b] = fa4{0.f, 0.f, 0.f, 0.f};
+    }
     stage(0);
     __syncthreads();
     for (int step = 0; step < steps; ++step) {
         const bool more = step + 1 < steps;
         const int nkey = key_of(step + 2);
         int npage = 0;
-        if (PAGED && wv == 7) npage = M.page_of(s.slot, nkey);
-        if (!wave_on) {
+        if (PAGED && wv == NW - 1) npage = M.page_of(s.slot, nkey);
+        if (!wave_on && (more || !TIGHT)) {
             issue_k(step + 1);
             issue_v(step + 1);
         }
         if (wave_on) {
-            const _Float16 *ks = kv[step & 1][par], *vts = ks + KB;
-            fa4 sc[2];
 #pragma unroll
-            for (int hh = 0; hh < 2; ++hh) {
-                fa4 a0{0.f, 0.f, 0.f, 0.f}, a1{0.f, 0.f, 0.f, 0.f};
-                const _Float16 *kp = ks + (16 * hh + c) * LDK + 8 * g;
+            for (int p = 0; p < NP; ++p) {
+                const int own = (NP * par + p) ^ flip, kb = k0 + 64 * step + 32 * own;
+                if (TIGHT && kb >= k_hi) continue;
+                const _Float16 *ks = kv[step & 1][own], *vts = ks + KB;
+                fa4 sc[2];
 #pragma unroll
-                for (int u = 0; u < HD / 32; ++u) {
-                    const fh8 a = *reinterpret_cast<const fh8 *>(kp + 32 * u);
-                    a0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qh[u], a0, 0, 0, 0);
-                    a1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, ql[u], a1, 0, 0, 0);
+                for (int hh = 0; hh < 2; ++hh) {
+                    fa4 a0{0.f, 0.f, 0.f, 0.f}, a1{0.f, 0.f, 0.f, 0.f};
+                    const _Float16 *kp = ks + (16 * hh + c) * LDK + 8 * g;
+#pragma unroll
+                    for (int u = 0; u < HD / 32; ++u) {
+                        const fh8 a = *reinterpret_cast<const fh8 *>(kp + 32 * u);
+                        a0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qh[u], a0, 0, 0, 0);
+                        a1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, ql[u], a1, 0, 0, 0);
+                    }
+                    sc[hh] = (a0 + a1) * sinv;
                 }
-                sc[hh] = (a0 + a1) * sinv;
+                fa16_ahead<HD / 16>();
+                __builtin_amdgcn_sched_barrier(0);
+                if (p == 0 && (more || !TIGHT)) {
+                    issue_k(step + 1);
+                    issue_v(step + 1);
+                }
+                fa16_softmax_pv<HD>(sc, kb, k_hi, qs, qe, vts, m[p], l[p], o[p]);
             }
-            fa16_ahead<HD / 16>();
-            __builtin_amdgcn_sched_barrier(0);
-            issue_k(step + 1);
-            issue_v(step + 1);
-            fa16_softmax_pv<HD>(sc, k0 + 64 * step + 32 * par, k_hi, qs, qe, vts, m, l, o);
         }
         if (more) stage(step + 1);
-        if (wv == 7) rowtab[step & 1][lane] = M.row_in<PAGED>(npage, kvh, nkey) * HD;
+        if (wv == NW - 1) rowtab[step & 1][lane] = M.row_in<PAGED>(npage, kvh, nkey) * HD;
         __syncthreads();
     }
-    // Wave 2 i + 1 hands its sums to wave 2 i (same lane layout): 16 query vectors x HD fp32 per head.
-    float *oh = reinterpret_cast<float *>(&kv[0][0][0]) + (wv >> 1) * 16 * HD;
-    if (par == 1) {
+    // The two parities of a head meet: wave 2 i + 1 hands its sums to wave 2 i (same lane layout), 16 query vectors x HD
+    // fp32 per head; one wave with both has them already.
+    float *oh = reinterpret_cast<float *>(&kv[0][0][0]) + hw * 16 * HD;
+    if constexpr (PH == 2) {
+        if (par == 1) {
 #pragma unroll
-        for (int b = 0; b < HD / 16; ++b) *reinterpret_cast<fa4 *>(oh + 256 * b + 4 * lane) = o[b];
-        if (g == 0) {
-            sml[wv >> 1][0][c] = m;
-            sml[wv >> 1][1][c] = l;
+            for (int b = 0; b < HD / 16; ++b) *reinterpret_cast<fa4 *>(oh + 256 * b + 4 * lane) = o[0][b];
+            if (g == 0) {
+                sml[hw][0][c] = m[0];
+                sml[hw][1][c] = l[0];
+            }
         }
+        __syncthreads();
     }
-    __syncthreads();
-    // o[b][r]: head dim 16 b + 4 g + r of query row tq
+    // o[.][b][r]: head dim 16 b + 4 g + r of query row tq
     if (wave_on && par == 0 && c < nq) {
         float *orow = out + (static_cast<size_t>(s.row0 + t0 + c) * heads + h) * HD;
-        const float m1 = sml[wv >> 1][0][c], l1 = sml[wv >> 1][1][c];
-        const float mx = fmaxf(m, m1);
-        const float f0 = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mx);
+        const float m1 = PH == 2 ? sml[hw][0][c] : m[NP - 1], l1 = PH == 2 ? sml[hw][1][c] : l[NP - 1];
+        const float mx = fmaxf(m[0], m1);
+        const float f0 = m[0] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m[0] - mx);
         const float f1 = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m1 - mx);
-        const float lt = fmaf(l1, f1, l * f0);
+        const float lt = fmaf(l1, f1, l[0] * f0);
         const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
 #pragma unroll
         for (int b = 0; b < HD / 16; ++b) {
-            const fa4 o1 = *reinterpret_cast<const fa4 *>(oh + 256 * b + 4 * lane);
+            const fa4 o1 = PH == 2 ? *reinterpret_cast<const fa4 *>(oh + 256 * b + 4 * lane) : o[NP - 1][b];
             float r[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) r[j] = fmaf(o1[j], f1, o[b][j] * f0) * inv;
+            for (int j = 0; j < 4; ++j) r[j] = fmaf(o1[j], f1, o[0][b][j] * f0) * inv;
             *reinterpret_cast<float4 *>(orow + 16 * b + 4 * g) = float4{r[0], r[1], r[2], r[3]};
         }
     }
@@ -1649,18 +1669,37 @@ void launch_mfma_hd(bool fast, dim3 grid, hipStream_t s, const float *q, const C
                                                                 chunks);
 }
 
-// Query heads per workgroup: a kv head's heads dealt evenly over as few workgroups as four heads each allow (6: 3 + 3).
+// Query heads per workgroup: a kv head's heads dealt evenly over as few workgroups as the form allows (6 of up to four:
+// 3 + 3). Every form gives the same bits, so the choice may look at the pass. hd 256: eight waves, up to four heads in
+// halves. hd 64 and 128: four waves, up to two heads in halves (whose 170 registers let two workgroups and more share a
+// CU), or, with three heads and more of a kv head, up to four heads, each whole in one wave: less work in all (K and V
+// staged once for four heads, queries split once), more per wave. The whole form pays when it has more than a workgroup for
+// every CU, and the shorter the contexts the later; under a short window from 192 workgroups on (192: 15.8 / 14.6 us, 128:
+// 12.5 / 14.1). hd 128, 32 heads on 8 kv heads, halves / whole, us (eight waves of
+// halves, the kernel before that): 512 rows 17.4 / 20.3 (20.8, 25.5), over 2048 keys 54 / 62 (58, 85); 640 rows 20.5 / 24.7
+// (23.5, 36), over 2048 keys 84 / 66 (85, 109); 2048 rows 141 / 113 (141, 188), windows of 256 53 / 39 (55, 49); 16 heads
+// of their own, 512 rows over 2048 keys 45 (82, 88), windows of 128 11 (19, 14).
 template <bool PAGED>
 void launch_prompt16(int tiles, hipStream_t s, const float *q, const _Float16 *kc, const _Float16 *vc, float *out,
-                     const SegTable &T, const KvMap &M, int heads, int hd, int bidirectional, int window, int chunks) {
-    const int G = heads / M.kv_heads, hpw = (G + chunks - 1) / chunks;
-    const dim3 grid(static_cast<unsigned>(tiles) * M.kv_heads * chunks);
-    if (hd == 64)
-        attention_prompt16_kernel<64, PAGED><<<grid, 512, 0, s>>>(q, kc, vc, out, T, M, heads, bidirectional, window, chunks, hpw);
-    else if (hd == 128)
-        attention_prompt16_kernel<128, PAGED><<<grid, 512, 0, s>>>(q, kc, vc, out, T, M, heads, bidirectional, window, chunks, hpw);
-    else
-        attention_prompt16_kernel<256, PAGED><<<grid, 512, 0, s>>>(q, kc, vc, out, T, M, heads, bidirectional, window, chunks, hpw);
+                     const SegTable &T, const KvMap &M, int heads, int hd, int bidirectional, int window) {
+    const int G = heads / M.kv_heads;
+    const int pairs = tiles * M.kv_heads;
+    auto go = [&](auto kernel, int waves, int most) {
+        const int chunks = (G + most - 1) / most, hpw = (G + chunks - 1) / chunks;
+        const dim3 grid(static_cast<unsigned>(pairs) * chunks);
+        kernel<<<grid, 64 * waves, 0, s>>>(q, kc, vc, out, T, M, heads, bidirectional, window, chunks, hpw);
+    };
+    constexpr int kCus = 256, kLong = 1000, kBrief = 512;
+    int keys = 0;
+    for (int i = 0; i < T.n; ++i) keys = max(keys, T.s[i].pos0 + T.s[i].rows);
+    const long long wgs = static_cast<long long>(pairs) * ((G + 3) / 4);
+    const bool whole = G > 2 && (window > 0 && window <= kBrief ? wgs >= kCus * 3 / 4
+                                                                : wgs > kCus && wgs * min(keys, kLong) > kCus * kLong);
+    if (hd == 256) go(attention_prompt16_kernel<256, PAGED, 8, 2>, 8, 4);
+    else if (hd == 128 && whole) go(attention_prompt16_kernel<128, PAGED, 4, 1>, 4, 4);
+    else if (hd == 128) go(attention_prompt16_kernel<128, PAGED, 4, 2>, 4, 2);
+    else if (whole) go(attention_prompt16_kernel<64, PAGED, 4, 1>, 4, 4);
+    else go(attention_prompt16_kernel<64, PAGED, 4, 2>, 4, 2);
 }
 
 // fp16 caches with hd 64, 128 or 256 and 16-byte aligned q, K, V and out: the f16 MFMA kernels.
@@ -1679,8 +1718,8 @@ void launch_attention_mfma(const float *q, const C *kc, const C *vc, float *out,
     const dim3 grid(tiles, M.kv_heads * chunks);
     if constexpr (sizeof(C) == 2) {
         if (fa16_ok(q, kc, vc, out, hd)) {
-            if (M.pt != nullptr) launch_prompt16<true>(tiles, s, q, kc, vc, out, T, M, heads, hd, bidirectional, window, chunks);
-            else launch_prompt16<false>(tiles, s, q, kc, vc, out, T, M, heads, hd, bidirectional, window, chunks);
+            if (M.pt != nullptr) launch_prompt16<true>(tiles, s, q, kc, vc, out, T, M, heads, hd, bidirectional, window);
+            else launch_prompt16<false>(tiles, s, q, kc, vc, out, T, M, heads, hd, bidirectional, window);
             return;
         }
     }
