@@ -17,6 +17,7 @@ from __future__ import annotations
 import contextlib
 import ctypes
 import math
+import types
 from dataclasses import dataclass
 from typing import Sequence
 
@@ -42,8 +43,11 @@ class _Tensor:
     home: str = "own"  # where the bytes live: "own" allocation, "arena", or "group:<id>"
     streamed: bool = False  # uploaded with resident=False (served from HBM all the same)
 
+    lent: bool = False  # data is a caller's own tensor (upload_device): see _Buffer.lent
+
     def __post_init__(self) -> None:
-        self.ptr = self.data.data_ptr()  # data lives as long as this entry; asking torch costs 0.2 us per use
+        self.address = self.data.data_ptr
+        self.ptr = self.address()
 
 
 @dataclass
@@ -70,9 +74,16 @@ WEIGHT_GRANULE = 2 << 20
 class _Buffer:
     data: torch.Tensor  # float32 or float16
     elem: int
+    # data was handed out (buffer_tensor): its storage may be exchanged or resized, so every use asks for the address
+    # (0.1 us), and for the size where that has changed. A storage that is this entry's alone keeps both.
+    lent: bool = False
 
     def __post_init__(self) -> None:
-        self.ptr, self.n = self.data.data_ptr(), self.data.numel()
+        self.address = self.data.data_ptr
+        self.look_again()
+
+    def look_again(self) -> None:
+        self.ptr, self.n = self.address(), self.data.numel()
 
 
 def _check_upload_args(name: str, nbytes_given: int, type_id: int, cols: int, rows: int) -> tuple[int, int]:
@@ -157,12 +168,16 @@ class Runtime:
         t = self.tensors.get(name)
         if t is None:
             raise KeyError(f"weight tensor {name} is not loaded")
+        if t.lent:
+            t.ptr = t.address()
         return t
 
     def _any_buffer(self, name: str) -> _Buffer:
         b = self.buffers.get(name)
         if b is None:
             raise KeyError(f"device buffer {name} is not allocated")
+        if b.lent and b.address() != b.ptr:
+            b.look_again()
         return b
 
     def _f32_buffer(self, name: str, min_n: int) -> _Buffer:
@@ -170,6 +185,8 @@ class Runtime:
         b = self.buffers.get(name)
         if b is None:
             raise KeyError(f"device buffer {name} is not allocated")
+        if b.lent and b.address() != b.ptr:
+            b.look_again()
         if b.elem != 4:
             raise TypeError(f"device buffer {name} is fp16 (KV cache), not fp32")
         if b.n < min_n:
@@ -225,7 +242,7 @@ class Runtime:
             raise ValueError(f"{name}: device tensor needs {nbytes + 16} bytes (16 bytes of tail padding)")
         if data.data_ptr() % 16:
             raise ValueError(f"{name}: device tensor must be 16-byte aligned")
-        self.tensors[name] = _Tensor(data, int(type_id), int(rows), int(cols), row_bytes, nbytes)
+        self.tensors[name] = _Tensor(data, int(type_id), int(rows), int(cols), row_bytes, nbytes, lent=True)
 
     def free(self, name: str) -> None:
         if name not in self.tensors:
@@ -401,8 +418,11 @@ class Runtime:
         return self._any_buffer(name).elem
 
     def buffer_tensor(self, name: str) -> torch.Tensor:
-        """The torch tensor behind a buffer (for zero-copy interop)."""
-        return self._any_buffer(name).data
+        """The torch tensor behind a buffer (for zero-copy interop). From then on every call asks it for its address and
+        size, so that an exchanged or resized storage is followed."""
+        b = self._any_buffer(name)
+        b.lent = True
+        return b.data
 
     # ---- the hot path -------------------------------------------------------------------------------
     def qmv(self, weight: str, x: str, y: str, ntok: int = 1) -> None:
@@ -713,6 +733,13 @@ class Runtime:
         self._seg_ready()
         return self._seg_span
 
+    def _page_table(self) -> tuple[int, int, int]:
+        """Address of the page table, page size and pages per sequence."""
+        pt, page, pps, _ = self._paging
+        if pt.lent and pt.address() != pt.ptr:
+            pt.look_again()
+        return pt.ptr, page, pps
+
     def _seg_chunks(self) -> list[tuple[ctypes.Array, int]]:
         """The segment table as int32 arrays of at most VQ_MAX_SEGMENTS segments (one launch each)."""
         return self._seg_tables
@@ -744,10 +771,10 @@ class Runtime:
         rowsz = kv_heads * hd
         kb, vb = self._f32_buffer(k, rowsz * self._seg_rows()), self._f32_buffer(v, rowsz * self._seg_rows())
         kcb, vcb = self._kv_pair(kc, vc, rowsz)
-        pt, page, pps, _ = self._paging
+        pt, page, pps = self._page_table()
         for arr, n in self._seg_chunks():
             _lib.check(self._lib.vq_kv_append_seg(kb.ptr, vb.ptr, kcb.ptr, vcb.ptr,
-                                                  kcb.elem, arr, n, kv_heads, hd, pt.ptr, page, pps,
+                                                  kcb.elem, arr, n, kv_heads, hd, pt, page, pps,
                                                   self._stream()), "kv_append_seg")
 
     def attention_seg(self, q: str, kc: str, vc: str, out: str, heads: int, kv_heads: int, hd: int) -> None:
@@ -760,19 +787,19 @@ class Runtime:
         qb = self._f32_buffer(q, rowsz * self._seg_rows())
         kcb, vcb = self._kv_pair(kc, vc, 1)
         ob = self._f32_buffer(out, rowsz * self._seg_rows())
-        pt, page, pps, _ = self._paging
+        pt, page, pps = self._page_table()
         tiled = self._tiled_attention(self._seg_longest)
         for arr, n in self._seg_chunks():
             if tiled:  # prompt rows in the pass, or batch-invariant mode
                 _lib.check(self._lib.vq_attention_seg_tiled(qb.ptr, kcb.ptr, vcb.ptr,
                                                             ob.ptr, kcb.elem, arr, n, heads, kv_heads, hd,
-                                                            pt.ptr, page, pps, self._stream()), "attention_seg")
+                                                            pt, page, pps, self._stream()), "attention_seg")
                 continue
             nws = self._lib.vq_attention_seg_workspace_bytes(arr, n, heads, kv_heads, hd)
             ws = self._workspace(nws).data_ptr() if nws else None
             _lib.check(self._lib.vq_attention_seg_ws(qb.ptr, kcb.ptr, vcb.ptr,
                                                      ob.ptr, kcb.elem, arr, n, heads, kv_heads, hd,
-                                                     pt.ptr, page, pps, ws, nws, self._stream()),
+                                                     pt, page, pps, ws, nws, self._stream()),
                        "attention_seg")
 
     def conv_update_seg(self, x: str, state: str, w: str, out: str, channels: int, K: int, snap: str | None = None,
@@ -782,7 +809,7 @@ class Runtime:
         segs = self._seg_ready()
         if K > _lib.VQ_CONV_MAX_K:
             raise ValueError(f"conv kernel size {K} > {_lib.VQ_CONV_MAX_K}")
-        ntok, stride = self._seg_rows(), channels * K
+        ntok, stride = self._seg_span, channels * K
         xb = self._f32_buffer(x, channels * ntok)
         sb = self._f32_buffer(state, stride * self._paging[3])
         ob = self._f32_buffer(out, channels * ntok)
@@ -805,7 +832,7 @@ class Runtime:
         segs = self._seg_ready()
         if key_heads <= 0 or value_heads % key_heads != 0:
             raise ValueError("value heads must be a multiple of key heads")
-        ntok = self._seg_rows()
+        ntok = self._seg_span
         conv_dim = 2 * key_heads * kd + value_heads * vd
         state_n = value_heads * kd * vd
         cb = self._f32_buffer(conv, conv_dim * ntok)
@@ -1041,4 +1068,7 @@ class HipWeightRuntime:
         self._rt.write(name, np.ascontiguousarray(values, dtype="<f4").tobytes(), offset)
 
     def __getattr__(self, name: str):
-        return getattr(self._rt, name)
+        value = getattr(self._rt, name)
+        if isinstance(value, types.MethodType):  # found without this detour (0.4 us) from now on
+            self.__dict__[name] = value
+        return value
