@@ -17,6 +17,7 @@ from __future__ import annotations
 import contextlib
 import ctypes
 import math
+import threading
 import types
 from dataclasses import dataclass
 from typing import Sequence
@@ -109,6 +110,43 @@ def _check_qmv_args(name: str, cols: int, ntok: int) -> None:
         raise ValueError(f"{name}: matvec cols must be a multiple of 32")
 
 
+class _Scratch:
+    """Device scratch of one stream's calls: the workspace, the argmax ids and the batch-invariant argmax's logits, grown
+    on demand and reused in stream order. Calls on different streams may overlap on the device and have one each; calls
+    of several threads on one stream hold `lock` from the first look at the scratch to their last launch (and reading the
+    ids), so that one call's launches are not torn apart by another's. Memory that was outgrown is kept: a captured graph
+    may still replay into it (sizes at least double, so it is less than the present one's)."""
+
+    def __init__(self, device: torch.device) -> None:
+        self.lock = threading.RLock()
+        self.device = device
+        self.argmax = torch.empty(MAX_ARGMAX_ROWS, dtype=torch.int32, device=device)
+        self.argmax_ptr = self.argmax.data_ptr()
+        self.held: dict[str, torch.Tensor] = {}
+        self.outgrown: list[torch.Tensor] = []
+
+    def _get(self, what: str, nbytes: int) -> int:
+        t = self.held.get(what)
+        if t is None or t.numel() < nbytes:
+            size = nbytes
+            if t is not None:
+                size = max(nbytes, 2 * t.numel())
+                self.outgrown.append(t)
+            t = self.held[what] = torch.empty(size, dtype=torch.uint8, device=self.device)
+        return t.data_ptr()
+
+    def workspace(self, nbytes: int) -> int | None:
+        """Address of nbytes of workspace; None for none."""
+        return self._get("workspace", nbytes) if nbytes else None
+
+    def logits(self, n: int) -> int:
+        """Address of n fp32 logits (apart from the workspace, which the matvec itself may use)."""
+        return self._get("logits", 4 * n)
+
+    def nbytes(self) -> int:
+        return 4 * self.argmax.numel() + sum(t.numel() for t in (*self.held.values(), *self.outgrown))
+
+
 class Runtime:
     """Persistent device store of raw GGUF tensors and fp32 buffers, keyed by name."""
 
@@ -126,8 +164,7 @@ class Runtime:
                 _lib.check(self._lib.vq_set_iq3s_grid(grid), "vq_set_iq3s_grid")
         self.tensors: dict[str, _Tensor] = {}
         self.buffers: dict[str, _Buffer] = {}
-        self._argmax_out = torch.empty(MAX_ARGMAX_ROWS, dtype=torch.int32, device=self.device)
-        self._ws: dict[int, torch.Tensor] = {}  # per stream: calls on different streams may overlap
+        self._scratches: dict[int, _Scratch] = {}  # by stream
         self.gemm_min_rows = 0
         self.batch_invariant = False
         self.gemm_f16_activations = False
@@ -147,22 +184,18 @@ class Runtime:
         # torch.cuda.current_stream(device).cuda_stream without the Stream object (0.9 us less on every call)
         return torch._C._cuda_getCurrentRawStream(self.device.index)
 
-    def _workspace(self, nbytes: int) -> torch.Tensor:
-        """Device scratch of the calls on the current stream, grown on demand and reused (stream-ordered)."""
+    def _scratch(self) -> _Scratch:
+        """The current stream's scratch."""
         stream = self._stream()
-        ws = self._ws.get(stream)
-        if ws is None or ws.numel() < nbytes:
-            size = nbytes if ws is None else max(nbytes, 2 * ws.numel())
-            ws = self._ws[stream] = torch.empty(size, dtype=torch.uint8, device=self.device)
-        return ws
+        scratch = self._scratches.get(stream)
+        return scratch if scratch is not None else self._scratches.setdefault(stream, _Scratch(self.device))
 
-    def _logits_scratch(self, n: int) -> torch.Tensor:
-        """fp32 logits of the batch-invariant argmax when the caller keeps none: grown on demand and reused
-        (separate from the workspace, which the matvec itself may use)."""
-        buf = getattr(self, "_logits", None)
-        if buf is None or buf.numel() < n:
-            buf = self._logits = torch.empty(n, dtype=torch.float32, device=self.device)
-        return buf
+    def _launch(self, nws: int, call, *args) -> int:
+        """call(*args, workspace, nws, stream) on the current stream."""
+        if not nws:
+            return call(*args, None, 0, self._stream())
+        with (sc := self._scratch()).lock:
+            return call(*args, sc.workspace(nws), nws, self._stream())
 
     def _tensor(self, name: str) -> _Tensor:
         t = self.tensors.get(name)
@@ -334,11 +367,11 @@ class Runtime:
 
     def vram_bytes(self) -> int:
         """Device memory this runtime holds: arena, weight groups, tensors in their own allocations, buffers and
-        the matvec workspace (qwen_runtime.cu:1436-1446)."""
+        the scratch of each stream it was used on (qwen_runtime.cu:1436-1446)."""
         total = sum(g.data.numel() for g in self._groups)
         total += self._arena.data.numel() if self._arena is not None else 0
         total += sum(t.data.numel() for t in self.tensors.values() if t.home == "own")
-        return total + self.buffer_bytes() + sum(w.numel() for w in self._ws.values())
+        return total + self.buffer_bytes() + sum(s.nbytes() for s in list(self._scratches.values()))
 
     def buffer_bytes(self) -> int:
         return sum(b.data.numel() * b.elem for b in self.buffers.values())
@@ -444,26 +477,21 @@ class Runtime:
             ng = self._lib.vq_qgemm_workspace_bytes_ex(t.type, t.rows, t.cols, ntok, flags)
             if self.gemm_f16_activations and ng:
                 # The reference's own numerics: fp32 activations rounded to f16 inside the call.
-                buf = self._workspace(ng)
-                st = self._lib.vq_qgemm_f16x_ws(t.type, t.ptr, t.rows, t.cols, x_ptr, ntok, y_ptr,
-                                                buf.data_ptr(), ng, flags, self._stream())
+                with (sc := self._scratch()).lock:
+                    st = self._lib.vq_qgemm_f16x_ws(t.type, t.ptr, t.rows, t.cols, x_ptr, ntok, y_ptr,
+                                                    sc.workspace(ng), ng, flags, self._stream())
                 _lib.check(st, "qgemm launch")
                 return
             nx = (self._lib.vq_xpack_bytes(t.cols, ntok) + 255) // 256 * 256
-            buf = self._workspace(nx + ng)
-            xp = buf.data_ptr()
-            _lib.check(self._lib.vq_pack_x(x_ptr, ntok, t.cols, xp, self._stream()), "pack_x")
-            st = self._lib.vq_qgemm_ws_ex(t.type, t.ptr, t.rows, t.cols, xp, ntok, y_ptr,
-                                          (xp + nx) if ng else None, ng, flags, self._stream())
+            with (sc := self._scratch()).lock:
+                xp = sc.workspace(nx + ng)
+                _lib.check(self._lib.vq_pack_x(x_ptr, ntok, t.cols, xp, self._stream()), "pack_x")
+                st = self._lib.vq_qgemm_ws_ex(t.type, t.ptr, t.rows, t.cols, xp, ntok, y_ptr,
+                                              (xp + nx) if ng else None, ng, flags, self._stream())
             _lib.check(st, "qgemm launch")
             return
-        if t.type in (0, 1):
-            ws = None
-            nws = 0
-        else:
-            nws = self._lib.vq_qmv_workspace_bytes_for(t.type, t.rows, t.cols, ntok)
-            ws = self._workspace(nws).data_ptr() if nws else None
-        st = self._lib.vq_qmv(t.type, t.ptr, t.rows, t.cols, x_ptr, ntok, y_ptr, ws, nws, self._stream())
+        nws = 0 if t.type in (0, 1) else self._lib.vq_qmv_workspace_bytes_for(t.type, t.rows, t.cols, ntok)
+        st = self._launch(nws, self._lib.vq_qmv, t.type, t.ptr, t.rows, t.cols, x_ptr, ntok, y_ptr)
         _lib.check(st, "qmv launch")
 
     def qmv_staged(self, weight: str, x: str, y: str, ntok: int = 1, *, x2: str | None = None,
@@ -499,10 +527,8 @@ class Runtime:
         # 5-16 tokens of the f16 small-batch types stage inside that kernel (vq_qmv_staged_ws, with the RMS
         # prepass and partial sums in the runtime's workspace); other calls stream (vq_qmv_staged).
         nws = self._lib.vq_qmv_staged_workspace_bytes(t.type, t.rows, t.cols, ntok)
-        ws = self._workspace(nws) if nws else None
-        st = self._lib.vq_qmv_staged_ws(t.type, t.ptr, t.rows, t.cols, xb.ptr, x2p, nwp,
-                                        float(eps), flags, ntok, yb.ptr, ws.data_ptr() if ws is not None else None,
-                                        nws, self._stream())
+        st = self._launch(nws, self._lib.vq_qmv_staged_ws, t.type, t.ptr, t.rows, t.cols, xb.ptr, x2p, nwp, float(eps),
+                          flags, ntok, yb.ptr)
         _lib.check(st, "qmv_staged launch")
 
     # ---- ops around the matvec (the reference runtime's elementwise / norm ops) ------------------------------
@@ -612,10 +638,8 @@ class Runtime:
                                                     int(bidirectional), int(window), self._stream()), "attention")
             return
         nws = self._lib.vq_attention_workspace_bytes(heads, kv_heads, hd, seq_len, ntok, int(window))
-        ws = self._workspace(nws).data_ptr() if nws else None
-        _lib.check(self._lib.vq_attention_ws(qb.ptr, kcb.ptr, vcb.ptr, ob.ptr,
-                                             kcb.elem, heads, kv_heads, hd, max_seq, seq_len, ntok, int(bidirectional),
-                                             int(window), ws, nws, self._stream()), "attention")
+        _lib.check(self._launch(nws, self._lib.vq_attention_ws, qb.ptr, kcb.ptr, vcb.ptr, ob.ptr, kcb.elem, heads, kv_heads,
+                                hd, max_seq, seq_len, ntok, int(bidirectional), int(window)), "attention")
 
     def conv_update(self, x: str, state: str, w: str, out: str, channels: int, K: int, ntok: int = 1,
                     snap: str | None = None, write_state: int = 1) -> None:
@@ -652,20 +676,18 @@ class Runtime:
         sa, dtt = self._f32_weight(ssm_a, value_heads), self._f32_weight(dt, value_heads)
         snp = self._f32_buffer(snap, state_n * (ntok - 1)).ptr if snap is not None else None
         seg = (ctypes.c_int32 * 4)(0, 0, ntok, 0)
-        ws, nws = self._gated_delta_ws(seg, 1, ntok, key_heads, value_heads, kd, vd, snp)
-        _lib.check(self._lib.vq_gated_delta_seg_ws(cb.ptr, bb.ptr, ab.ptr, sa.ptr,
-                                                   dtt.ptr, sb.ptr, 4, ob.ptr, key_heads,
-                                                   value_heads, kd, vd, float(eps), int(head_order), seg, 1, snp,
-                                                   int(bool(write_state)), ws, nws, self._stream()), "gated_delta")
+        nws = self._gated_delta_ws(seg, 1, ntok, key_heads, value_heads, kd, vd, snp)
+        _lib.check(self._launch(nws, self._lib.vq_gated_delta_seg_ws, cb.ptr, bb.ptr, ab.ptr, sa.ptr, dtt.ptr, sb.ptr, 4,
+                                ob.ptr, key_heads, value_heads, kd, vd, float(eps), int(head_order), seg, 1, snp,
+                                int(bool(write_state))), "gated_delta")
 
     def _gated_delta_ws(self, segs, nseg: int, rows: int, key_heads: int, value_heads: int, kd: int, vd: int,
-                        snap: int | None) -> tuple[int | None, int]:
-        """Workspace (address, bytes) of the chunked gated delta kernels: none for decode-length passes, snapshot
-        passes, and batch-invariant mode (a token's sums then do not depend on where its prompt was cut into passes)."""
+                        snap: int | None) -> int:
+        """Workspace bytes of the chunked gated delta kernels: none for decode-length passes, snapshot passes, and
+        batch-invariant mode (a token's sums then do not depend on where its prompt was cut into passes)."""
         if snap is not None or rows <= MAX_TOKENS or self.batch_invariant:
-            return None, 0
-        nws = self._lib.vq_gated_delta_seg_workspace_bytes(segs, nseg, key_heads, value_heads, kd, vd)
-        return (self._workspace(nws).data_ptr() if nws else None), nws
+            return 0
+        return self._lib.vq_gated_delta_seg_workspace_bytes(segs, nseg, key_heads, value_heads, kd, vd)
 
     def concat_rows(self, dst: str, a: str, b: str, rows: int, width: int) -> None:
         """dst[r] = [a[r] | b[r]] for rows of width floats (Runtime_concat_rows, qwen_runtime.cu:2567-2587)."""
@@ -716,10 +738,8 @@ class Runtime:
             raise ValueError("no segments")
         self._segments = table
         # Built once for the pass: every layer's *_seg ops read them.
-        self._seg_tables = []
-        for i in range(0, len(table), _lib.VQ_MAX_SEGMENTS):
-            part = table[i:i + _lib.VQ_MAX_SEGMENTS]
-            self._seg_tables.append(((ctypes.c_int32 * (4 * len(part)))(*[v for sg in part for v in sg]), len(part)))
+        parts = [table[i:i + _lib.VQ_MAX_SEGMENTS] for i in range(0, len(table), _lib.VQ_MAX_SEGMENTS)]
+        self._seg_tables = [((ctypes.c_int32 * (4 * len(p)))(*[v for sg in p for v in sg]), len(p)) for p in parts]
         self._seg_span = max(r0 + n for _, _, n, r0 in table)
         self._seg_longest = max(n for _, _, n, _ in table)
         return row0
@@ -796,11 +816,8 @@ class Runtime:
                                                             pt, page, pps, self._stream()), "attention_seg")
                 continue
             nws = self._lib.vq_attention_seg_workspace_bytes(arr, n, heads, kv_heads, hd)
-            ws = self._workspace(nws).data_ptr() if nws else None
-            _lib.check(self._lib.vq_attention_seg_ws(qb.ptr, kcb.ptr, vcb.ptr,
-                                                     ob.ptr, kcb.elem, arr, n, heads, kv_heads, hd,
-                                                     pt, page, pps, ws, nws, self._stream()),
-                       "attention_seg")
+            _lib.check(self._launch(nws, self._lib.vq_attention_seg_ws, qb.ptr, kcb.ptr, vcb.ptr, ob.ptr, kcb.elem, arr, n,
+                                    heads, kv_heads, hd, pt, page, pps), "attention_seg")
 
     def conv_update_seg(self, x: str, state: str, w: str, out: str, channels: int, K: int, snap: str | None = None,
                         write_state: int = 1) -> None:
@@ -851,12 +868,10 @@ class Runtime:
             snp = self._f32_buffer(snap, state_n * (ntok - 1)).ptr
         rows = self._seg_longest
         for arr, n in self._seg_chunks():
-            ws, nws = self._gated_delta_ws(arr, n, rows, key_heads, value_heads, kd, vd, snp)
-            _lib.check(self._lib.vq_gated_delta_seg_ws(cb.ptr, bb.ptr, ab.ptr, sa.ptr,
-                                                       dtt.ptr, sbuf.ptr, sbuf.elem, ob.ptr,
-                                                       key_heads, value_heads, kd, vd, float(eps), int(head_order), arr,
-                                                       n, snp, int(bool(write_state)), ws, nws, self._stream()),
-                       "gated_delta_seg")
+            nws = self._gated_delta_ws(arr, n, rows, key_heads, value_heads, kd, vd, snp)
+            _lib.check(self._launch(nws, self._lib.vq_gated_delta_seg_ws, cb.ptr, bb.ptr, ab.ptr, sa.ptr, dtt.ptr, sbuf.ptr,
+                                    sbuf.elem, ob.ptr, key_heads, value_heads, kd, vd, float(eps), int(head_order), arr, n,
+                                    snp, int(bool(write_state))), "gated_delta_seg")
 
     def copy(self, dst: str, dst_off: int, src: str, src_off: int, n: int) -> None:
         """dst[dst_off:+n] = src[src_off:+n] in elements, buffers of one precision (Runtime_copy,
@@ -903,9 +918,7 @@ class Runtime:
             # One type: the streaming group launch, or for small batches the MFMA paths qmv would take (5-16
             # tokens of Q3_K..Q6_K as one launch over all the matrices).
             nws = self._lib.vq_qmv_group_workspace_bytes(t0.type, n, ra, t0.cols, ntok)
-            ws = self._workspace(nws).data_ptr() if nws else None
-            st = self._lib.vq_qmv_group_ws(t0.type, n, wa, ra, ya, t0.cols, xb.ptr, ntok, ws, nws,
-                                           self._stream())
+            st = self._launch(nws, self._lib.vq_qmv_group_ws, t0.type, n, wa, ra, ya, t0.cols, xb.ptr, ntok)
         _lib.check(st, "qmv_group launch")
 
     def lmhead_argmax(self, weight: str, x: str, ntok: int = 1, logits: str | None = None) -> list[int]:
@@ -920,20 +933,18 @@ class Runtime:
             raise ValueError(f"{weight}: lmhead_argmax needs a quantized weight")
         _check_qmv_args(weight, t.cols, ntok)
         xb = self._f32_buffer(x, t.cols * ntok)
-        if self.batch_invariant:  # the matvec on the invariant path, then the row argmax
-            yp = (self._f32_buffer(logits, t.rows * ntok).ptr if logits is not None
-                  else self._logits_scratch(t.rows * ntok).data_ptr())
-            self._qmv_ptrs(t, xb.ptr, yp, ntok)
-            _lib.check(self._lib.vq_argmax_rows(yp, t.rows, ntok, self._argmax_out.data_ptr(),
-                                                self._stream()), "argmax_rows")
-            return [int(v) for v in self._argmax_out[:ntok].tolist()]
-        lp = self._f32_buffer(logits, t.rows * ntok).ptr if logits is not None else None
-        nws = self._lib.vq_lmhead_argmax_workspace_bytes(t.type, t.rows, t.cols, ntok)
-        ws = self._workspace(nws)
-        st = self._lib.vq_lmhead_argmax(t.type, t.ptr, t.rows, t.cols, xb.ptr, ntok,
-                                        self._argmax_out.data_ptr(), lp, ws.data_ptr(), nws, self._stream())
-        _lib.check(st, "lmhead_argmax")
-        return [int(v) for v in self._argmax_out[:ntok].tolist()]
+        with (sc := self._scratch()).lock:
+            if self.batch_invariant:  # the matvec on the invariant path, then the row argmax
+                yp = self._f32_buffer(logits, t.rows * ntok).ptr if logits is not None else sc.logits(t.rows * ntok)
+                self._qmv_ptrs(t, xb.ptr, yp, ntok)
+                _lib.check(self._lib.vq_argmax_rows(yp, t.rows, ntok, sc.argmax_ptr, self._stream()), "argmax_rows")
+                return sc.argmax[:ntok].tolist()
+            lp = self._f32_buffer(logits, t.rows * ntok).ptr if logits is not None else None
+            nws = self._lib.vq_lmhead_argmax_workspace_bytes(t.type, t.rows, t.cols, ntok)
+            st = self._lib.vq_lmhead_argmax(t.type, t.ptr, t.rows, t.cols, xb.ptr, ntok, sc.argmax_ptr, lp,
+                                            sc.workspace(nws), nws, self._stream())
+            _lib.check(st, "lmhead_argmax")
+            return sc.argmax[:ntok].tolist()
 
     def qmv_tensor(self, weight: str, x: torch.Tensor, y: torch.Tensor | None = None) -> torch.Tensor:
         """Tensor form: x [ntok, cols] fp32 on the device -> y [ntok, rows] fp32."""
@@ -968,17 +979,18 @@ class Runtime:
     def argmax(self, name: str, n: int) -> int:
         """Index of the largest of the first n floats; ties -> lowest index (Runtime_argmax, :2167-2179)."""
         xb = self._f32_buffer(name, n)
-        _lib.check(self._lib.vq_argmax_rows(xb.ptr, n, 1, self._argmax_out.data_ptr(), self._stream()), "argmax")
-        return int(self._argmax_out[0].item())
+        with (sc := self._scratch()).lock:
+            _lib.check(self._lib.vq_argmax_rows(xb.ptr, n, 1, sc.argmax_ptr, self._stream()), "argmax")
+            return int(sc.argmax[0].item())
 
     def argmax_rows(self, name: str, n: int, ntok: int) -> list[int]:
         """Row-wise argmax of ntok rows of n floats (Runtime_argmax_rows, :2181-2197)."""
         if ntok < 1 or ntok > MAX_ARGMAX_ROWS:
             raise ValueError(f"ntok must be in [1, {MAX_ARGMAX_ROWS}]")
         xb = self._f32_buffer(name, n * ntok)
-        _lib.check(self._lib.vq_argmax_rows(xb.ptr, n, ntok, self._argmax_out.data_ptr(), self._stream()),
-                   "argmax_rows")
-        return [int(v) for v in self._argmax_out[:ntok].tolist()]
+        with (sc := self._scratch()).lock:
+            _lib.check(self._lib.vq_argmax_rows(xb.ptr, n, ntok, sc.argmax_ptr, self._stream()), "argmax_rows")
+            return sc.argmax[:ntok].tolist()
 
     def set_gemm_min_rows(self, n: int) -> None:
         """qmv calls with ntok >= n take the MFMA prefill contraction (0 = never) (qwen_runtime.cu:2324-2330)."""
