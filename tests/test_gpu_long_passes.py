@@ -240,6 +240,55 @@ def test_gated_delta_many_long_segments(rt, oracle_mod, elem):
         assert np.abs(st[slot, :1] - fin[slot]).max() <= (2e-6 if elem == 4 else 5e-4) * np.abs(fin[slot]).max()
 
 
+def test_gated_delta_batch_invariant_cuts(rt):
+    """In batch-invariant mode a prompt's bits do not depend on where it is cut into passes: 70 rows at once, as 40 + 30, and
+    as 40 rows beside another sequence's and 30 alone; outside the mode the first of them runs in chunks."""
+    shape = kh, vh, kd, vd = 1, 2, 128, 64
+    rng = np.random.default_rng(13)
+    rt.alloc("pt", 64)
+    rt.set_paging("pt", 128, 16, 4)
+    inp = gated_delta_inputs(rng, 110, kh, vh, kd, vd, 4)
+
+    def part(lo, hi, state=inp["state"]):
+        return dict(inp, state=state, **{k: inp[k][lo:hi] for k in ("conv", "b", "a")})
+
+    chunked, _ = run_gated_delta(rt, part(0, 70), [(1, 0, 70, 0)], shape, 4, 0, 1)
+    rt.set_batch_invariant(True)
+    whole, fin = run_gated_delta(rt, part(0, 70), [(1, 0, 70, 0)], shape, 4, 0, 1)
+    first, mid = run_gated_delta(rt, part(0, 40), [(1, 0, 40, 0)], shape, 4, 0, 1)
+    beside, st = run_gated_delta(rt, inp, [(2, 0, 40, 70), (1, 0, 40, 0)], shape, 4, 0, 1)
+    assert np.array_equal(first, whole[:40]) and np.array_equal(beside[:40], whole[:40])
+    assert np.array_equal(st[1], mid[1])
+    rest, end = run_gated_delta(rt, part(40, 70, mid), [(1, 40, 30, 0)], shape, 4, 0, 1)
+    assert np.array_equal(rest, whole[40:]) and np.array_equal(end[1], fin[1])
+    rt.set_batch_invariant(False)
+    assert not np.array_equal(chunked, whole)
+    assert np.abs(chunked - whole).max() <= 4e-6 * np.abs(whole).max()
+
+
+@pytest.mark.parametrize("bad", [5, 511, 512, 600, 699])
+def test_gated_delta_chunks_flagged_in_any_launch(rt, oracle_mod, bad):
+    """One infinite value in a pass of 22 chunks over two launch pairs, in each of them and at their edge: its column from its
+    token on, and nothing else (bound as above)."""
+    shape = kh, vh, kd, vd = 1, 2, 128, 64
+    rng = np.random.default_rng(14)
+    n = 700
+    rt.alloc("pt", 64)
+    rt.set_paging("pt", 1024, 16, 1)
+    inp = gated_delta_inputs(rng, n, kh, vh, kd, vd, 1)
+    segs = [(0, 0, n, 0)]
+    expect, fin = gated_delta_rows(oracle_mod, inp, segs, inp["state"], kh, vh, kd, vd, 0)
+    inp["conv"][bad, 2 * kh * kd + vd + 37] = -np.inf  # head 1, column 37
+    out, st = run_gated_delta(rt, inp, segs, shape, 4, 0, 1)
+    touched = np.zeros((n, vh, vd), bool)
+    touched[bad:, 1, 37] = True
+    assert np.array_equal(~np.isfinite(out), touched)
+    assert np.abs(np.where(touched, 0, out - expect)).max() <= 2e-6 * np.abs(expect).max()
+    assert not np.isfinite(st[0, 1, :, 37]).any()
+    st[0, 1, :, 37] = fin[0, 1, :, 37] = 0.0
+    assert np.abs(st - fin).max() <= 2e-6 * np.abs(fin).max()
+
+
 # Largest error of the outputs and of the state, as a multiple of the per-token kernel's (measured: independent keys 0.85
 # and 0.8-1.1, correlated ones 1.1 and 1.1, equal ones 1.3-1.6 and 1.4-1.8).
 @pytest.mark.parametrize("keys,out_bound,state_bound", [("independent", 1.0, 1.25), ("correlated", 1.3, 1.3),

@@ -1001,7 +1001,8 @@ class Runtime:
     def set_batch_invariant(self, on: bool = True) -> None:
         """Every pass on the kernels whose per-row results do not depend on the other rows of the pass: qmv through
         the prompt contraction with a K split fixed by the matrix (gemm_min_rows = 1), attention through the tiled
-        kernel. The reference's --batch-invariant mode (qwen_cli.py:47-49; it sets gemm_min_rows to 1 for every
+        kernel, gated delta token by token (outside the mode segments of 24 rows and more run in chunks, and a token's sums
+        depend on where its prompt was cut into passes). The reference's --batch-invariant mode (qwen_cli.py:47-49; it sets gemm_min_rows to 1 for every
         pass, qwen_gpu.py:738-744): slower for a lone request, and a request's outputs never depend on what runs
         beside it. Off restores gemm_min_rows = 0."""
         self.batch_invariant = bool(on)
