@@ -170,7 +170,7 @@ class Runtime:
         self.gemm_f16_activations = False
         self._paging: tuple[_Buffer, int, int, int] | None = None
         self._segments: list[tuple[int, int, int, int]] = []
-        self._seg_tables: list[tuple[ctypes.Array, int]] = []  # the same as int32 tables of one launch each
+        self._seg_tables: list[tuple[ctypes.Array, int]] = []  # as int32 tables of one launch each
         self._seg_span = self._seg_longest = 0
         # Resident-weight memory: an optional arena and the executor's per-layer weight groups. Nothing streams
         # over PCIe here, so the stream order only records which uploads were requested as streamed.
@@ -676,16 +676,15 @@ class Runtime:
         sa, dtt = self._f32_weight(ssm_a, value_heads), self._f32_weight(dt, value_heads)
         snp = self._f32_buffer(snap, state_n * (ntok - 1)).ptr if snap is not None else None
         seg = (ctypes.c_int32 * 4)(0, 0, ntok, 0)
-        nws = self._gated_delta_ws(seg, 1, ntok, key_heads, value_heads, kd, vd, snp)
+        nws = self._gated_delta_ws(seg, 1, key_heads, value_heads, kd, vd, snp) if ntok > MAX_TOKENS else 0
         _lib.check(self._launch(nws, self._lib.vq_gated_delta_seg_ws, cb.ptr, bb.ptr, ab.ptr, sa.ptr, dtt.ptr, sb.ptr, 4,
                                 ob.ptr, key_heads, value_heads, kd, vd, float(eps), int(head_order), seg, 1, snp,
                                 int(bool(write_state))), "gated_delta")
 
-    def _gated_delta_ws(self, segs, nseg: int, rows: int, key_heads: int, value_heads: int, kd: int, vd: int,
-                        snap: int | None) -> int:
-        """Workspace bytes of the chunked gated delta kernels: none for decode-length passes, snapshot passes, and
-        batch-invariant mode (a token's sums then do not depend on where its prompt was cut into passes)."""
-        if snap is not None or rows <= MAX_TOKENS or self.batch_invariant:
+    def _gated_delta_ws(self, segs, nseg: int, key_heads: int, value_heads: int, kd: int, vd: int, snap: int | None) -> int:
+        """Workspace bytes of the chunked gated delta kernels: none for snapshot passes and batch-invariant mode (a
+        token's sums then do not depend on where its prompt was cut into passes)."""
+        if snap is not None or self.batch_invariant:
             return 0
         return self._lib.vq_gated_delta_seg_workspace_bytes(segs, nseg, key_heads, value_heads, kd, vd)
 
@@ -760,10 +759,6 @@ class Runtime:
             pt.look_again()
         return pt.ptr, page, pps
 
-    def _seg_chunks(self) -> list[tuple[ctypes.Array, int]]:
-        """The segment table as int32 arrays of at most VQ_MAX_SEGMENTS segments (one launch each)."""
-        return self._seg_tables
-
     def _kv_pair(self, kc: str, vc: str, min_n: int) -> tuple[_Buffer, _Buffer]:
         """find_kv_buffer for a K/V cache pair of one precision (qwen_runtime.cu:1226-1248)."""
         kcb, vcb = self._any_buffer(kc), self._any_buffer(vc)
@@ -780,7 +775,7 @@ class Runtime:
         if rot <= 0 or rot % 2 != 0 or rot > hd:
             raise ValueError(f"invalid rotary dim {rot}")
         xb = self._f32_buffer(x, heads * hd * self._seg_rows())
-        for arr, n in self._seg_chunks():
+        for arr, n in self._seg_tables:
             _lib.check(self._lib.vq_rope_seg(xb.ptr, arr, n, heads, hd, rot, float(base), self._stream()),
                        "rope_seg")
 
@@ -792,7 +787,7 @@ class Runtime:
         kb, vb = self._f32_buffer(k, rowsz * self._seg_rows()), self._f32_buffer(v, rowsz * self._seg_rows())
         kcb, vcb = self._kv_pair(kc, vc, rowsz)
         pt, page, pps = self._page_table()
-        for arr, n in self._seg_chunks():
+        for arr, n in self._seg_tables:
             _lib.check(self._lib.vq_kv_append_seg(kb.ptr, vb.ptr, kcb.ptr, vcb.ptr,
                                                   kcb.elem, arr, n, kv_heads, hd, pt, page, pps,
                                                   self._stream()), "kv_append_seg")
@@ -809,7 +804,7 @@ class Runtime:
         ob = self._f32_buffer(out, rowsz * self._seg_rows())
         pt, page, pps = self._page_table()
         tiled = self._tiled_attention(self._seg_longest)
-        for arr, n in self._seg_chunks():
+        for arr, n in self._seg_tables:
             if tiled:  # prompt rows in the pass, or batch-invariant mode
                 _lib.check(self._lib.vq_attention_seg_tiled(qb.ptr, kcb.ptr, vcb.ptr,
                                                             ob.ptr, kcb.elem, arr, n, heads, kv_heads, hd,
@@ -836,7 +831,7 @@ class Runtime:
             if len(segs) != 1:
                 raise ValueError("snapshots need a single-segment pass")
             snp = self._f32_buffer(snap, stride * (ntok - 1)).ptr
-        for arr, n in self._seg_chunks():
+        for arr, n in self._seg_tables:
             _lib.check(self._lib.vq_conv_update_seg(xb.ptr, sb.ptr, wt.ptr, ob.ptr, channels,
                                                     K, arr, n, snp, int(bool(write_state)), self._stream()),
                        "conv_update_seg")
@@ -867,11 +862,17 @@ class Runtime:
                 raise ValueError("snapshots need a single-segment pass")
             snp = self._f32_buffer(snap, state_n * (ntok - 1)).ptr
         rows = self._seg_longest
-        for arr, n in self._seg_chunks():
-            nws = self._gated_delta_ws(arr, n, rows, key_heads, value_heads, kd, vd, snp)
-            _lib.check(self._launch(nws, self._lib.vq_gated_delta_seg_ws, cb.ptr, bb.ptr, ab.ptr, sa.ptr, dtt.ptr, sbuf.ptr,
-                                    sbuf.elem, ob.ptr, key_heads, value_heads, kd, vd, float(eps), int(head_order), arr, n,
-                                    snp, int(bool(write_state))), "gated_delta_seg")
+        for arr, n in self._seg_tables:
+            if rows <= MAX_TOKENS:  # decode and verify passes, which are short: the call itself
+                st = self._lib.vq_gated_delta_seg(cb.ptr, bb.ptr, ab.ptr, sa.ptr, dtt.ptr, sbuf.ptr, sbuf.elem, ob.ptr,
+                                                  key_heads, value_heads, kd, vd, float(eps), int(head_order), arr, n, snp,
+                                                  int(bool(write_state)), self._stream())
+            else:
+                nws = self._gated_delta_ws(arr, n, key_heads, value_heads, kd, vd, snp)
+                st = self._launch(nws, self._lib.vq_gated_delta_seg_ws, cb.ptr, bb.ptr, ab.ptr, sa.ptr, dtt.ptr, sbuf.ptr,
+                                  sbuf.elem, ob.ptr, key_heads, value_heads, kd, vd, float(eps), int(head_order), arr, n, snp,
+                                  int(bool(write_state)))
+            _lib.check(st, "gated_delta_seg")
 
     def copy(self, dst: str, dst_off: int, src: str, src_off: int, n: int) -> None:
         """dst[dst_off:+n] = src[src_off:+n] in elements, buffers of one precision (Runtime_copy,
