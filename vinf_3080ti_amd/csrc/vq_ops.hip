@@ -784,6 +784,26 @@ __device__ __forceinline__ void fa16_ahead() {
     __builtin_amdgcn_sched_group_barrier(kMfma, 2 * kFaAhead, 0);
 }
 
+// S^T of a 32-key block from its K rows in LDS (ks, HD + 16 apart): sc[h] holds keys 16 h + 4 g + r of query column c.
+template <int HD>
+__device__ __forceinline__ void fa16_scores(const _Float16 *ks, int c, int g, const fh8 (&qh)[HD / 32],
+                                            const fh8 (&ql)[HD / 32], float sinv, fa4 (&sc)[2]) {
+#pragma unroll
+    for (int hh = 0; hh < 2; ++hh) {
+        fa4 a0{0.f, 0.f, 0.f, 0.f}, a1{0.f, 0.f, 0.f, 0.f};
+        const _Float16 *kp = ks + (16 * hh + c) * (HD + 16) + 8 * g;
+#pragma unroll
+        for (int u = 0; u < HD / 32; ++u) {
+            const fh8 a = *reinterpret_cast<const fh8 *>(kp + 32 * u);
+            a0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qh[u], a0, 0, 0, 0);
+            a1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, ql[u], a1, 0, 0, 0);
+        }
+        sc[hh] = (a0 + a1) * sinv;
+    }
+    fa16_ahead<HD / 16>();
+    __builtin_amdgcn_sched_barrier(0);
+}
+
 // Online softmax over the S^T values of block [kb, kb + 32) (s[h][r]: key kb + 16 h + 4 g + r, query column c sees
 // keys [qs, qe), keys at or past k_hi masked), then O^T += V^T P^T from the block's V^T in LDS (vt, read at rows
 // 16 b + c, positions 8 g ..). The caller makes vt visible first.
@@ -895,7 +915,7 @@ __device__ __forceinline__ void fa16_consume(const Fa16Raw<HD> &rw, int kb, int 
 // products and 1900 of other vector instructions per step and do both in step; giving one of them priority changed nothing.
 // For hd 64 and 128, see launch_prompt16.
 template <int HD, bool PAGED, int NW, int PH>
-__global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attention_prompt16_kernel(const float *__restrict__ q,
+__global__ __launch_bounds__(64 * NW, 2) void attention_prompt16_kernel(const float *__restrict__ q,
                                                                  const _Float16 *__restrict__ kc,
                                                                  const _Float16 *__restrict__ vc, float *__restrict__ out,
                                                                  SegTable T, KvMap M, int heads, int bidirectional,
@@ -913,7 +933,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attention_prompt16_k
     __shared__ __align__(16) size_t rowtab[2][64];     // first element of the cache row of a step's keys
     __shared__ float sml[NW / 2][2][16];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int c = lane & 15, g = lane >> 4, hw = wv / PH, par = wv % PH;
+    const int c = lane & 15, g = lane >> 4, hw = wv / PH, par = wv & (PH - 1);
     // Consecutive workgroups take the kv heads in turn (with 8 (kv head, chunk) pairs each XCD's L2 holds one kv head),
     // the last tiles, which see the most keys, first.
     const int per = M.kv_heads * chunks, kvc = blockIdx.x % per, kvh = kvc / chunks, gi0 = (kvc - kvh * chunks) * hpw;
@@ -944,7 +964,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attention_prompt16_k
     __syncthreads();
     // Half sp of the threads stages the block of parity sp: K chunks i = st + ST k (key i / CR, chunk i % CR), V units
     // st + ST k (key quad & 7, chunk >> 3).
-    const int sp = tid / ST, st = tid % ST;
+    const int sp = tid / ST, st = tid & (ST - 1);
     fh8 rk[KU], rv[VU][4];
     auto issue_k = [&](int step) {
         const size_t *rt = rowtab[step & 1] + 32 * sp;
@@ -1000,31 +1020,25 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attention_prompt16_k
             issue_v(step + 1);
         }
         if (wave_on) {
-#pragma unroll
-            for (int p = 0; p < NP; ++p) {
-                const int own = (NP * par + p) ^ flip, kb = k0 + 64 * step + 32 * own;
-                if (TIGHT && kb >= k_hi) continue;
+            const int own = (NP * par) ^ flip;
+            if (!TIGHT || k0 + 64 * step + 32 * own < k_hi) {
                 const _Float16 *ks = kv[step & 1][own], *vts = ks + KB;
                 fa4 sc[2];
-#pragma unroll
-                for (int hh = 0; hh < 2; ++hh) {
-                    fa4 a0{0.f, 0.f, 0.f, 0.f}, a1{0.f, 0.f, 0.f, 0.f};
-                    const _Float16 *kp = ks + (16 * hh + c) * LDK + 8 * g;
-#pragma unroll
-                    for (int u = 0; u < HD / 32; ++u) {
-                        const fh8 a = *reinterpret_cast<const fh8 *>(kp + 32 * u);
-                        a0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qh[u], a0, 0, 0, 0);
-                        a1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, ql[u], a1, 0, 0, 0);
-                    }
-                    sc[hh] = (a0 + a1) * sinv;
-                }
-                fa16_ahead<HD / 16>();
-                __builtin_amdgcn_sched_barrier(0);
-                if (p == 0 && (more || !TIGHT)) {
+                fa16_scores<HD>(ks, c, g, qh, ql, sinv, sc);
+                if (more || !TIGHT) {
                     issue_k(step + 1);
                     issue_v(step + 1);
                 }
-                fa16_softmax_pv<HD>(sc, kb, k_hi, qs, qe, vts, m[p], l[p], o[p]);
+                fa16_softmax_pv<HD>(sc, k0 + 64 * step + 32 * own, k_hi, qs, qe, vts, m[0], l[0], o[0]);
+            }
+            if constexpr (NP == 2) {
+                const int kb = k0 + 64 * step + 32 * (own ^ 1);
+                if (kb < k_hi) {
+                    const _Float16 *ks = kv[step & 1][own ^ 1], *vts = ks + KB;
+                    fa4 sc[2];
+                    fa16_scores<HD>(ks, c, g, qh, ql, sinv, sc);
+                    fa16_softmax_pv<HD>(sc, kb, k_hi, qs, qe, vts, m[1], l[1], o[1]);
+                }
             }
         }
         if (more) stage(step + 1);
