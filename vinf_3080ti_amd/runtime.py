@@ -165,6 +165,7 @@ class Runtime:
         self.tensors: dict[str, _Tensor] = {}
         self.buffers: dict[str, _Buffer] = {}
         self._scratches: dict[int, _Scratch] = {}  # by stream
+        self._scratch()
         self.gemm_min_rows = 0
         self.batch_invariant = False
         self.gemm_f16_activations = False
