@@ -86,6 +86,36 @@ def test_conv_update_spans(rt, oracle_mod, K, rows, in_place):
     assert np.array_equal(get(rt, "csn", (-1, ch, K))[:n - 1], snaps)
 
 
+# Two, four and eight rows at once, shorter segments beside them; three hundred channels leave a part of a workgroup.
+@pytest.mark.parametrize("K", [1, 3, 4, 8])
+@pytest.mark.parametrize("rows", [(2,), (3,), (4,), (5,), (8,), (1, 2), (4, 1, 2, 3), (8, 5, 1, 7)])
+def test_conv_update_short_segments(rt, oracle_mod, K, rows):
+    """Decode and verify passes of several sequences, state and snapshots; bounds as above."""
+    rng = np.random.default_rng(10 * K + sum(rows))
+    ch, slots = 300, 4
+    segs, n = segments(rt, rows, slots)
+    x = rng.standard_normal((n, ch)).astype(np.float32)
+    cs0 = rng.standard_normal((slots, ch, K)).astype(np.float32)
+    w = (rng.standard_normal((ch, K)) * 0.5).astype(np.float32)
+    put_weight(rt, "cw", w)
+    put(rt, "cx", x)
+    for write in (0, 1):
+        put(rt, "cs", cs0)
+        put(rt, "co", x)
+        put(rt, "csn", np.zeros((max(n - 1, 1), ch, K)))
+        snap = "csn" if len(rows) == 1 and n > 1 else None
+        rt.conv_update_seg("cx", "cs", "cw", "co", ch, K, snap, write)
+        expect, states = x.astype(np.float64), cs0.astype(np.float64)
+        for slot, _, m, r0 in segs:
+            expect[r0:r0 + m], fin, snaps = oracle_mod.conv_update(x[r0:r0 + m], cs0[slot], w)
+            if write:
+                states[slot] = fin
+        assert np.allclose(get(rt, "co", (n, ch)), expect, rtol=1e-5, atol=1e-6)
+        assert np.array_equal(get(rt, "cs", (slots, ch, K)), states)
+        if snap:
+            assert np.array_equal(get(rt, "csn", (-1, ch, K))[:n - 1], snaps)
+
+
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 128, 129, 200, 256, 257])
 def test_rmsnorm_short_groups(rt, n):
     """Groups of up to 256 values take one wave each (64, 128 or 256 values per wave), longer ones a workgroup: against

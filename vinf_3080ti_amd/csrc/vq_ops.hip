@@ -1286,10 +1286,13 @@ size_t split_ws_bytes(const SegTable &T, int span_rows, int heads, int kv_heads,
 // loads issued together, take 9.3 us (2560 workgroups; the rows read twice come from L2). The first span's
 // thread is the only one that touches the state: it reads it, and writes the last K inputs into it. A span of
 // all rows (span >= rows, grid.z 1) keeps every read of a channel's x ahead of the writes that follow it, which x ==
-// out needs.
+// out needs. TR rows' loads at once: as many as the longest segment has, up to the span.
+// The state's K words of a channel are read and written as they lie, in wide accesses: word by word (where the compiler
+// merged the two ways to a window, or chose each word's source by itself) 32 segments of 4 rows x 10240 channels took
+// 6.4 us at K 4 and 13.7 at K 8, now 5.1 and 6.4 (one thread per channel and row by row: 5.3 and 6.6).
 constexpr int kConvRows = 8;  // rows whose loads are in flight together, and the span of a long pass
 static_assert(kConvRows >= VQ_CONV_MAX_K, "the K rows before a later span lie in the segment");
-template <int K, int TR>
+template <int K, int TR, bool SPANS = false>  // SPANS: grid.z > 1
 __global__ __launch_bounds__(256) void conv_update_kernel(const float *x, float *__restrict__ state,
                                                           const float *__restrict__ w, float *out, int channels,
                                                           SegTable T, float *__restrict__ snap, int write_state,
@@ -1297,7 +1300,7 @@ __global__ __launch_bounds__(256) void conv_update_kernel(const float *x, float 
     const int c = blockIdx.x * 256 + threadIdx.x;
     const Seg &s = T.s[blockIdx.y];
     // TR == 1: a pass of one row per segment.
-    const int rows = TR == 1 ? 1 : s.rows, ta = TR == 1 ? 0 : blockIdx.z * span, tb = min(ta + span, rows);
+    const int rows = TR == 1 ? 1 : s.rows, ta = SPANS ? blockIdx.z * span : 0, tb = min(ta + span, rows);
     if (c >= channels || ta >= rows) return;
     float *st = state + (static_cast<size_t>(s.slot) * channels + c) * K;
     const float *const xc = x + static_cast<size_t>(s.row0) * channels + c;
@@ -1306,12 +1309,15 @@ __global__ __launch_bounds__(256) void conv_update_kernel(const float *x, float 
 #pragma unroll
     for (int k = 0; k < K; ++k) wc[k] = w[static_cast<size_t>(c) * K + k];
     // Window slot k before row ta: input ta - K + k, for the first span the state.
-    if (ta == 0) {
+    if (!SPANS || ta == 0) {
 #pragma unroll
         for (int k = 0; k < K; ++k) win[k] = st[k];
     } else {
 #pragma unroll
         for (int k = 0; k < K; ++k) win[k] = xc[static_cast<size_t>(ta - K + k) * channels];
+        // Or the loads of both branches become one run of single words: 0.3 us less for one segment of 512 rows, but 46
+        // instead of 42 us for 64 of 64 at K 8.
+        if constexpr (K > 4) __builtin_amdgcn_sched_barrier(0);
     }
     for (int t0 = ta; t0 < (TR == 1 ? 1 : tb); t0 += TR) {
         float xi[TR];
@@ -1336,9 +1342,12 @@ __global__ __launch_bounds__(256) void conv_update_kernel(const float *x, float 
         }
     }
     if (write_state && ta == 0) {
+        if (SPANS && tb < rows) {
 #pragma unroll
-        for (int k = 0; k < K; ++k)
-            st[k] = TR == 1 || tb == rows ? win[k] : xc[static_cast<size_t>(rows - K + k) * channels];
+            for (int k = 0; k < K; ++k) win[k] = xc[static_cast<size_t>(rows - K + k) * channels];
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) st[k] = win[k];
     }
 }
 
@@ -1870,13 +1879,15 @@ int launch_conv_update(const float *x, float *state, const float *w, float *out,
     const bool overlap = x < out + n && out < x + n;
     const int span = max_rows <= kConvRows || overlap ? max_rows : kConvRows;
     const dim3 grid((channels + 255) / 256, T.n, (max_rows + span - 1) / span);
+    auto go = [&](auto kernel) { kernel<<<grid, 256, 0, s>>>(x, state, w, out, channels, T, snap, write_state, span); };
     switch (K) {
 #define VQ_CONV_CASE(KK)                                                                                              \
     case KK:                                                                                                          \
-        if (max_rows == 1)                                                                                            \
-            conv_update_kernel<KK, 1><<<grid, 256, 0, s>>>(x, state, w, out, channels, T, snap, write_state, span);   \
-        else                                                                                                          \
-            conv_update_kernel<KK, kConvRows><<<grid, 256, 0, s>>>(x, state, w, out, channels, T, snap, write_state, span); \
+        if (max_rows == 1) go(conv_update_kernel<KK, 1>);                                                             \
+        else if (max_rows == 2) go(conv_update_kernel<KK, 2>);                                                        \
+        else if (max_rows <= 4) go(conv_update_kernel<KK, 4>);                                                        \
+        else if (grid.z == 1) go(conv_update_kernel<KK, kConvRows>);                                                  \
+        else go(conv_update_kernel<KK, kConvRows, true>);                                                             \
         break;
         VQ_CONV_CASE(1) VQ_CONV_CASE(2) VQ_CONV_CASE(3) VQ_CONV_CASE(4)
         VQ_CONV_CASE(5) VQ_CONV_CASE(6) VQ_CONV_CASE(7) VQ_CONV_CASE(8)
