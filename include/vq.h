@@ -260,12 +260,15 @@ int vq_gated_delta_seg(const float *conv, const float *b, const float *a, const 
                        void *stream);
 
 /* Workspace bytes of vq_gated_delta_seg_ws for this segment table: non-zero when a segment is long enough for the
- * chunked kernels (24 rows; kd 128, vd a multiple of 32 up to 128), else 0 (the call then runs token by token). */
+ * chunked kernels (24 rows; kd 128, vd a multiple of 32 up to 128), else 0 (the call then runs token by token). At most
+ * 32 MiB of operands and, where a segment has more than 16 chunks of 32 rows, the fp32 states of the segments that share
+ * them, however many segments there are (one chunk's operands where 32 MiB do not hold it: over 3640 value heads). */
 size_t vq_gated_delta_seg_workspace_bytes(const int32_t *segs, int nseg, int key_heads, int value_heads, int kd, int vd);
 
 /* vq_gated_delta_seg with a workspace (16-byte aligned, >= vq_gated_delta_seg_workspace_bytes, else
  * VQ_ERR_WORKSPACE; NULL: as vq_gated_delta_seg): long segments run in chunks of 32 tokens on fp32 MFMA, whose
- * sums group differently from the per-token kernel's (same precision). Each segment takes its path by its own row
+ * sums group differently from the per-token kernel's (same precision); a chunk with a value that is not finite or near
+ * the end of the fp32 range, or with decays above one, token by token. Each segment takes its path by its own row
  * count alone. With snap every segment runs token by token. Replaces: Runtime.gated_delta_seg
  * (qwen_runtime.cu:2513-2565). */
 int vq_gated_delta_seg_ws(const float *conv, const float *b, const float *a, const float *ssm_a, const float *dt,
