@@ -34,11 +34,11 @@
 // a B operand as it stands, and an A operand is one float4 of a row.
 //
 // A value that is not finite, given or arising on the way, would meet zeros of T and P in these products and reach tokens
-// before its own. Chunks that could hold one are taken token by token: the prep kernel flags those
-// whose sums of squares lie past kGcSquare or whose scales past kGcScale, the walk those whose V or S0 lies past kGcHuge.
-// Below these bounds no product or sum of a chunk leaves the fp32 range. So are chunks whose decays above one multiply to kGcGrow or more: the entries of T
-// reach that product (one otherwise), and with it the rounding of d. Equal keys, beta 0.9975, against float64: decays of
-// 1.1 1.3e-6 (token by token 1.2e-7), of 1.3 1.4e-4.
+// before its own. Chunks that could hold one are taken token by token: the prep kernel flags those whose sums of squares
+// lie past kGcSquare or whose scales past kGcScale, the walk those whose V or S0 lies past kGcHuge; below these bounds no
+// product or sum of a chunk leaves the fp32 range. So are chunks whose decays above one multiply to kGcGrow or more: the
+// entries of T reach that product (one otherwise), and with it the rounding of d. Equal keys, beta 0.9975, against
+// float64: decays of 1.1 1.3e-6 (token by token 1.2e-7), of 1.3 1.4e-4.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stddef.h>

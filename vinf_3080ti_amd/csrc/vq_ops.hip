@@ -1696,12 +1696,12 @@ void launch_mfma_hd(bool fast, dim3 grid, hipStream_t s, const float *q, const C
 // 3 + 3). Every form gives the same bits, so the choice may look at the pass. hd 256: eight waves, up to four heads in
 // halves. hd 64 and 128: four waves, up to two heads in halves (whose 170 registers let two workgroups and more share a
 // CU), or, with three heads and more of a kv head, up to four heads, each whole in one wave: less work in all (K and V
-// staged once for four heads, queries split once), more per wave. The whole form pays when it has more than a workgroup for
-// every CU, and the shorter the contexts the later; under a short window from 192 workgroups on (192: 15.8 / 14.6 us, 128:
-// 12.5 / 14.1). hd 128, 32 heads on 8 kv heads, halves / whole, us (eight waves of
-// halves, the kernel before that): 512 rows 17.4 / 20.3 (20.8, 25.5), over 2048 keys 54 / 62 (58, 85); 640 rows 20.5 / 24.7
-// (23.5, 36), over 2048 keys 84 / 66 (85, 109); 2048 rows 141 / 113 (141, 188), windows of 256 53 / 39 (55, 49); 16 heads
-// of their own, 512 rows over 2048 keys 45 (82, 88), windows of 128 11 (19, 14).
+// staged once for four heads, queries split once), more per wave. The whole form pays when it has more than a workgroup
+// for every CU, and the shorter the contexts the later; under a short window from 192 workgroups on (192: 15.8 / 14.6 us,
+// 128: 12.5 / 14.1). hd 128, 32 heads on 8 kv heads, halves / whole, us (eight waves of halves, one wave per head with
+// single buffering): 512 rows 17.4 / 20.3 (20.8, 25.5), over 2048 keys 54 / 62 (58, 85); 640 rows 20.5 / 24.7 (23.5, 36),
+// over 2048 keys 84 / 66 (85, 109); 2048 rows 141 / 113 (141, 188), windows of 256 53 / 39 (55, 49); 16 heads of their
+// own, 512 rows over 2048 keys 45 (82, 88), windows of 128 11 (18, 14).
 template <bool PAGED>
 void launch_prompt16(int tiles, hipStream_t s, const float *q, const _Float16 *kc, const _Float16 *vc, float *out,
                      const SegTable &T, const KvMap &M, int heads, int hd, int bidirectional, int window) {
